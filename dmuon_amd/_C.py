@@ -27,7 +27,20 @@ NS_GRAM = 1
 # DMUON_ABI_VERSION of include/dmuon_amd.h: the argument lists below are those of this
 # version, and a library that reports another one is refused (its entry points would be
 # called with the wrong arguments).
-ABI_VERSION = 108
+ABI_VERSION = 109
+
+MAX_GROUPS = 8         # DMUON_MAX_GROUPS
+
+
+class MuonGroup(ctypes.Structure):
+    """``dmuon_muon_group``: one oriented shape of a several-shapes call."""
+
+    _fields_ = [(k, c_vp) for k in ("g_ptrs", "buf_ptrs", "est_ptrs", "w_ptrs", "pub_ptrs")] + \
+        [(k, c_int) for k in ("g_dtype", "w_dtype", "pub_dtype", "rows", "cols", "batch",
+                              "n_transposed", "first_step")]
+
+
+c_gp = ctypes.POINTER(MuonGroup)
 
 # name -> (restype, argtypes); mirrors include/dmuon_amd.h
 _SIGNATURES = {
@@ -79,6 +92,12 @@ _SIGNATURES = {
     "dmuon_muon_apply_group": (c_int, [c_vp, c_int, c_vp, c_int, c_int, c_int, c_int, c_int, c_d,
                                        c_d, c_fp, c_int, c_int, c_ip, c_int, c_vp, c_i64, c_int,
                                        c_vp]),
+    "dmuon_muon_plan_groups": (c_int, [c_gp, c_int, c_int, c_int, c_int, ctypes.POINTER(c_int),
+                                       ctypes.POINTER(c_i64), ctypes.POINTER(c_d)]),
+    "dmuon_muon_stage_groups": (c_int, [c_gp, c_int, c_d, c_int, c_int, c_f, c_vp, c_i64, c_int,
+                                        c_vp]),
+    "dmuon_muon_apply_groups": (c_int, [c_gp, c_int, c_d, c_d, c_fp, c_int, c_int, c_ip, c_int,
+                                        c_vp, c_i64, c_int, c_vp]),
     "dmuon_newton_schulz_group": (c_int, [c_vp, c_int, c_vp, c_int, c_int, c_int, c_int, c_int,
                                           c_fp, c_int, c_int, c_ip, c_int, c_f, c_vp, c_i64,
                                           c_int, c_vp]),
@@ -165,6 +184,18 @@ def plan(rows: int, cols: int, batch: int, tile: int = 0, num_cus: int = 0,
     check(lib().dmuon_ns_plan(rows, cols, batch, tile, num_cus, backend, ctypes.byref(t),
                               ctypes.byref(mp), ctypes.byref(np_), ctypes.byref(ws)))
     return t.value, mp.value, np_.value, ws.value
+
+
+def plan_groups(shapes, tile: int = 0, num_cus: int = 0, backend: int = NS_DIRECT):
+    """(tile, workspace_bytes, estimated us of the products) of the groups ``[(rows, cols,
+    batch), ...]`` run in one call."""
+    descs = (MuonGroup * len(shapes))()
+    for d, (rows, cols, batch) in zip(descs, shapes):
+        d.rows, d.cols, d.batch = rows, cols, batch
+    t, ws, us = c_int(), c_i64(), c_d()
+    check(lib().dmuon_muon_plan_groups(descs, len(shapes), tile, num_cus, backend,
+                                       ctypes.byref(t), ctypes.byref(ws), ctypes.byref(us)))
+    return t.value, ws.value, us.value
 
 
 def restart_array(restarts) -> tuple:

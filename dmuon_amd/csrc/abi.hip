@@ -6,6 +6,7 @@
 
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/dmuon_amd.h"
@@ -208,6 +209,258 @@ int plan(int rows, int cols, int batch, int tile_req, int num_cus, int gram, int
   return 0;
 }
 
+// Estimated time (us) of the Newton-Schulz products of a call's groups on `tile`-tiles: each
+// product is one launch over all of them, whose time is that of its longest tile or of its
+// work spread over the machine, whichever is more, plus a fixed part per launch. A tile's time is
+// fixed + slices of K (64 wide) at the kernel's rate, measured on MI355X as K sweeps of triangle
+// products (us): 256-tiles 13 + 1.0 per slice, 128-tiles one per CU 6 + 0.39, two per CU
+// 6 + 0.68 for the pair, 64-tiles 5 + 0.18. Only the comparison of two splits matters.
+double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, bool gram) {
+  // launches of one NS run of five steps: X X^T, m x m triangle products, Q updates, P X
+  const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_full = gram ? 3 : 0,
+               n_px = gram ? 2 : 5;
+  auto launch = [&](auto&& dims) {   // dims(group, tile): (tiles of one matrix, K)
+    auto total = [&](int t) {
+      double tiles = 0;
+      for (int i = 0; i < n; ++i) tiles += dims(g[i], t).first * g[i].batch;
+      return tiles;
+    };
+    int t = tile;
+    double fixed = 13.0, slice = 1.0, slots = num_cus;
+    if (tile == 128) {
+      if (total(64) <= num_cus) t = 64, fixed = 5.0, slice = 0.18;
+      else if (total(128) <= num_cus) fixed = 6.0, slice = 0.39;
+      else fixed = 6.0, slice = 0.68, slots = 2.0 * num_cus;
+    }
+    double longest = 0, sum = 0;
+    for (int i = 0; i < n; ++i) {
+      const std::pair<double, double> d = dims(g[i], t);
+      const double us = fixed + slice * ceil(d.second / 64.0);
+      longest = us > longest ? us : longest;
+      sum += us * d.first * g[i].batch;
+    }
+    // a last wave that is partly empty: half a tile on average
+    const double spread = sum / slots + (total(t) > slots ? 0.5 * longest : 0.0);
+    return (spread > longest ? spread : longest) + 2.0;
+  };
+  auto sides = [](const dmuon_muon_group& q, int t) {
+    const int64_t m = q.rows < q.cols ? q.rows : q.cols, w = q.rows < q.cols ? q.cols : q.rows;
+    return std::pair<double, double>((double)((m + t - 1) / t), (double)((w + t - 1) / t));
+  };
+  auto m_of = [](const dmuon_muon_group& q) { return (double)(q.rows < q.cols ? q.rows : q.cols); };
+  auto n_of = [](const dmuon_muon_group& q) { return (double)(q.rows < q.cols ? q.cols : q.rows); };
+  typedef std::pair<double, double> dims_t;
+  const double tri_m = launch([&](const dmuon_muon_group& q, int t) {
+    const double s = sides(q, t).first;
+    return dims_t(s * (s + 1) / 2, m_of(q));
+  });
+  const double tri_n = launch([&](const dmuon_muon_group& q, int t) {
+    const double s = sides(q, t).first;
+    return dims_t(s * (s + 1) / 2, n_of(q));
+  });
+  const double full = launch([&](const dmuon_muon_group& q, int t) {
+    const double s = sides(q, t).first;
+    return dims_t(s * s, m_of(q));
+  });
+  const double px = launch([&](const dmuon_muon_group& q, int t) {
+    const std::pair<double, double> s = sides(q, t);
+    return dims_t(s.first * s.second, m_of(q));
+  });
+  return n_xx * tri_n + n_tri * tri_m + n_full * full + n_px * px;
+}
+
+// Tile, workspace and estimated time of several groups in one call. One group takes the tile
+// plan() gives it; several the tile whose estimate is lower (either gives every matrix the same
+// bits).
+int plan_groups(const dmuon_muon_group* g, int n, int tile_req, int num_cus, int gram, int* tile,
+                int64_t* bytes, double* cost_us) {
+  if (num_cus <= 0) num_cus = 256;
+  int t = tile_req, mp, np;
+  int64_t total = 0, one;
+  if (t == 0 && n > 1)
+    t = groups_cost_us(g, n, 256, num_cus, gram) <= groups_cost_us(g, n, 128, num_cus, gram)
+            ? 256 : 128;
+  for (int i = 0; i < n; ++i) {
+    if (plan(g[i].rows, g[i].cols, g[i].batch, t, num_cus, gram, tile, &mp, &np, &one)) return 1;
+    total += one;
+  }
+  *bytes = total;
+  if (cost_us) *cost_us = groups_cost_us(g, n, *tile, num_cus, gram);
+  return 0;
+}
+
+// One group of a call: `batch` matrices of one oriented shape, their tables, workspace and the
+// state of their Newton-Schulz iteration.
+struct Group {
+  void* const* g_ptrs; int g_dtype;
+  float* const* buf_ptrs;
+  float* const* est_ptrs;
+  void* const* w_ptrs; int w_dtype;
+  void* const* pub_ptrs; int pub_dtype;
+  void* const* out_ptrs; int out_dtype;
+  int rows, cols, batch, n_t, first_step;
+  float lrs;
+  // derived (group_setup)
+  int m, n, m_pad, n_pad, km, kn, n_flip;
+  bool tall;
+  long long xs, as;
+  Workspace w;
+  // NS: the current X and the buffer the next one is written to, whether it is still the staged
+  // one, the scale of the stored R (or A), the Q slots and the row form of a slot's Q
+  uint16_t *x_cur, *x_nxt;
+  bool x_staged;
+  float rs;
+  uint16_t* qslot[2];
+  uint16_t* qbuf[2];
+};
+
+// What one call runs: up to kMaxGroups groups of different shapes, each product of the iteration
+// one launch over all of them. The groups share the tile size, the coefficients and the restarts;
+// a matrix's bits depend on none of the others.
+struct Call {
+  Group* g;
+  int n, tile;
+  hipStream_t stream;
+  const char* who;
+};
+
+double syrk_flops(const Group& g) { return (double)g.batch * g.m * (g.m + 1.0) * g.n; }
+double poly_flops(const Group& g) { return (double)g.batch * g.m * (g.m + 1.0) * g.m; }
+double gemm_flops(const Group& g) { return 2.0 * g.batch * (double)g.m * g.m * g.n; }
+double square_flops(const Group& g) { return 2.0 * g.batch * (double)g.m * g.m * g.m; }
+double update_bytes(const Group& g) {
+  const double elems = (double)g.rows * g.cols * g.batch;
+  auto width = [](int dtype) { return dtype == DMUON_DTYPE_F32 ? 4.0 : 2.0; };
+  return elems * ((g.w_ptrs ? 2.0 * width(g.w_dtype) : 0.0) +
+                  (g.out_ptrs ? width(g.out_dtype) : 0.0) +
+                  (g.pub_ptrs ? width(g.pub_dtype) : 0.0));
+}
+
+// One product of the iteration over the groups of a call: fill(group, args) sets a group's
+// operands, work(group) its useful FLOPs.
+template <class Fill>
+int nt_product(const Call& c, int cls, double (*work)(const Group&), Fill&& fill) {
+  NtArgs a[kMaxGroups];
+  double flops = 0.0, bytes = 0.0;
+  for (int i = 0; i < c.n; ++i) {
+    Group& g = c.g[i];
+    NtArgs& s = a[i];
+    s = NtArgs{};
+    s.elt = ELT_F16;
+    s.L = g.batch;
+    fill(g, s);
+    s.mt = s.M / c.tile;
+    s.nt = s.N / c.tile;
+    s.tiles_per_mat = s.tri ? tri_tiles(s.M, c.tile) : s.mt * s.nt;
+    flops += work(g);
+    if (cls == PC_FINAL) bytes += update_bytes(g);
+  }
+  return timed(cls, flops, bytes, c.stream, c.who,
+               [&] { return launch_nt_batch(a, c.n, c.tile, c.stream); });
+}
+
+// K loop lengths: the operands are zero past m (n), so the products multiply only m (n) rounded
+// up to the 64-wide slice (km, kn), not the tile-padded m_pad (n_pad); rows and columns past
+// that are never read, which live_rows / live_cols state.
+void square_operands(const Group& g, NtArgs& s, const uint16_t* A, const uint16_t* B,
+                     const uint16_t* C) {
+  s.A = A; s.B = B; s.C = C;
+  s.lda = s.ldb = s.ldc = s.ldd = s.lddt = g.m_pad;
+  s.sA = s.sB = s.sC = s.sD = s.sDT = g.as;
+  s.M = s.N = s.K = g.m_pad;
+  s.k_loop = g.km;
+  s.live_rows = s.live_cols = g.km < g.m_pad ? g.km : 0;
+}
+
+// D = alpha * A B^T + beta * C + diag * I, m x m, upper tiles mirrored (a symmetric result), and
+// optionally D2 = D + diag2 * I
+void symmetric_square(const Group& g, NtArgs& s, const uint16_t* A, const uint16_t* B,
+                      const uint16_t* C, uint16_t* D, float alpha, float beta, float diag,
+                      uint16_t* D2 = nullptr, float diag2 = 0.f) {
+  square_operands(g, s, A, B, C);
+  s.tri = 1; s.sym_exact = 1; s.diag_skip = kDiagSkipPoly;
+  s.mode = EPI_SYM; s.alpha = alpha; s.beta = beta; s.diag = diag;
+  s.c_in = C == A ? C_IS_A : C_NONE;   // C's tile is the A panel's last slices
+  s.D = D; s.D2 = D2; s.diag2 = diag2;
+}
+
+// R = alpha X X^T. The staged X may carry an estimated scale: the first products that read it
+// multiply by the per-matrix correction (ratio for X, ratio_sq for X X^T; 1 after an exact
+// staging). Later X are exactly scaled.
+void gram_of_x(const Group& g, NtArgs& s, uint16_t* R, float alpha) {
+  s.alpha_dev = g.x_staged ? g.w.ratio_sq : nullptr;
+  s.A = s.B = g.x_cur;
+  s.lda = s.ldb = g.n_pad;
+  s.sA = s.sB = g.xs;
+  s.M = s.N = g.m_pad; s.K = g.n_pad; s.k_loop = g.kn;
+  s.live_rows = s.live_cols = g.km < g.m_pad ? g.km : 0;
+  s.tri = 1; s.sym_exact = 1; s.diag_skip = kDiagSkipGram;
+  s.mode = EPI_SYM; s.alpha = alpha;
+  s.D = R; s.ldd = g.m_pad; s.sD = g.as;
+}
+
+// X' = P X + beta X into the other X buffer (X is the k-major B operand, read across the whole K
+// range, so the new X goes elsewhere)
+void px_next(const Group& g, NtArgs& s, const uint16_t* P, float beta) {
+  s.alpha_dev = g.x_staged ? g.w.ratio : nullptr;
+  s.A = P; s.lda = g.m_pad; s.sA = g.as;
+  s.B = g.x_cur; s.ldb = g.n_pad; s.sB = g.xs; s.b_kmajor = 1;
+  s.M = g.m_pad; s.N = g.n_pad; s.K = g.m_pad; s.k_loop = g.km;
+  s.live_rows = g.km < g.m_pad ? g.km : 0;
+  s.live_cols = g.kn < g.n_pad ? g.kn : 0;
+  s.alpha = 1.f; s.beta = beta;
+  s.mode = EPI_NS;
+  s.D = g.x_nxt; s.ldd = g.n_pad; s.sD = g.xs;
+}
+void x_advance(Call& c) {
+  for (int i = 0; i < c.n; ++i) {
+    std::swap(c.g[i].x_cur, c.g[i].x_nxt);
+    c.g[i].x_staged = false;
+  }
+}
+
+// the last product: U = (P X + beta X) / KX with the Muon update in the epilogue
+void px_final(const Group& g, NtArgs& s, const uint16_t* P, float beta, float decay) {
+  px_next(g, s, P, beta);
+  s.alpha = 1.f / kNsKx;
+  s.mode = EPI_FINAL;
+  s.D = nullptr;
+  s.out_ptrs = g.out_ptrs; s.out_dtype = g.out_dtype;
+  s.w_ptrs = g.w_ptrs; s.w_dtype = g.w_dtype; s.decay = decay; s.lrs = g.lrs;
+  s.pub_ptrs = g.pub_ptrs; s.pub_dtype = g.pub_dtype;
+  s.m_real = g.m; s.n_real = g.n; s.transposed = g.tall ? 1 : 0; s.n_flip = g.n_flip;
+}
+
+// Direct NS on the same fp16 operands as the Gram form: X carries the power-of-two scale kNsKx
+// throughout; the first A (eigenvalues ~1/m) carries kr until its polynomial.
+int run_direct(Call& c, const float* coeffs, int T, float decay) {
+  for (int it = 0; it < T; ++it) {
+    const float ca = coeffs[3 * it], cb = coeffs[3 * it + 1], cc = coeffs[3 * it + 2];
+    if (it > 0)
+      for (int i = 0; i < c.n; ++i) c.g[i].rs = 1.f;
+    // A = rs * X X^T of the normalised X (the stored X is kNsKx * X)
+    if (nt_product(c, PC_SYRK, syrk_flops, [&](Group& g, NtArgs& s) {
+          gram_of_x(g, s, g.w.Am, g.rs / (kNsKx * kNsKx));
+        }))
+      return 1;
+    // P = c A A^T + b A
+    if (nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
+          symmetric_square(g, s, g.w.Am, g.w.Am, g.w.Am, g.w.Pm, cc / (g.rs * g.rs), cb / g.rs,
+                           0.f);
+        }))
+      return 1;
+    // X' = P X + a X; the final step writes U = X' / kNsKx
+    if (nt_product(c, it + 1 < T ? PC_GEMM : PC_FINAL, gemm_flops, [&](Group& g, NtArgs& s) {
+          if (it + 1 < T) px_next(g, s, g.w.Pm, ca);
+          else px_final(g, s, g.w.Pm, ca, decay);
+          s.C = g.x_cur; s.ldc = g.n_pad; s.sC = g.xs;
+        }))
+      return 1;
+    x_advance(c);
+  }
+  return 0;
+}
+
 // Gram-space NS (the reference's gram_newton_schulz, newton_schulz.py:333-448) on the fp16 NT
 // kernels, for X (m x n, m <= n) staged as fp16(KX * ns_in / ||ns_in||). With R = X X^T and
 // Z_i = c_i R^2 + b_i R, one NS step maps X to P_i X, P_i = Z_i + a_i I, so per step
@@ -223,96 +476,12 @@ int plan(int rows, int cols, int batch, int tile_req, int num_cus, int gram, int
 // loses the small eigenvalues of R). Power-of-two scales keep every operand normal in fp16:
 // X carries KX = 2^12 throughout, the first R (eigenvalues ~1/m) carries kr = 2^floor(log2 m)
 // (at most 2^12) until its first update; all scale changes are folded into alpha / beta.
-int run_gram(const Workspace& w, int m, int n, int m_pad, int n_pad, int tile, int batch, bool tall,
-             int n_flip,
-             const float* coeffs, int T, const int* restarts, int n_restarts,
-             void* const* w_ptrs, int w_dtype, void* const* pub_ptrs, int pub_dtype,
-             void* const* out_ptrs, int out_dtype, float decay, float lrs, double syrk_flops,
-             double tri_sq_flops, double gemm_flops, double final_bytes, hipStream_t stream,
-             const char* who) {
-  const long long xs = (long long)m_pad * n_pad, as = (long long)m_pad * m_pad;
-  const double full_sq_flops = 2.0 * batch * (double)m * m * m;
-  // K loop lengths: the operands are zero past m (n), so the products multiply only m (n)
-  // rounded up to the 64-wide slice, not the tile-padded m_pad (n_pad)
-  const int km = (int)round_up(m, 64), kn = (int)round_up(n, 64);
+int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_restarts,
+             float decay) {
   auto is_restart = [&](int it) {
     for (int r = 0; r < n_restarts; ++r)
       if (restarts[r] == it) return true;
     return false;
-  };
-  // D = alpha * A B^T + beta * C + diag * I, m x m; tri: upper tiles mirrored (symmetric result)
-  auto sq = [&](const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, float alpha,
-                float beta, float diag, bool tri, uint16_t* D2 = nullptr,
-                float diag2 = 0.f) -> int {
-    NtArgs s{};
-    s.elt = ELT_F16;
-    s.A = A; s.lda = m_pad; s.sA = as;
-    s.B = B; s.ldb = m_pad; s.sB = as;
-    s.M = m_pad; s.N = m_pad; s.K = m_pad; s.L = batch; s.k_loop = km;
-    s.mt = s.nt = m_pad / tile;
-    s.tiles_per_mat = tri ? tri_tiles(m_pad, tile) : s.mt * s.nt; s.tri = tri ? 1 : 0;
-    s.sym_exact = 1; s.diag_skip = kDiagSkipPoly;
-    s.live_rows = s.live_cols = km < m_pad ? km : 0;   // rows and columns past m: never read
-    s.mode = EPI_SYM; s.alpha = alpha; s.beta = C ? beta : 0.f; s.diag = diag;
-    s.C = C; s.ldc = m_pad; s.sC = as;
-    s.c_in = (C && C == A) ? C_IS_A : C_NONE;   // C's tile is the A panel's last slices
-    s.D = D; s.ldd = m_pad; s.sD = as;
-    s.D2 = D2; s.diag2 = diag2;
-    return timed(PC_POLY, tri ? tri_sq_flops : full_sq_flops, 0.0, stream, who,
-                 [&] { return launch_nt(s, tile, stream); });
-  };
-  // The staged X may carry an estimated scale: the first products that read it multiply by the
-  // per-matrix correction (ratio for X, ratio_sq for X X^T; 1 after an exact staging). A
-  // restart rewrites X exactly scaled.
-  bool x_staged = true;
-  // the current X and the buffer a restart writes the next one into
-  uint16_t* x_cur = w.X;
-  uint16_t* x_nxt = w.X2;
-  // R = alpha X X^T
-  auto gram_of_x = [&](uint16_t* R, float alpha) -> int {
-    NtArgs s{};
-    s.alpha_dev = x_staged ? w.ratio_sq : nullptr;
-    s.elt = ELT_F16;
-    s.A = x_cur; s.lda = n_pad; s.sA = xs;
-    s.B = x_cur; s.ldb = n_pad; s.sB = xs;
-    s.M = m_pad; s.N = m_pad; s.K = n_pad; s.L = batch; s.k_loop = kn;
-    s.mt = s.nt = m_pad / tile; s.tiles_per_mat = tri_tiles(m_pad, tile); s.tri = 1;
-    s.sym_exact = 1; s.diag_skip = kDiagSkipGram;
-    s.live_rows = s.live_cols = km < m_pad ? km : 0;
-    s.mode = EPI_SYM; s.alpha = alpha;
-    s.D = R; s.ldd = m_pad; s.sD = as;
-    return timed(PC_SYRK, syrk_flops, 0.0, stream, who, [&] { return launch_nt(s, tile, stream); });
-  };
-  // X <- Q X (an NS restart), or the final U = Q X / KX with the Muon update in the epilogue
-  auto qx = [&](const uint16_t* Q, bool last) -> int {
-    NtArgs g{};
-    g.alpha_dev = x_staged ? w.ratio : nullptr;
-    g.elt = ELT_F16;
-    g.A = Q; g.lda = m_pad; g.sA = as;
-    g.B = x_cur; g.ldb = n_pad; g.sB = xs; g.b_kmajor = 1;
-    g.M = m_pad; g.N = n_pad; g.K = m_pad; g.L = batch; g.k_loop = km;
-    g.live_rows = km < m_pad ? km : 0;
-    g.live_cols = kn < n_pad ? kn : 0;
-    g.mt = m_pad / tile; g.nt = n_pad / tile; g.tiles_per_mat = g.mt * g.nt; g.tri = 0;
-    g.beta = 0.f;
-    if (!last) {
-      g.alpha = 1.f;
-      g.mode = EPI_NS;
-      g.D = x_nxt; g.ldd = n_pad; g.sD = xs;   // X is the B operand: the new X goes elsewhere
-      if (timed(PC_GEMM, gemm_flops, 0.0, stream, who, [&] { return launch_nt(g, tile, stream); }))
-        return 1;
-      uint16_t* t = x_cur; x_cur = x_nxt; x_nxt = t;
-      x_staged = false;
-      return 0;
-    }
-    g.alpha = 1.f / kNsKx;
-    g.mode = EPI_FINAL;
-    g.out_ptrs = out_ptrs; g.out_dtype = out_dtype;
-    g.w_ptrs = w_ptrs; g.w_dtype = w_dtype; g.decay = decay; g.lrs = lrs;
-    g.pub_ptrs = pub_ptrs; g.pub_dtype = pub_dtype;
-    g.m_real = m; g.n_real = n; g.transposed = tall ? 1 : 0; g.n_flip = n_flip;
-    return timed(PC_FINAL, gemm_flops, final_bytes, stream, who,
-                 [&] { return launch_nt(g, tile, stream); });
   };
   // Q <- P Q = Z Q + a Q as a full product (Q is a product of polynomials that no longer
   // commute once rounded; its factor order must match R's). Z is symmetric, so the update runs
@@ -321,25 +490,16 @@ int run_gram(const Workspace& w, int m, int n, int m_pad, int n_pad, int tile, i
   // that consumes Q, which writes only its transposed output, the row form Q that Q X reads.
   // A Q that is still P itself (after a start or restart) is symmetric and serves as either
   // form. Two slots, used in turn.
-  uint16_t* qslot[2] = {w.Q0, w.Q1};
-  uint16_t* qbuf[2] = {w.Q0, w.Q1};          // the row form of a slot's Q, once it has one
-  auto q_update = [&](const uint16_t* Zm, int from, float a_, bool last) -> int {
+  auto q_update = [&](int from, float a_, bool last) -> int {
     const int to = 1 - from;
-    NtArgs g{};
-    g.elt = ELT_F16;
-    g.M = m_pad; g.N = m_pad; g.K = m_pad; g.L = batch; g.k_loop = km;
-    g.live_rows = g.live_cols = km < m_pad ? km : 0;
-    g.mt = g.nt = m_pad / tile; g.tiles_per_mat = g.mt * g.nt; g.tri = 0;
-    g.mode = EPI_NS; g.alpha = 1.f; g.beta = a_;
-    g.lda = g.ldb = g.ldc = g.ldd = g.lddt = m_pad;
-    g.sA = g.sB = g.sC = g.sD = g.sDT = as;
-    g.A = qslot[from]; g.B = Zm; g.C = qslot[from];
-    g.c_in = C_IS_A;                           // the addend is the A panel's last slices
-    if (last) g.DT = qslot[to];                // Q, the row form
-    else g.D = qslot[to];                      // Q^T
-    qbuf[to] = qslot[to];
-    return timed(PC_POLY, full_sq_flops, 0.0, stream, who,
-                 [&] { return launch_nt(g, tile, stream); });
+    return nt_product(c, PC_POLY, square_flops, [&](Group& g, NtArgs& s) {
+      square_operands(g, s, g.qslot[from], g.w.Pm, g.qslot[from]);
+      s.mode = EPI_NS; s.alpha = 1.f; s.beta = a_;
+      s.c_in = C_IS_A;                           // the addend is the A panel's last slices
+      if (last) s.DT = g.qslot[to];              // Q, the row form
+      else s.D = g.qslot[to];                    // Q^T
+      g.qbuf[to] = g.qslot[to];
+    });
   };
   // iterations from it up to the next restart (or T): the Q updates the segment has left
   auto updates_left = [&](int it) {
@@ -347,75 +507,213 @@ int run_gram(const Workspace& w, int m, int n, int m_pad, int n_pad, int tile, i
     while (end < T && !is_restart(end)) ++end;
     return end - it;
   };
-  int kr = 1;
-  while (kr * 2 <= m && kr < 4096) kr *= 2;
-  uint16_t* R = w.Am;
-  uint16_t* Z = w.Pm;
-  uint16_t* W = w.Wm;
+  auto gram = [&]() {
+    return nt_product(c, PC_SYRK, syrk_flops, [&](Group& g, NtArgs& s) {
+      gram_of_x(g, s, g.w.Am, g.rs / (kNsKx * kNsKx));
+    });
+  };
   int qs = -1;               // slot of the current Q, -1: none since the last (re)start
-  float rs = (float)kr;      // the stored R is rs * (X X^T of the normalised X)
-  if (gram_of_x(R, rs / (kNsKx * kNsKx))) return 1;
+  if (gram()) return 1;
   for (int it = 0; it < T; ++it) {
     if (it != 0 && is_restart(it) && qs >= 0) {
-      if (qx(qbuf[qs], false)) return 1;
-      rs = 1.f;
-      if (gram_of_x(R, 1.f / (kNsKx * kNsKx))) return 1;
+      if (nt_product(c, PC_GEMM, gemm_flops,
+                     [&](Group& g, NtArgs& s) { px_next(g, s, g.qbuf[qs], 0.f); }))
+        return 1;
+      x_advance(c);
+      for (int i = 0; i < c.n; ++i) c.g[i].rs = 1.f;
+      if (gram()) return 1;
       qs = -1;
     }
     const float ca = coeffs[3 * it], cb = coeffs[3 * it + 1], cc = coeffs[3 * it + 2];
     const bool evolve = it + 1 < T && !is_restart(it + 1);
-    const float zr2 = cc / (rs * rs), zr1 = cb / rs;
-    if (qs < 0 && !evolve) {
-      // Q = Z + a I in one product (Z itself is not needed); symmetric, its own transpose
-      if (sq(R, R, R, qslot[0], zr2, zr1, ca, true)) return 1;
-      qbuf[0] = qslot[0];
-      qs = 0;
-      continue;
-    }
-    if (qs < 0) {
-      // Z = c R^2 + b R, and Q = Z + a I written by the same epilogue
-      if (sq(R, R, R, Z, zr2, zr1, 0.f, true, qslot[0], ca)) return 1;
-      qbuf[0] = qslot[0];
+    // Z = c R^2 + b R; after a (re)start also Q = Z + a I, as the epilogue's second output, or,
+    // when R is not updated afterwards (Z itself is not needed), as the only one
+    const bool fresh = qs < 0, only_q = fresh && !evolve;
+    if (nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
+          uint16_t* R = g.w.Am;
+          symmetric_square(g, s, R, R, R, only_q ? g.qslot[0] : g.w.Pm, cc / (g.rs * g.rs),
+                           cb / g.rs, only_q ? ca : 0.f, fresh && evolve ? g.qslot[0] : nullptr,
+                           fresh && evolve ? ca : 0.f);
+          if (fresh) g.qbuf[0] = g.qslot[0];
+        }))
+      return 1;
+    if (fresh) {
       qs = 0;
     } else {
-      if (sq(R, R, R, Z, zr2, zr1, 0.f, true)) return 1;   // Z = c R^2 + b R
-      if (q_update(Z, qs, ca, updates_left(it) == 1)) return 1;   // Q <- Z Q + a Q
+      if (q_update(qs, ca, updates_left(it) == 1)) return 1;   // Q <- Z Q + a Q
       qs = 1 - qs;
     }
     if (evolve) {
-      if (sq(Z, R, R, W, 1.f, ca, 0.f, true)) return 1;               // rs * (P R)
-      if (sq(W, Z, W, R, 1.f / rs, ca / rs, 0.f, true)) return 1;     // P R P
-      rs = 1.f;
+      // W = Z R + a R (the stored R is rs times R), then R = P R P = W Z + a W
+      if (nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
+            symmetric_square(g, s, g.w.Pm, g.w.Am, g.w.Am, g.w.Wm, 1.f, ca, 0.f);
+          }) ||
+          nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
+            symmetric_square(g, s, g.w.Wm, g.w.Pm, g.w.Wm, g.w.Am, 1.f / g.rs, ca / g.rs, 0.f);
+          }))
+        return 1;
+      for (int i = 0; i < c.n; ++i) c.g[i].rs = 1.f;
     }
   }
-  return qx(qbuf[qs], true);
+  return nt_product(c, PC_FINAL, gemm_flops,
+                    [&](Group& g, NtArgs& s) { px_final(g, s, g.qbuf[qs], 0.f, decay); });
 }
 
-// The whole Newton-Schulz + optional update sequence of one group; see dmuon_muon_step_group.
+// Momentum, norm and NS operands of every group of a call.
+// A group's matrices share the m x n NS shape: [0, batch - n_t) are rows x cols and the last n_t
+// are cols x rows (their transposes). Each orientation is staged into its slice of the
+// workspace; everything after the staging sees one m x n batch, and the final epilogue writes
+// each matrix back in its own orientation. (Square shapes have one orientation: the n_t part is
+// staged and written like the rest.)
+int run_stage(const Call& c, float mu, int nesterov, float eps) {
+  PreArgs p[2 * kMaxGroups];
+  int np = 0;
+  bool est = false, exact = false;
+  double pre_bytes = 0.0, st_bytes = 0.0, norm_bytes = 0.0;
+  NormArgs na[kMaxGroups];
+  for (int i = 0; i < c.n; ++i) {
+    const Group& g = c.g[i];
+    (g.est_ptrs ? est : exact) = true;
+    for (int part = 0; part < 2; ++part) {
+      const int l0 = part == 0 ? 0 : g.batch - g.n_t, L = part == 0 ? g.batch - g.n_t : g.n_t;
+      if (L == 0) continue;
+      const int r_ = part == 0 ? g.rows : g.cols, c_ = part == 0 ? g.cols : g.rows;
+      const bool tall_ = r_ > c_;
+      PreArgs& q = p[np++];
+      q = PreArgs{};
+      q.g_ptrs = g.g_ptrs + l0;
+      q.g_dtype = g.g_dtype;
+      q.buf_ptrs = g.buf_ptrs ? g.buf_ptrs + l0 : nullptr;
+      q.est_ptrs = g.est_ptrs ? g.est_ptrs + l0 : nullptr;
+      q.Y = q.YT = g.w.X + l0 * g.xs;
+      q.ldy = tall_ ? g.m_pad : g.n_pad;
+      q.ldyt = tall_ ? g.n_pad : g.m_pad;
+      q.sY = q.sYT = g.xs;
+      q.partials = g.w.partials + (long long)l0 * g.w.nparts;
+      q.rows = r_;
+      q.cols = c_;
+      q.Rp = tall_ ? g.n_pad : g.m_pad;
+      q.Cp = tall_ ? g.m_pad : g.n_pad;
+      q.L = L;
+      q.mu = mu;
+      q.first_step = g.first_step;
+      q.nesterov = nesterov;
+      q.kx = kNsKx;
+      q.scale = g.w.scale + l0;
+      q.restage = g.est_ptrs ? g.w.restage + l0 : nullptr;
+      // the NS products read X k-major, so only X is staged: by the direct write for a wide
+      // orientation, by the transposed one for a tall orientation
+      q.skip_y = tall_ ? 1 : 0;
+      q.skip_yt = tall_ ? 0 : 1;
+      // algorithmic bytes (what one ideal pass moves): gradient read, fp32 momentum read (not on
+      // the first step) and write, one 2-byte copy of the normalised ns_in. The second pass's
+      // re-read of the gradient and the new momentum (fp16 cannot hold an un-normalised
+      // gradient, so the copy waits for the norm) is overhead, not counted.
+      const double elems = (double)r_ * c_ * L;
+      pre_bytes += elems * ((g.g_dtype == DMUON_DTYPE_F32 ? 4.0 : 2.0) +
+                            (g.buf_ptrs ? (g.first_step ? 4.0 : 8.0) : 0.0) +
+                            (g.est_ptrs ? 2.0 : 0.0));
+      if (!g.est_ptrs) st_bytes += elems * 2.0;
+    }
+    na[i] = NormArgs{g.w.partials, g.w.nparts, g.batch, g.w.scale, g.w.scale_sq, g.est_ptrs,
+                     g.w.ratio, g.w.ratio_sq, g.w.restage};
+    norm_bytes += (double)g.batch * g.w.nparts * 4;
+  }
+  if (est && exact)
+    return fail("%s: est_ptrs must be given for every group of a call or for none", c.who);
+  // With est_ptrs (a per-matrix scale kept from the previous step) the first pass also writes
+  // the fp16 copy as fp16(kx * est * ns_in); the norm finalize then keeps that copy when
+  // r = scale / est is within [1/4, 4] (the first products multiply by r or r^2, and every copy
+  // entry stays below kx / r <= 2^14) and otherwise flags the matrix for the second pass,
+  // which then stages exactly as without an estimate.
+  auto stage = [&](int st, bool flagged) {
+    for (int k = 0; k < np; ++k) {
+      p[k].stage = st;
+      if (!flagged) p[k].restage = nullptr;
+    }
+  };
+  const int* flags[2 * kMaxGroups];
+  for (int k = 0; k < np; ++k) flags[k] = p[k].restage;
+  stage(est ? PRE_EST : PRE_NORM, false);
+  if (timed(PC_PRE, 0.0, pre_bytes, c.stream, c.who,
+            [&] { return launch_pre_batch(p, np, c.stream); }))
+    return 1;
+  if (timed(PC_NORM, 0.0, norm_bytes, c.stream, c.who,
+            [&] { return launch_norm_finalize_est(na, c.n, eps, c.stream); }))
+    return 1;
+  for (int k = 0; k < np; ++k) p[k].restage = flags[k];
+  stage(PRE_F16, est);
+  return timed(PC_PRE, 0.0, st_bytes, c.stream, c.who,
+               [&] { return launch_pre_batch(p, np, c.stream); });
+}
+
+// Argument checks and the workspace of a call's groups, `c.g[i]` holding the caller's fields.
 // phases: PH_STAGE (momentum, norm, NS operand staging into the workspace), PH_APPLY (the NS
 // products and the fused update / output from a staged workspace), or both.
 enum { PH_STAGE = 1, PH_APPLY = 2 };
-int run_group(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs, float* const* est_ptrs,
-              void* const* w_ptrs, int w_dtype, void* const* pub_ptrs, int pub_dtype, void* const* out_ptrs,
-              int out_dtype, int rows, int cols, int batch, int n_t,
-              float mu, int nesterov, int first_step, float decay, float lrs, const float* coeffs,
-              int T, int backend, const int* restarts, int n_restarts, float eps, void* workspace,
-              int64_t workspace_bytes, int tile_req, hipStream_t stream, const char* who,
-              int phases = PH_STAGE | PH_APPLY) {
-  const bool do_stage = phases & PH_STAGE, do_apply = phases & PH_APPLY;
-  if (do_stage) {
-    if (!g_ptrs) return fail("%s: g_ptrs is NULL", who);
-    if (g_dtype != DMUON_DTYPE_F32 && g_dtype != DMUON_DTYPE_BF16)
-      return fail("%s: unsupported gradient dtype code %d", who, g_dtype);
+int group_setup(Call& c, int tile_req, int backend, void* workspace, int64_t workspace_bytes,
+                int phases) {
+  const char* who = c.who;
+  const int gram = backend == DMUON_NS_GRAM;
+  if (!workspace || !aligned16(workspace)) return fail("%s: workspace NULL or misaligned", who);
+  int64_t off = 0;
+  for (int i = 0; i < c.n; ++i) {
+    Group& g = c.g[i];
+    if (phases & PH_STAGE) {
+      if (!g.g_ptrs) return fail("%s: g_ptrs is NULL", who);
+      if (g.g_dtype != DMUON_DTYPE_F32 && g.g_dtype != DMUON_DTYPE_BF16)
+        return fail("%s: unsupported gradient dtype code %d", who, g.g_dtype);
+    }
+    if (phases & PH_APPLY) {
+      if (g.w_ptrs && g.w_dtype != DMUON_DTYPE_F32 && g.w_dtype != DMUON_DTYPE_BF16)
+        return fail("%s: unsupported weight dtype code %d", who, g.w_dtype);
+      if (g.out_ptrs && g.out_dtype != DMUON_DTYPE_F32 && g.out_dtype != DMUON_DTYPE_BF16)
+        return fail("%s: unsupported output dtype code %d", who, g.out_dtype);
+      if (g.pub_ptrs && !g.w_ptrs)
+        return fail("%s: pub_ptrs needs w_ptrs (it copies the new W)", who);
+      if (g.pub_ptrs && g.pub_dtype != DMUON_DTYPE_F32 && g.pub_dtype != DMUON_DTYPE_BF16)
+        return fail("%s: unsupported publish dtype code %d", who, g.pub_dtype);
+    }
+    if (g.n_t < 0 || g.n_t > g.batch)
+      return fail("%s: n_transposed=%d outside [0, batch=%d]", who, g.n_t, g.batch);
+    int tile;
+    int64_t need;
+    if (plan(g.rows, g.cols, g.batch, tile_req, 0, gram, &tile, &g.m_pad, &g.n_pad, &need))
+      return 1;
+    c.tile = tile;                       // several groups come with the tile of their plan
+    if (workspace_bytes - off < need)
+      return fail("%s: workspace of %lld bytes is smaller than the %lld bytes planned", who,
+                  (long long)workspace_bytes, (long long)(off + need));
+    g.tall = g.rows > g.cols;
+    g.m = g.tall ? g.cols : g.rows;
+    g.n = g.tall ? g.rows : g.cols;
+    g.km = (int)round_up(g.m, 64);
+    g.kn = (int)round_up(g.n, 64);
+    g.n_flip = g.rows == g.cols ? 0 : g.n_t;
+    g.xs = (long long)g.m_pad * g.n_pad;
+    g.as = (long long)g.m_pad * g.m_pad;
+    g.w = carve(static_cast<char*>(workspace) + off, g.m_pad, g.n_pad,
+                g.tall ? g.n_pad : g.m_pad, g.tall ? g.m_pad : g.n_pad, g.batch, gram);
+    off += need;
+    g.x_cur = g.w.X;
+    g.x_nxt = g.w.X2;
+    g.x_staged = true;
+    int kr = 1;
+    while (kr * 2 <= g.m && kr < 4096) kr *= 2;
+    g.rs = (float)kr;                    // the stored R is rs * (X X^T of the normalised X)
+    g.qslot[0] = g.qbuf[0] = g.w.Q0;
+    g.qslot[1] = g.qbuf[1] = g.w.Q1;
   }
-  if (do_apply) {
-    if (w_ptrs && w_dtype != DMUON_DTYPE_F32 && w_dtype != DMUON_DTYPE_BF16)
-      return fail("%s: unsupported weight dtype code %d", who, w_dtype);
-    if (out_ptrs && out_dtype != DMUON_DTYPE_F32 && out_dtype != DMUON_DTYPE_BF16)
-      return fail("%s: unsupported output dtype code %d", who, out_dtype);
-    if (pub_ptrs && !w_ptrs) return fail("%s: pub_ptrs needs w_ptrs (it copies the new W)", who);
-    if (pub_ptrs && pub_dtype != DMUON_DTYPE_F32 && pub_dtype != DMUON_DTYPE_BF16)
-      return fail("%s: unsupported publish dtype code %d", who, pub_dtype);
+  return 0;
+}
+
+// The whole Newton-Schulz + optional update sequence of a call's groups; see
+// dmuon_muon_step_group.
+int run_groups(Call& c, float mu, int nesterov, float decay, const float* coeffs, int T,
+               int backend, const int* restarts, int n_restarts, float eps, void* workspace,
+               int64_t workspace_bytes, int tile_req, int phases = PH_STAGE | PH_APPLY) {
+  const char* who = c.who;
+  if (phases & PH_APPLY) {
     if (!coeffs || T <= 0)
       return fail("%s: need at least one (a, b, c) coefficient triple", who);
     if (n_restarts < 0 || (n_restarts > 0 && !restarts))
@@ -423,181 +721,19 @@ int run_group(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs, float* c
   }
   if (backend != DMUON_NS_DIRECT && backend != DMUON_NS_GRAM)
     return fail("%s: unknown NS backend %d", who, backend);
-  if (n_t < 0 || n_t > batch)
-    return fail("%s: n_transposed=%d outside [0, batch=%d]", who, n_t, batch);
-  const int gram = backend == DMUON_NS_GRAM;
-  if (!workspace || !aligned16(workspace)) return fail("%s: workspace NULL or misaligned", who);
-  int tile, m_pad, n_pad;
-  int64_t need;
-  if (plan(rows, cols, batch, tile_req, 0, gram, &tile, &m_pad, &n_pad, &need)) return 1;
-  if (workspace_bytes < need)
-    return fail("%s: workspace of %lld bytes is smaller than the %lld bytes planned", who,
-                (long long)workspace_bytes, (long long)need);
-  const bool tall = rows > cols;
-  const int m = tall ? cols : rows, n = tall ? rows : cols;
-  const int Rp = tall ? n_pad : m_pad, Cp = tall ? m_pad : n_pad;
-  Workspace w = carve(static_cast<char*>(workspace), m_pad, n_pad, Rp, Cp, batch, gram);
-  const long long xs = (long long)m_pad * n_pad, as = (long long)m_pad * m_pad;
-
-  (void)Rp; (void)Cp;
-  // The group's matrices share the m x n NS shape: [0, batch - n_t) are rows x cols and the last
-  // n_t are cols x rows (their transposes). Each orientation is staged by its own launch into
-  // its slice of the workspace; everything after the staging sees one m x n batch, and the final
-  // epilogue writes each matrix back in its own orientation. (Square shapes have one
-  // orientation: the n_t part is staged and written like the rest.)
-  const int n_flip = rows == cols ? 0 : n_t;
-  auto pre_args = [&](int part) {
-    const int l0 = part == 0 ? 0 : batch - n_t;
-    const int r_ = part == 0 ? rows : cols, c_ = part == 0 ? cols : rows;
-    const bool tall_ = r_ > c_;
-    PreArgs q{};
-    q.g_ptrs = g_ptrs ? g_ptrs + l0 : nullptr;
-    q.g_dtype = g_dtype;
-    q.buf_ptrs = buf_ptrs ? buf_ptrs + l0 : nullptr;
-    q.est_ptrs = est_ptrs ? est_ptrs + l0 : nullptr;
-    q.Y = w.X + l0 * xs;
-    q.ldy = tall_ ? m_pad : n_pad;
-    q.sY = xs;
-    q.YT = w.X + l0 * xs;
-    q.ldyt = tall_ ? n_pad : m_pad;
-    q.sYT = xs;
-    q.partials = w.partials + (long long)l0 * w.nparts;
-    q.rows = r_;
-    q.cols = c_;
-    q.Rp = tall_ ? n_pad : m_pad;
-    q.Cp = tall_ ? m_pad : n_pad;
-    q.L = part == 0 ? batch - n_t : n_t;
-    q.mu = mu;
-    q.first_step = first_step;
-    q.nesterov = nesterov;
-    q.kx = kNsKx;
-    q.scale = w.scale + l0;
-    // the NS products read X k-major, so only X is staged: by the direct write for a wide
-    // orientation, by the transposed one for a tall orientation
-    q.skip_y = tall_ ? 1 : 0;
-    q.skip_yt = tall_ ? 0 : 1;
-    return q;
-  };
-  const double Ld = batch, md = m, nd = n, elems = (double)rows * cols * batch;
-  const double gbytes = g_dtype == DMUON_DTYPE_F32 ? 4.0 : 2.0;
-  if (do_stage) {
-  // algorithmic bytes (what one ideal pass moves): gradient read, fp32 momentum read (not on
-  // the first step) and write, one 2-byte copy of the normalised ns_in. The second pass's
-  // re-read of the gradient and the new momentum (fp16 cannot hold an un-normalised gradient,
-  // so the copy waits for the norm) is overhead, not counted.
-  // With est_ptrs (a per-matrix scale kept from the previous step) the first pass also writes
-  // the fp16 copy as fp16(kx * est * ns_in); the norm finalize then keeps that copy when
-  // r = scale / est is within [1/4, 4] (the first products multiply by r or r^2, and every copy
-  // entry stays below kx / r <= 2^14) and otherwise flags the matrix for the second pass,
-  // which then stages exactly as without an estimate.
-  const bool est = est_ptrs != nullptr;
-  const double mom_bytes = buf_ptrs ? (first_step ? 4.0 : 8.0) : 0.0;
-  for (int part = 0; part < 2; ++part) {
-    PreArgs p = pre_args(part);
-    if (p.L == 0) continue;
-    p.stage = est ? PRE_EST : PRE_NORM;
-    const double pre_bytes = elems * p.L / batch * (gbytes + mom_bytes + (est ? 2.0 : 0.0));
-    if (timed(PC_PRE, 0.0, pre_bytes, stream, who, [&] { return launch_pre(p, stream); }))
-      return 1;
-  }
-  if (timed(PC_NORM, 0.0, (double)batch * w.nparts * 4, stream, who, [&] {
-        return launch_norm_finalize_est(w.partials, w.nparts, batch, eps, w.scale, w.scale_sq,
-                                        est_ptrs, w.ratio, w.ratio_sq, w.restage, stream);
-      }))
-    return 1;
-  for (int part = 0; part < 2; ++part) {
-    PreArgs p = pre_args(part);
-    if (p.L == 0) continue;
-    p.stage = PRE_F16;
-    p.restage = est ? w.restage + (part == 0 ? 0 : batch - n_t) : nullptr;
-    const double st_bytes = est ? 0.0 : elems * p.L / batch * 2.0;
-    if (timed(PC_PRE, 0.0, st_bytes, stream, who, [&] { return launch_pre(p, stream); }))
-      return 1;
-  }
-  }  // do_stage
-  if (!do_apply) return 0;
-  const double syrk_flops = Ld * md * (md + 1) * nd, poly_flops = Ld * md * (md + 1) * md;
-  const double gemm_flops = 2.0 * Ld * md * md * nd;
-  const double wbytes = w_ptrs ? 2.0 * elems * (w_dtype == DMUON_DTYPE_F32 ? 4.0 : 2.0) : 0.0;
-  const double obytes = out_ptrs ? elems * (out_dtype == DMUON_DTYPE_F32 ? 4.0 : 2.0) : 0.0;
-  const double pbytes = pub_ptrs ? elems * (pub_dtype == DMUON_DTYPE_F32 ? 4.0 : 2.0) : 0.0;
-
-  if (gram)
-    return run_gram(w, m, n, m_pad, n_pad, tile, batch, tall, n_flip, coeffs, T, restarts,
-                    n_restarts,
-                    w_ptrs, w_dtype, pub_ptrs, pub_dtype, out_ptrs, out_dtype, decay, lrs,
-                    syrk_flops, poly_flops, gemm_flops, wbytes + obytes + pbytes, stream, who);
-  // Direct NS on the same fp16 operands as the Gram form: X carries the power-of-two scale
-  // kNsKx throughout; the first A (eigenvalues ~1/m) carries kr until its polynomial.
-  int kr = 1;
-  while (kr * 2 <= m && kr < 4096) kr *= 2;
-  const int km = (int)round_up(m, 64), kn = (int)round_up(n, 64);   // K loops (zero past m, n)
-  // the current X and the buffer the next one is written to
-  uint16_t* x_cur = w.X;
-  uint16_t* x_nxt = w.X2;
-  for (int it = 0; it < T; ++it) {
-    const float ca = coeffs[3 * it], cb = coeffs[3 * it + 1], cc = coeffs[3 * it + 2];
-    const float rs = it == 0 ? (float)kr : 1.f;   // the stored A is rs * (X X^T)
-    // A = X X^T of the normalised X (the stored X is kNsKx * X)
-    NtArgs s{};
-    s.elt = ELT_F16;
-    s.A = x_cur; s.lda = n_pad; s.sA = xs;
-    s.B = x_cur; s.ldb = n_pad; s.sB = xs;
-    s.M = m_pad; s.N = m_pad; s.K = n_pad; s.L = batch; s.k_loop = kn;
-    s.mt = s.nt = m_pad / tile; s.tiles_per_mat = tri_tiles(m_pad, tile); s.tri = 1;
-    s.sym_exact = 1; s.diag_skip = kDiagSkipGram;
-    s.live_rows = s.live_cols = km < m_pad ? km : 0;
-    s.mode = EPI_SYM; s.alpha = rs / (kNsKx * kNsKx); s.beta = 0.f; s.diag = 0.f;
-    s.alpha_dev = it == 0 ? w.ratio_sq : nullptr;   // the staged X's scale correction
-    s.D = w.Am; s.ldd = m_pad; s.sD = as;
-    if (timed(PC_SYRK, syrk_flops, 0.0, stream, who, [&] { return launch_nt(s, tile, stream); }))
-      return 1;
-    // P = c A A^T + b A
-    NtArgs q{};
-    q.elt = ELT_F16;
-    q.A = w.Am; q.lda = m_pad; q.sA = as;
-    q.B = w.Am; q.ldb = m_pad; q.sB = as;
-    q.M = m_pad; q.N = m_pad; q.K = m_pad; q.L = batch; q.k_loop = km;
-    q.mt = q.nt = m_pad / tile; q.tiles_per_mat = s.tiles_per_mat; q.tri = 1;
-    q.sym_exact = 1; q.diag_skip = kDiagSkipPoly;
-    q.live_rows = q.live_cols = km < m_pad ? km : 0;
-    q.mode = EPI_SYM; q.alpha = cc / (rs * rs); q.beta = cb / rs; q.diag = 0.f;
-    q.C = w.Am; q.ldc = m_pad; q.sC = as;
-    q.c_in = C_IS_A;
-    q.D = w.Pm; q.ldd = m_pad; q.sD = as;
-    if (timed(PC_POLY, poly_flops, 0.0, stream, who, [&] { return launch_nt(q, tile, stream); }))
-      return 1;
-    // X' = P X + a X (scale kNsKx kept); the final step writes U = X' / kNsKx
-    NtArgs g{};
-    g.elt = ELT_F16;
-    g.A = w.Pm; g.lda = m_pad; g.sA = as;
-    g.B = x_cur; g.ldb = n_pad; g.sB = xs; g.b_kmajor = 1;
-    g.M = m_pad; g.N = n_pad; g.K = m_pad; g.L = batch; g.k_loop = km;
-    g.live_rows = km < m_pad ? km : 0;
-    g.live_cols = kn < n_pad ? kn : 0;
-    g.mt = m_pad / tile; g.nt = n_pad / tile; g.tiles_per_mat = g.mt * g.nt; g.tri = 0;
-    g.alpha = it + 1 < T ? 1.f : 1.f / kNsKx; g.beta = ca;
-    g.alpha_dev = it == 0 ? w.ratio : nullptr;
-    g.C = x_cur; g.ldc = n_pad; g.sC = xs;
-    if (it + 1 < T) {
-      g.mode = EPI_NS;
-      g.D = x_nxt; g.ldd = n_pad; g.sD = xs;   // X is the B operand: the new X goes elsewhere
-      if (timed(PC_GEMM, gemm_flops, 0.0, stream, who, [&] { return launch_nt(g, tile, stream); }))
-        return 1;
-      uint16_t* t = x_cur; x_cur = x_nxt; x_nxt = t;
-    } else {
-      g.mode = EPI_FINAL;
-      g.out_ptrs = out_ptrs; g.out_dtype = out_dtype;
-      g.w_ptrs = w_ptrs; g.w_dtype = w_dtype; g.decay = decay; g.lrs = lrs;
-      g.pub_ptrs = pub_ptrs; g.pub_dtype = pub_dtype;
-      g.m_real = m; g.n_real = n; g.transposed = tall ? 1 : 0; g.n_flip = n_flip;
-      if (timed(PC_FINAL, gemm_flops, wbytes + obytes + pbytes, stream, who,
-                [&] { return launch_nt(g, tile, stream); }))
-        return 1;
-    }
-  }
-  return 0;
+  if (group_setup(c, tile_req, backend, workspace, workspace_bytes, phases)) return 1;
+  if ((phases & PH_STAGE) && run_stage(c, mu, nesterov, eps)) return 1;
+  if (!(phases & PH_APPLY)) return 0;
+  return backend == DMUON_NS_GRAM ? run_gram(c, coeffs, T, restarts, n_restarts, decay)
+                                  : run_direct(c, coeffs, T, decay);
 }
+
+// The update scale of a shape, lr * 0.2 sqrt(max(rows, cols)), and the weight decay factor: host
+// scalars in double, rounded once to fp32, as torch does with Python-float arguments.
+float update_scale(double lr, int rows, int cols) {
+  return (float)(lr * (0.2 * sqrt((double)(rows > cols ? rows : cols))));
+}
+float decay_of(double lr, double wd) { return wd > 0.0 ? (float)(1.0 - lr * wd) : 1.f; }
 
 // ---- scratch of dmuon_muon_step_group_noalloc (the array itself is at file scope above) --------
 constexpr int64_t kScratchBytes = DMUON_NOALLOC_SCRATCH_BYTES;
@@ -1161,6 +1297,22 @@ int dmuon_ns_plan(int rows, int cols, int batch, int tile_req, int num_cus, int 
               workspace_bytes);
 }
 
+// The one group of the single-group entry points.
+static Group one_group(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs,
+                       float* const* est_ptrs, void* const* w_ptrs, int w_dtype,
+                       void* const* pub_ptrs, int pub_dtype, int rows, int cols, int batch,
+                       int n_transposed, int first_step, double lr) {
+  Group g{};
+  g.g_ptrs = g_ptrs; g.g_dtype = g_dtype;
+  g.buf_ptrs = buf_ptrs; g.est_ptrs = est_ptrs;
+  g.w_ptrs = w_ptrs; g.w_dtype = w_dtype;
+  g.pub_ptrs = pub_ptrs; g.pub_dtype = pub_dtype;
+  g.rows = rows; g.cols = cols; g.batch = batch; g.n_t = n_transposed;
+  g.first_step = first_step;
+  g.lrs = update_scale(lr, rows, cols);
+  return g;
+}
+
 int dmuon_muon_step_group(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs,
                           float* const* est_ptrs, void* const* w_ptrs, int w_dtype,
                           void* const* pub_ptrs, int pub_dtype, int rows, int cols, int batch,
@@ -1172,14 +1324,11 @@ int dmuon_muon_step_group(void* const* g_ptrs, int g_dtype, float* const* buf_pt
   const char* who = "dmuon_muon_step_group";
   if (batch == 0) return 0;
   if (!buf_ptrs || !w_ptrs) return fail("%s: buf_ptrs and w_ptrs must be non-NULL", who);
-  // host scalars in double, rounded once to fp32, as torch does with Python-float arguments
-  const double scale = 0.2 * sqrt((double)(rows > cols ? rows : cols));
-  const float decay = wd > 0.0 ? (float)(1.0 - lr * wd) : 1.f;
-  const float lrs = (float)(lr * scale);
-  return run_group(g_ptrs, g_dtype, buf_ptrs, est_ptrs, w_ptrs, w_dtype, pub_ptrs, pub_dtype,
-                   nullptr, 0, rows, cols, batch, n_transposed, (float)mu, nesterov, first_step,
-                   decay, lrs, coeffs, T, backend, restarts, n_restarts, eps, workspace, workspace_bytes, tile,
-                   static_cast<hipStream_t>(stream), who);
+  Group g = one_group(g_ptrs, g_dtype, buf_ptrs, est_ptrs, w_ptrs, w_dtype, pub_ptrs, pub_dtype,
+                      rows, cols, batch, n_transposed, first_step, lr);
+  Call c{&g, 1, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, (float)mu, nesterov, decay_of(lr, wd), coeffs, T, backend, restarts,
+                    n_restarts, eps, workspace, workspace_bytes, tile);
 }
 
 int dmuon_muon_step_group_noalloc(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs,
@@ -1205,13 +1354,11 @@ int dmuon_muon_step_group_noalloc(void* const* g_ptrs, int g_dtype, float* const
   void* ws = nullptr;
   if (scratch_of_current_device(who, &ws, true, static_cast<hipStream_t>(stream))) return 1;
   NoEvents no_events;
-  const double scale = 0.2 * sqrt((double)(rows > cols ? rows : cols));
-  const float decay = wd > 0.0 ? (float)(1.0 - lr * wd) : 1.f;
-  const float lrs = (float)(lr * scale);
-  return run_group(g_ptrs, g_dtype, buf_ptrs, est_ptrs, w_ptrs, w_dtype, pub_ptrs, pub_dtype,
-                   nullptr, 0, rows, cols, batch, n_transposed, (float)mu, nesterov, first_step,
-                   decay, lrs, coeffs, T, backend, restarts, n_restarts, eps, ws, kScratchBytes, tile,
-                   static_cast<hipStream_t>(stream), who);
+  Group g = one_group(g_ptrs, g_dtype, buf_ptrs, est_ptrs, w_ptrs, w_dtype, pub_ptrs, pub_dtype,
+                      rows, cols, batch, n_transposed, first_step, lr);
+  Call c{&g, 1, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, (float)mu, nesterov, decay_of(lr, wd), coeffs, T, backend, restarts,
+                    n_restarts, eps, ws, kScratchBytes, tile);
 }
 
 int dmuon_noalloc_init(void** scratch_out, int64_t* scratch_bytes) {
@@ -1230,10 +1377,12 @@ int dmuon_newton_schulz_group(void* const* g_ptrs, int g_dtype, void* const* out
   const char* who = "dmuon_newton_schulz_group";
   if (batch == 0) return 0;
   if (!out_ptrs) return fail("%s: out_ptrs must be non-NULL", who);
-  return run_group(g_ptrs, g_dtype, nullptr, nullptr, nullptr, 0, nullptr, 0, out_ptrs, out_dtype,
-                   rows, cols, batch, n_transposed, 0.f, 0, 1, 1.f, 0.f, coeffs, T, backend,
-                   restarts, n_restarts, eps, workspace, workspace_bytes, tile,
-                   static_cast<hipStream_t>(stream), who);
+  Group g = one_group(g_ptrs, g_dtype, nullptr, nullptr, nullptr, 0, nullptr, 0, rows, cols, batch,
+                      n_transposed, 1, 0.0);
+  g.out_ptrs = out_ptrs; g.out_dtype = out_dtype;
+  Call c{&g, 1, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, 0.f, 0, 1.f, coeffs, T, backend, restarts, n_restarts, eps, workspace,
+                    workspace_bytes, tile);
 }
 
 int dmuon_muon_stage_group(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs,
@@ -1244,11 +1393,11 @@ int dmuon_muon_stage_group(void* const* g_ptrs, int g_dtype, float* const* buf_p
   const char* who = "dmuon_muon_stage_group";
   if (batch == 0) return 0;
   if (!buf_ptrs) return fail("%s: buf_ptrs must be non-NULL", who);
-  return run_group(g_ptrs, g_dtype, buf_ptrs, est_ptrs, nullptr, 0, nullptr, 0, nullptr, 0, rows,
-                   cols, batch, n_transposed, (float)mu, nesterov, first_step, 1.f, 0.f, nullptr,
-                   0, backend,
-                   nullptr, 0, eps, workspace, workspace_bytes, tile,
-                   static_cast<hipStream_t>(stream), who, PH_STAGE);
+  Group g = one_group(g_ptrs, g_dtype, buf_ptrs, est_ptrs, nullptr, 0, nullptr, 0, rows, cols,
+                      batch, n_transposed, first_step, 0.0);
+  Call c{&g, 1, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, (float)mu, nesterov, 1.f, nullptr, 0, backend, nullptr, 0, eps, workspace,
+                    workspace_bytes, tile, PH_STAGE);
 }
 
 int dmuon_muon_apply_group(void* const* w_ptrs, int w_dtype, void* const* pub_ptrs,
@@ -1260,13 +1409,70 @@ int dmuon_muon_apply_group(void* const* w_ptrs, int w_dtype, void* const* pub_pt
   const char* who = "dmuon_muon_apply_group";
   if (batch == 0) return 0;
   if (!w_ptrs) return fail("%s: w_ptrs must be non-NULL", who);
-  const double scale = 0.2 * sqrt((double)(rows > cols ? rows : cols));
-  const float decay = wd > 0.0 ? (float)(1.0 - lr * wd) : 1.f;
-  const float lrs = (float)(lr * scale);
-  return run_group(nullptr, 0, nullptr, nullptr, w_ptrs, w_dtype, pub_ptrs, pub_dtype, nullptr, 0,
-                   rows, cols, batch, n_transposed, 0.f, 0, 0, decay, lrs, coeffs, T, backend,
-                   restarts, n_restarts, 0.f, workspace, workspace_bytes, tile, static_cast<hipStream_t>(stream), who,
-                   PH_APPLY);
+  Group g = one_group(nullptr, 0, nullptr, nullptr, w_ptrs, w_dtype, pub_ptrs, pub_dtype, rows,
+                      cols, batch, n_transposed, 0, lr);
+  Call c{&g, 1, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, 0.f, 0, decay_of(lr, wd), coeffs, T, backend, restarts, n_restarts, 0.f,
+                    workspace, workspace_bytes, tile, PH_APPLY);
+}
+
+// The groups of a several-shapes entry point, from the caller's descriptors.
+static int caller_groups(const char* who, const dmuon_muon_group* groups, int n, double lr,
+                         Group* out) {
+  if (n < 1 || n > DMUON_MAX_GROUPS || !groups)
+    return fail("%s: needs 1 .. %d groups, got %d", who, DMUON_MAX_GROUPS, n);
+  for (int i = 0; i < n; ++i) {
+    const dmuon_muon_group& d = groups[i];
+    out[i] = one_group(d.g_ptrs, d.g_dtype, d.buf_ptrs, d.est_ptrs, d.w_ptrs, d.w_dtype,
+                       d.pub_ptrs, d.pub_dtype, d.rows, d.cols, d.batch, d.n_transposed,
+                       d.first_step, lr);
+  }
+  return 0;
+}
+static_assert(DMUON_MAX_GROUPS == kMaxGroups, "groups of a call and of a launch");
+
+int dmuon_muon_plan_groups(const dmuon_muon_group* groups, int n, int tile, int num_cus,
+                           int backend, int* tile_out, int64_t* workspace_bytes,
+                           double* cost_us) {
+  const char* who = "dmuon_muon_plan_groups";
+  if (!groups || n < 1 || n > DMUON_MAX_GROUPS)
+    return fail("%s: needs 1 .. %d groups, got %d", who, DMUON_MAX_GROUPS, n);
+  if (!tile_out || !workspace_bytes) return fail("%s: NULL output", who);
+  if (backend != DMUON_NS_DIRECT && backend != DMUON_NS_GRAM)
+    return fail("%s: unknown NS backend %d", who, backend);
+  return plan_groups(groups, n, tile, num_cus, backend == DMUON_NS_GRAM, tile_out,
+                     workspace_bytes, cost_us);
+}
+
+int dmuon_muon_stage_groups(const dmuon_muon_group* groups, int n, double mu, int nesterov,
+                            int backend, float eps, void* workspace, int64_t workspace_bytes,
+                            int tile, void* stream) {
+  const char* who = "dmuon_muon_stage_groups";
+  Group g[kMaxGroups];
+  if (caller_groups(who, groups, n, 0.0, g)) return 1;
+  for (int i = 0; i < n; ++i)
+    if (!g[i].buf_ptrs) return fail("%s: buf_ptrs must be non-NULL", who);
+  if (n > 1 && tile != 128 && tile != 256)
+    return fail("%s: several groups need the tile of their plan (128 or 256), got %d", who, tile);
+  Call c{g, n, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, (float)mu, nesterov, 1.f, nullptr, 0, backend, nullptr, 0, eps, workspace,
+                    workspace_bytes, tile, PH_STAGE);
+}
+
+int dmuon_muon_apply_groups(const dmuon_muon_group* groups, int n, double lr, double wd,
+                            const float* coeffs, int T, int backend, const int* restarts,
+                            int n_restarts, void* workspace, int64_t workspace_bytes, int tile,
+                            void* stream) {
+  const char* who = "dmuon_muon_apply_groups";
+  Group g[kMaxGroups];
+  if (caller_groups(who, groups, n, lr, g)) return 1;
+  for (int i = 0; i < n; ++i)
+    if (!g[i].w_ptrs) return fail("%s: w_ptrs must be non-NULL", who);
+  if (n > 1 && tile != 128 && tile != 256)
+    return fail("%s: several groups need the tile of their plan (128 or 256), got %d", who, tile);
+  Call c{g, n, 0, static_cast<hipStream_t>(stream), who};
+  return run_groups(c, 0.f, 0, decay_of(lr, wd), coeffs, T, backend, restarts, n_restarts, 0.f,
+                    workspace, workspace_bytes, tile, PH_APPLY);
 }
 
 }  // extern "C"

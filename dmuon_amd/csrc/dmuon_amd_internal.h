@@ -69,8 +69,21 @@ struct NtArgs {
 enum { DIAG_SKIP_NONE = 0, DIAG_SKIP_WAVES = 1, DIAG_SKIP_BLOCKS = 2 };
 enum { C_NONE = 0, C_IS_A = 1, C_IS_B = 2 };
 
+// Products of several shapes in one launch: group g's tiles are the logical tiles first[g] ..
+// first[g + 1] - 1. All have the same mode, element type and B layout. The whole table is a
+// kernel argument (8 x ~330 bytes, under the 4 KiB of a launch).
+constexpr int kMaxGroups = 8;
+struct NtBatch {
+  int n;
+  int first[kMaxGroups + 1];
+  NtArgs a[kMaxGroups];
+};
+
 // Launches the NT MFMA kernel; picks the tile configuration from args (tile = 256 or 128).
 hipError_t launch_nt(const NtArgs& a, int tile, hipStream_t stream);
+// The same for n (1 .. kMaxGroups) fp16 products of one mode and B layout, in one launch. A
+// value's bits do not depend on what else the launch holds.
+hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream);
 // The logical tile the NT kernels give hardware block b of a launch of nb blocks (host copy of
 // the device mapping, for tests: it must be a permutation of 0 .. nb - 1).
 int nt_block_tile(int b, int nb);
@@ -101,6 +114,14 @@ struct PreArgs {
   int skip_y, skip_yt;
 };
 hipError_t launch_pre(const PreArgs& a, hipStream_t stream);
+// The same stage over n (1 .. 2 kMaxGroups) sets of matrices: one launch per kernel that some of
+// them need, or, for a PRE_F16 pass over flagged matrices, one launch.
+hipError_t launch_pre_batch(const PreArgs* a, int n, hipStream_t stream);
+struct PreBatch {
+  int n;
+  unsigned first[2 * kMaxGroups + 1];     // first block of each set
+  PreArgs a[2 * kMaxGroups];
+};
 int pre_blocks_per_mat(int Rp, int Cp);
 
 
@@ -112,10 +133,18 @@ hipError_t launch_norm_finalize(const float* partials, int nparts, int L, float 
 // est = *est_ptrs[l] > 0 and r = scale / est in [1/4, 4], ratio[l] = r, ratio_sq[l] = r^2 and
 // restage[l] = 0 (the staged copy times r is the exactly scaled one); otherwise ratio = 1,
 // ratio_sq = 1, restage = 1 (stage again with the exact scale). *est_ptrs[l] becomes scale.
-hipError_t launch_norm_finalize_est(const float* partials, int nparts, int L, float eps,
-                                    float* scale, float* scale_sq, float* const* est_ptrs,
-                                    float* ratio, float* ratio_sq, int* restage,
-                                    hipStream_t stream);
+// One launch for up to kMaxGroups groups of matrices.
+struct NormArgs {
+  const float* partials; int nparts, L;
+  float* scale; float* scale_sq; float* const* est_ptrs;
+  float* ratio; float* ratio_sq; int* restage;
+};
+struct NormBatch {
+  int n;
+  int first[kMaxGroups + 1];              // first matrix of each group
+  NormArgs a[kMaxGroups];
+};
+hipError_t launch_norm_finalize_est(const NormArgs* a, int n, float eps, hipStream_t stream);
 
 // dst[l][r][c] = r < rows && c < cols ? src[l][r][c] : 0 over rows_out x cols_out (16-bit)
 // dst = src, n16 chunks of 16 bytes (both 16-byte aligned, not overlapping)

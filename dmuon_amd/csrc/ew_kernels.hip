@@ -216,21 +216,35 @@ __device__ __forceinline__ float pre_tile(const PreArgs& a, int l, int r0, int c
   return ss;
 }
 
+// The set of matrices a staging block works on, and the block's index among that set's blocks
+// (matrix by matrix). A launch holds one set (PreArgs) or several of different shapes (PreBatch).
+__device__ __forceinline__ const PreArgs& block_args(const PreArgs& p, unsigned& b) {
+  b = blockIdx.x;
+  return p;
+}
+__device__ __forceinline__ const PreArgs& block_args(const PreBatch& p, unsigned& b) {
+  int g = 0;
+  while (g + 1 < p.n && blockIdx.x >= p.first[g + 1]) ++g;
+  g = __builtin_amdgcn_readfirstlane(g);
+  b = blockIdx.x - p.first[g];
+  return p.a[g];
+}
+
 // Partial sums of ns_in^2: one per 1024 elements' unit of work of whichever staging kernel ran
 // (a wave of a 64x64 tile, a 1024-element block of a wide matrix, four rows of a tall one's 64 x
 // 256 tile), (Rp / 32) * (Cp / 32) per matrix, summed in a fixed order by the norm finalize.
-template <int ST>
-__global__ __launch_bounds__(256) void muon_pre_kernel(const PreArgs a) {
+template <int ST, class ARGS>
+__global__ __launch_bounds__(256) void muon_pre_kernel(const ARGS args) {
   __shared__ __attribute__((aligned(16))) uint16_t tileT[kTile][kTile + kPad];
   const int tid = threadIdx.x;
-  float ss = pre_tile<ST>(a, blockIdx.z, blockIdx.y * kTile, blockIdx.x * kTile, tileT);
+  unsigned blk;
+  const PreArgs& a = block_args(args, blk);
+  const unsigned tx = a.Cp / kTile, per = tx * (a.Rp / kTile);
+  const unsigned l = blk / per, t = blk - l * per;
+  float ss = pre_tile<ST>(a, l, (int)(t / tx) * kTile, (int)(t % tx) * kTile, tileT);
   if constexpr (ST == PRE_F16) return;
   ss = wave_sum(ss);
-  if ((tid & 63) == 0) {
-    const long long blk = (long long)blockIdx.z * gridDim.x * gridDim.y +
-                          blockIdx.y * gridDim.x + blockIdx.x;
-    a.partials[blk * 4 + (tid >> 6)] = ss;
-  }
+  if ((tid & 63) == 0) a.partials[(long long)blk * 4 + (tid >> 6)] = ss;
 }
 
 // The per-element arithmetic of every staging kernel (the reference's order of roundings):
@@ -295,10 +309,13 @@ __device__ __forceinline__ float pre_scale(const PreArgs& a, int l, bool& copy) 
 // against 67% for the 64x64 tiles (whose wave instructions cover four 256-byte row pieces), and
 // 58-70% for 8 elements per thread or several pieces per block. The copy is stored non-temporal:
 // the products read it only after the whole batch is staged.
-template <int ST, bool GF>
-__global__ __launch_bounds__(256) void muon_pre_wide_kernel(const PreArgs a) {
-  const int l = blockIdx.y;
-  const long long i = (long long)blockIdx.x * 1024 + 4 * threadIdx.x;
+template <int ST, bool GF, class ARGS>
+__global__ __launch_bounds__(256) void muon_pre_wide_kernel(const ARGS args) {
+  unsigned blk;
+  const PreArgs& a = block_args(args, blk);
+  const unsigned per = (unsigned)((long long)a.rows * a.cols / 1024);
+  const unsigned l = blk / per;
+  const long long i = (long long)(blk - l * per) * 1024 + 4 * threadIdx.x;
   const void* g = a.g_ptrs[l];
   float* buf = a.buf_ptrs ? a.buf_ptrs[l] : nullptr;
   const bool read_buf = buf && (ST == PRE_F16 || !a.first_step);
@@ -329,7 +346,7 @@ __global__ __launch_bounds__(256) void muon_pre_wide_kernel(const PreArgs a) {
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   if (threadIdx.x == 0)
-    a.partials[(long long)l * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    a.partials[blk] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // Tall orientation without padding (rows % 64 == 0, cols % 256 == 0; only the transposed copy
@@ -338,13 +355,16 @@ __global__ __launch_bounds__(256) void muon_pre_wide_kernel(const PreArgs a) {
 // in the wide kernel), eight rows' loads in flight; the copy goes through LDS and leaves as X rows
 // of 64 values (128-byte runs). Measured on a 32 x 14336x4096 batch: 76% of 8 TB/s against 65%
 // for the 64x64 tiles (128 x 256 tiles: 74%, four rows in flight: 75%).
-template <int ST, bool GF>
-__global__ __launch_bounds__(256) void muon_pre_tall_kernel(const PreArgs a) {
+template <int ST, bool GF, class ARGS>
+__global__ __launch_bounds__(256) void muon_pre_tall_kernel(const ARGS args) {
   constexpr int TR = 64, TC = 256, RB = 8;
   __shared__ __attribute__((aligned(16))) uint16_t tt[TC][TR + kPad];
-  const int l = blockIdx.z;
+  unsigned blk;
+  const PreArgs& a = block_args(args, blk);
+  const unsigned tx = a.cols / TC, per = tx * (a.rows / TR);
+  const unsigned l = blk / per, t = blk - l * per;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const long long r0 = (long long)blockIdx.y * TR, c0 = (long long)blockIdx.x * TC;
+  const long long r0 = (long long)(t / tx) * TR, c0 = (long long)(t % tx) * TC;
   const int c = 4 * lane;
   const void* g = a.g_ptrs[l];
   float* buf = a.buf_ptrs ? a.buf_ptrs[l] : nullptr;
@@ -400,26 +420,33 @@ __global__ __launch_bounds__(256) void muon_pre_tall_kernel(const PreArgs a) {
     }
   }
   if constexpr (ST == PRE_F16) return;
-  const long long blk = (long long)l * gridDim.x * gridDim.y + blockIdx.y * gridDim.x + blockIdx.x;
 #pragma unroll
   for (int j = 0; j < TR / 16; ++j) {
     const float s = wave_sum(ss[j]);
-    if (lane == 0) a.partials[blk * 16 + w * 4 + j] = s;
+    if (lane == 0) a.partials[(long long)blk * 16 + w * 4 + j] = s;
   }
 }
 
 // The exact-scale copy for the matrices flagged in a.restage (a scale that moved by more than
 // 4x, or none kept yet). Rarely any are, so the grid is small and strides over the tiles of
-// the flagged matrices only; with nothing flagged each block reads L flags and exits.
-__global__ __launch_bounds__(256) void muon_restage_kernel(const PreArgs a) {
+// the flagged matrices only; with nothing flagged each block reads the flags and exits.
+template <class ARGS>
+__global__ __launch_bounds__(256) void muon_restage_kernel(const ARGS args) {
   __shared__ __attribute__((aligned(16))) uint16_t tileT[kTile][kTile + kPad];
-  const int tx = a.Cp / kTile, per = tx * (a.Rp / kTile);
-  for (int l = 0; l < a.L; ++l) {
-    if (!a.restage[l]) continue;   // block-uniform
-    for (int t = blockIdx.x; t < per; t += gridDim.x) {
-      __syncthreads();   // the previous tile's transposed read of tileT is done
-      pre_tile<PRE_F16>(a, l, (t / tx) * kTile, (t % tx) * kTile, tileT);
+  auto restage = [&](const PreArgs& a) {
+    const int tx = a.Cp / kTile, per = tx * (a.Rp / kTile);
+    for (int l = 0; l < a.L; ++l) {
+      if (!a.restage[l]) continue;   // block-uniform
+      for (int t = blockIdx.x; t < per; t += gridDim.x) {
+        __syncthreads();   // the previous tile's transposed read of tileT is done
+        pre_tile<PRE_F16>(a, l, (t / tx) * kTile, (t % tx) * kTile, tileT);
+      }
     }
+  };
+  if constexpr (std::is_same<ARGS, PreArgs>::value) {
+    restage(args);
+  } else {
+    for (int g = 0; g < args.n; ++g) restage(args.a[g]);
   }
 }
 
@@ -486,31 +513,34 @@ __global__ __launch_bounds__(256) void muon_update_kernel(const UpdateArgs a) {
   }
 }
 
-__global__ __launch_bounds__(kFinThreads) void norm_finalize_est_kernel(
-    const float* partials, int nparts, float eps, float* scale, float* scale_sq,
-    float* const* est_ptrs, float* ratio, float* ratio_sq, int* restage) {
+__global__ __launch_bounds__(kFinThreads) void norm_finalize_est_kernel(const NormBatch b,
+                                                                        float eps) {
   __shared__ double red[kFinThreads];
-  const int l = blockIdx.x;
-  sum_partials(partials, nparts, l, red);
+  int g = 0;
+  while (g + 1 < b.n && (int)blockIdx.x >= b.first[g + 1]) ++g;
+  g = __builtin_amdgcn_readfirstlane(g);
+  const NormArgs& a = b.a[g];
+  const int l = blockIdx.x - b.first[g];
+  sum_partials(a.partials, a.nparts, l, red);
   if (threadIdx.x == 0) {
     const float nrm = (float)sqrt(red[0]);
     const float sc = 1.0f / (nrm + eps);
-    scale[l] = sc;
-    scale_sq[l] = sc * sc;
+    a.scale[l] = sc;
+    a.scale_sq[l] = sc * sc;
     float r = 1.f;
     bool ok = false;
-    if (est_ptrs) {
-      const float est = *est_ptrs[l];
+    if (a.est_ptrs) {
+      const float est = *a.est_ptrs[l];
       if (est > 0.f) {
         r = sc / est;
         ok = r >= 0.25f && r <= 4.f;   // false for NaN / inf too
       }
-      *est_ptrs[l] = sc;
+      *a.est_ptrs[l] = sc;
     }
     if (!ok) r = 1.f;
-    ratio[l] = r;
-    ratio_sq[l] = r * r;
-    restage[l] = ok ? 0 : 1;
+    a.ratio[l] = r;
+    a.ratio_sq[l] = r * r;
+    a.restage[l] = ok ? 0 : 1;
   }
 }
 
@@ -562,50 +592,101 @@ hipError_t launch_pad_copy(const uint16_t* src, long long lds, long long ss, uin
 
 int pre_blocks_per_mat(int Rp, int Cp) { return (Rp / 32) * (Cp / 32); }
 
-hipError_t launch_pre(const PreArgs& a, hipStream_t stream) {
-  dim3 block(256);
-  if (a.stage == PRE_F16 && a.restage) {
-    const int tiles = (a.Rp / kTile) * (a.Cp / kTile);
-    hipLaunchKernelGGL(muon_restage_kernel, dim3(std::min(tiles, 2048)), block, 0, stream, a);
-    return hipGetLastError();
-  }
-  // Which copy the launch writes: Y (the gradient's layout), YT (transposed), both or none
-  // (PRE_NORM writes none). Unpadded matrices with one copy take the contiguous-run kernels;
-  // everything else (padding, both copies) the 64x64 tiles. All three write the same partials
-  // layout size, (Rp / 32) * (Cp / 32) per matrix.
+namespace {
+
+// Which staging kernel a set of matrices takes. Which copy the launch writes: Y (the gradient's
+// layout), YT (transposed), both or none (PRE_NORM writes none). Unpadded matrices with one copy
+// take the contiguous-run kernels; everything else (padding, both copies) the 64x64 tiles. All
+// three write the same partials layout size, (Rp / 32) * (Cp / 32) per matrix.
+enum PreKernel { PRE_TILES, PRE_WIDE_BF16, PRE_WIDE_F32, PRE_TALL_BF16, PRE_TALL_F32, PRE_KERNELS };
+PreKernel pre_kernel_of(const PreArgs& a) {
   const bool y = a.stage != PRE_NORM && !a.skip_y, yt = a.stage != PRE_NORM && !a.skip_yt;
-  const bool unpadded = a.Rp == a.rows && a.Cp == a.cols;
+  const bool unpadded = a.Rp == a.rows && a.Cp == a.cols, gf = a.g_dtype == DT_F32;
   const bool wide = unpadded && !yt && (!y || a.ldy == a.cols);
-  const bool tall = !wide && unpadded && !y && a.rows % 64 == 0 && a.cols % 256 == 0;
-#define DMUON_PRE(KERNEL, GRID, ...)                                                           \
-  do {                                                                                         \
-    if (a.stage == PRE_NORM)                                                                   \
-      hipLaunchKernelGGL((KERNEL<PRE_NORM __VA_ARGS__>), GRID, block, 0, stream, a);           \
-    else if (a.stage == PRE_F16)                                                               \
-      hipLaunchKernelGGL((KERNEL<PRE_F16 __VA_ARGS__>), GRID, block, 0, stream, a);            \
-    else if (a.stage == PRE_EST)                                                               \
-      hipLaunchKernelGGL((KERNEL<PRE_EST __VA_ARGS__>), GRID, block, 0, stream, a);            \
-    else                                                                                       \
-      hipLaunchKernelGGL((KERNEL<PRE_BF16 __VA_ARGS__>), GRID, block, 0, stream, a);           \
-  } while (0)
-  const bool gf = a.g_dtype == DT_F32;
-  const dim3 gwide((unsigned)((long long)a.rows * a.cols / 1024), a.L);
-  const dim3 gtall(a.cols / 256, a.rows / 64, a.L);
-  if (wide && gf) DMUON_PRE(muon_pre_wide_kernel, gwide, , true);
-  else if (wide) DMUON_PRE(muon_pre_wide_kernel, gwide, , false);
-  else if (tall && gf) DMUON_PRE(muon_pre_tall_kernel, gtall, , true);
-  else if (tall) DMUON_PRE(muon_pre_tall_kernel, gtall, , false);
-  else DMUON_PRE(muon_pre_kernel, dim3(a.Cp / kTile, a.Rp / kTile, a.L));
-#undef DMUON_PRE
-  return hipGetLastError();
+  if (wide) return gf ? PRE_WIDE_F32 : PRE_WIDE_BF16;
+  if (unpadded && !y && a.rows % 64 == 0 && a.cols % 256 == 0)
+    return gf ? PRE_TALL_F32 : PRE_TALL_BF16;
+  return PRE_TILES;
+}
+long long pre_blocks_of(PreKernel k, const PreArgs& a) {
+  if (k == PRE_WIDE_BF16 || k == PRE_WIDE_F32) return (long long)a.rows * a.cols / 1024 * a.L;
+  if (k == PRE_TALL_BF16 || k == PRE_TALL_F32) return (long long)(a.cols / 256) * (a.rows / 64) * a.L;
+  return (long long)(a.Cp / kTile) * (a.Rp / kTile) * a.L;
 }
 
-hipError_t launch_norm_finalize_est(const float* partials, int nparts, int L, float eps,
-                                    float* scale, float* scale_sq, float* const* est_ptrs,
-                                    float* ratio, float* ratio_sq, int* restage,
-                                    hipStream_t stream) {
-  hipLaunchKernelGGL(norm_finalize_est_kernel, dim3(L), dim3(kFinThreads), 0, stream, partials,
-                     nparts, eps, scale, scale_sq, est_ptrs, ratio, ratio_sq, restage);
+template <int ST, class ARGS>
+void launch_pre_stage(PreKernel k, const ARGS& p, unsigned blocks, hipStream_t stream) {
+  const dim3 grid(blocks), block(256);
+  if (k == PRE_WIDE_F32)
+    hipLaunchKernelGGL((muon_pre_wide_kernel<ST, true, ARGS>), grid, block, 0, stream, p);
+  else if (k == PRE_WIDE_BF16)
+    hipLaunchKernelGGL((muon_pre_wide_kernel<ST, false, ARGS>), grid, block, 0, stream, p);
+  else if (k == PRE_TALL_F32)
+    hipLaunchKernelGGL((muon_pre_tall_kernel<ST, true, ARGS>), grid, block, 0, stream, p);
+  else if (k == PRE_TALL_BF16)
+    hipLaunchKernelGGL((muon_pre_tall_kernel<ST, false, ARGS>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((muon_pre_kernel<ST, ARGS>), grid, block, 0, stream, p);
+}
+template <class ARGS>
+void launch_pre_kernel(PreKernel k, int stage, const ARGS& p, unsigned blocks, hipStream_t stream) {
+  if (stage == PRE_NORM) launch_pre_stage<PRE_NORM>(k, p, blocks, stream);
+  else if (stage == PRE_F16) launch_pre_stage<PRE_F16>(k, p, blocks, stream);
+  else if (stage == PRE_EST) launch_pre_stage<PRE_EST>(k, p, blocks, stream);
+  else launch_pre_stage<PRE_BF16>(k, p, blocks, stream);
+}
+
+}  // namespace
+
+hipError_t launch_pre_batch(const PreArgs* a, int n, hipStream_t stream) {
+  if (n < 1 || n > 2 * kMaxGroups) return hipErrorInvalidValue;
+  for (int i = 1; i < n; ++i)
+    if (a[i].stage != a[0].stage || !a[i].restage != !a[0].restage) return hipErrorInvalidValue;
+  PreBatch b;
+  if (a[0].stage == PRE_F16 && a[0].restage) {
+    int tiles = 1;
+    b.n = n;
+    for (int i = 0; i < n; ++i) {
+      b.a[i] = a[i];
+      tiles = std::max(tiles, (a[i].Rp / kTile) * (a[i].Cp / kTile));
+    }
+    const dim3 grid(std::min(tiles, 2048)), block(256);
+    if (n == 1) hipLaunchKernelGGL(muon_restage_kernel<PreArgs>, grid, block, 0, stream, a[0]);
+    else hipLaunchKernelGGL(muon_restage_kernel<PreBatch>, grid, block, 0, stream, b);
+    return hipGetLastError();
+  }
+  for (int k = 0; k < PRE_KERNELS; ++k) {
+    long long blocks = 0;
+    b.n = 0;
+    for (int i = 0; i < n; ++i) {
+      if (a[i].L <= 0 || pre_kernel_of(a[i]) != (PreKernel)k) continue;
+      b.first[b.n] = (unsigned)blocks;
+      b.a[b.n++] = a[i];
+      blocks += pre_blocks_of((PreKernel)k, a[i]);
+    }
+    if (blocks == 0) continue;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (b.n == 1) launch_pre_kernel((PreKernel)k, a[0].stage, b.a[0], (unsigned)blocks, stream);
+    else launch_pre_kernel((PreKernel)k, a[0].stage, b, (unsigned)blocks, stream);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t launch_pre(const PreArgs& a, hipStream_t stream) { return launch_pre_batch(&a, 1, stream); }
+
+hipError_t launch_norm_finalize_est(const NormArgs* a, int n, float eps, hipStream_t stream) {
+  if (n < 1 || n > kMaxGroups) return hipErrorInvalidValue;
+  NormBatch b;
+  b.n = n;
+  b.first[0] = 0;
+  for (int g = 0; g < n; ++g) {
+    b.a[g] = a[g];
+    b.first[g + 1] = b.first[g] + a[g].L;
+  }
+  hipLaunchKernelGGL(norm_finalize_est_kernel, dim3(b.first[n]), dim3(kFinThreads), 0, stream, b,
+                     eps);
   return hipGetLastError();
 }
 

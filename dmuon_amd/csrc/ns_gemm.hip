@@ -288,11 +288,27 @@ struct TilePos {
   int l, bi, bj;
 };
 
+// The product this block works on, and its tile among that product's tiles. A launch holds one
+// product (NtArgs) or several of different shapes (NtBatch); the XCD windows run over all of
+// the launch's tiles.
+__device__ __forceinline__ const NtArgs& block_args(const NtArgs& p, int& lb) {
+  lb = xcd_remap(blockIdx.x, gridDim.x);
+  return p;
+}
+__device__ __forceinline__ const NtArgs& block_args(const NtBatch& p, int& lb) {
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  int g = 0;
+  while (g + 1 < p.n && t >= p.first[g + 1]) ++g;
+  g = __builtin_amdgcn_readfirstlane(g);
+  lb = t - p.first[g];
+  return p.a[g];
+}
+
 // tile rows per group of the walks (with the XCD windows, 4 or 16 rows for the triangle walk
 // and 4 or 16 for the rectangular one measured 0.3-0.9% slower per c5 step)
 constexpr int kTileGroupTri = 8, kTileGroupRect = 8;
-__device__ __forceinline__ TilePos decode_tile(const NtArgs& a, int hb, int nblocks) {
-  const int lb = xcd_remap(hb, nblocks);
+// tile `lb` of the product's own tiles (matrix by matrix)
+__device__ __forceinline__ TilePos decode_tile(const NtArgs& a, int lb) {
   const int l = lb / a.tiles_per_mat;
   int t = lb - l * a.tiles_per_mat;
   int bi, bj;
@@ -754,11 +770,11 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
   }
 }
 
-template <int BM, int BN, int BK, int S, int WM, int WN, int MODE, int E, bool BKM>
+template <int BM, int BN, int BK, int S, int WM, int WN, int MODE, int E, bool BKM, class ARGS>
 __global__ __launch_bounds__(64 * WM * WN)
 __attribute__((amdgpu_waves_per_eu(Occupancy<BM, BN, BK, S, WM, WN>::WPE,
                                    Occupancy<BM, BN, BK, S, WM, WN>::WPE)))
-void nt_mfma_kernel(const NtArgs a) {
+void nt_mfma_kernel(const ARGS args) {
   using T = Tile<BM, BN, BK, S, WM, WN>;
   __shared__ __attribute__((aligned(16))) char smem[T::LDS_BYTES];
   static_assert(T::LDS_BYTES <= 160 * 1024, "LDS budget");
@@ -773,7 +789,9 @@ void nt_mfma_kernel(const NtArgs a) {
   // ---- tile decode -------------------------------------------------------------------
   // the decode is the same for every lane; readfirstlane states it, so the buffer descriptors
   // and offsets built from it stay scalar whatever the compiler's uniformity analysis proves
-  const TilePos tp = decode_tile(a, blockIdx.x, gridDim.x);
+  int lb;
+  const NtArgs& a = block_args(args, lb);
+  const TilePos tp = decode_tile(a, lb);
   const int l = __builtin_amdgcn_readfirstlane(tp.l);
   const int bi = __builtin_amdgcn_readfirstlane(tp.bi), bj = __builtin_amdgcn_readfirstlane(tp.bj);
   const int i0 = bi * BM, j0 = bj * BN;
@@ -1160,15 +1178,17 @@ __device__ __forceinline__ void pp_tile(const NtArgs& a, char* smem, int l, int 
                             wj);
 }
 
-template <int BK, int S, int MODE, int E, bool BKM>
+template <int BK, int S, int MODE, int E, bool BKM, class ARGS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void nt_pp_kernel(const NtArgs a) {
+void nt_pp_kernel(const ARGS args) {
   using T = Tile<256, 256, BK, S, 2, 4>;
   __shared__ __attribute__((aligned(16))) char smem[T::LDS_BYTES];
   static_assert(T::LDS_BYTES <= 160 * 1024, "LDS budget");
   // the decode is the same for every lane; readfirstlane states it, so the buffer descriptors
   // and offsets built from it stay scalar whatever the compiler's uniformity analysis proves
-  const TilePos tp = decode_tile(a, blockIdx.x, gridDim.x);
+  int lb;
+  const NtArgs& a = block_args(args, lb);
+  const TilePos tp = decode_tile(a, lb);
   const int l = __builtin_amdgcn_readfirstlane(tp.l);
   const int bi = __builtin_amdgcn_readfirstlane(tp.bi), bj = __builtin_amdgcn_readfirstlane(tp.bj);
   // Which copy of the schedule this wave runs (one call site each: pp_tile is inlined wherever
@@ -1233,145 +1253,162 @@ constexpr int kT128S = 4, kT128WN = 4;
 
 int nt_block_tile(int b, int nb) { return xcd_remap(b, nb); }
 
-hipError_t launch_nt(const NtArgs& a, int tile, hipStream_t stream) {
-  const long long nb = (long long)a.tiles_per_mat * a.L;
-  if (nb <= 0) return hipSuccess;
+namespace {
+
+// What a product may not be (no access of the kernels then leaves its operands).
+bool nt_args_ok(const NtArgs& a) {
   // the K loops run whole 64-wide slices, at least one
-  if (a.K <= 0 || a.K % 64 != 0) return hipErrorInvalidValue;
+  if (a.K <= 0 || a.K % 64 != 0) return false;
   // the second output relies on the exactly symmetric diagonal-tile path for its diagonal
-  if (a.D2 && !(a.mode == EPI_SYM && a.tri && a.sym_exact)) return hipErrorInvalidValue;
+  if (a.D2 && !(a.mode == EPI_SYM && a.tri && a.sym_exact)) return false;
   // an output to write: D for a symmetric product, D or D^T for an NS step
-  if ((a.mode == EPI_SYM && !a.D) || (a.mode == EPI_NS && !a.D && !a.DT))
-    return hipErrorInvalidValue;
+  if ((a.mode == EPI_SYM && !a.D) || (a.mode == EPI_NS && !a.D && !a.DT)) return false;
   // k-major B: whole-panel buffer range and slice offsets in 32 bits, rows of whole tiles
-  if (a.b_kmajor && ((long long)a.K * a.ldb * 2 >= (1LL << 31) || a.ldb < a.N))
-    return hipErrorInvalidValue;
+  if (a.b_kmajor && ((long long)a.K * a.ldb * 2 >= (1LL << 31) || a.ldb < a.N)) return false;
   // An addend named as one of the operands (the K-loop rotation's C_IS_A / C_IS_B) is read by
   // the epilogue as an M x N matrix at ldc: that is the operand itself only for a square
   // product (K == M == N) with the operand's own layout. Anything else would read the addend
   // past the operand's rows (a 4096 x 64 panel read as 4096 x 4096), so it is refused.
   if (a.c_in == C_IS_A &&
       !(a.C == a.A && a.K == a.M && a.M == a.N && a.ldc == a.lda && (a.L <= 1 || a.sC == a.sA)))
-    return hipErrorInvalidValue;
+    return false;
   if (a.c_in == C_IS_B &&
       !(a.C == a.B && a.K == a.M && a.M == a.N && a.ldc == a.ldb && (a.L <= 1 || a.sC == a.sB)))
-    return hipErrorInvalidValue;
-  if (a.c_in != C_NONE && a.c_in != C_IS_A && a.c_in != C_IS_B) return hipErrorInvalidValue;
-  if (a.k_loop < 0 || a.k_loop > a.K || a.k_loop % 64 != 0) return hipErrorInvalidValue;
+    return false;
+  if (a.c_in != C_NONE && a.c_in != C_IS_A && a.c_in != C_IS_B) return false;
+  if (a.k_loop < 0 || a.k_loop > a.K || a.k_loop % 64 != 0) return false;
   if (a.live_rows < 0 || a.live_rows % 64 != 0 || a.live_cols < 0 || a.live_cols % 64 != 0 ||
       (a.tri && a.live_rows != a.live_cols))
-    return hipErrorInvalidValue;
-  dim3 grid((unsigned)nb);
-#define DMUON_NT3(TILE, BK, S, WM, WN, E, KM)                                                  \
-  do {                                                                                         \
-    dim3 block(64 * WM * WN);                                                                  \
-    if (a.mode == EPI_SYM)                                                                     \
-      hipLaunchKernelGGL((nt_mfma_kernel<TILE, TILE, BK, S, WM, WN, EPI_SYM, E, KM>), grid,    \
-                         block, 0, stream, a);                                                 \
-    else if (a.mode == EPI_NS)                                                                 \
-      hipLaunchKernelGGL((nt_mfma_kernel<TILE, TILE, BK, S, WM, WN, EPI_NS, E, KM>), grid,     \
-                         block, 0, stream, a);                                                 \
-    else                                                                                       \
-      hipLaunchKernelGGL((nt_mfma_kernel<TILE, TILE, BK, S, WM, WN, EPI_FINAL, E, KM>), grid,  \
-                         block, 0, stream, a);                                                 \
-  } while (0)
-#define DMUON_NT(TILE, BK, S, WM, WN, E)                                                       \
-  do {                                                                                         \
-    if (a.b_kmajor) DMUON_NT3(TILE, BK, S, WM, WN, E, true);                                   \
-    else DMUON_NT3(TILE, BK, S, WM, WN, E, false);                                             \
-  } while (0)
-#define DMUON_PP3(E, KM)                                                                       \
-  do {                                                                                         \
-    dim3 block(512);                                                                           \
-    if (a.mode == EPI_SYM)                                                                     \
-      hipLaunchKernelGGL((nt_pp_kernel<64, 2, EPI_SYM, E, KM>), grid, block, 0, stream, a);    \
-    else if (a.mode == EPI_NS)                                                                 \
-      hipLaunchKernelGGL((nt_pp_kernel<64, 2, EPI_NS, E, KM>), grid, block, 0, stream, a);     \
-    else                                                                                       \
-      hipLaunchKernelGGL((nt_pp_kernel<64, 2, EPI_FINAL, E, KM>), grid, block, 0, stream, a);  \
-  } while (0)
-#define DMUON_PP(E)                                                                            \
-  do {                                                                                         \
-    if (a.b_kmajor) DMUON_PP3(E, true);                                                        \
-    else DMUON_PP3(E, false);                                                                  \
-  } while (0)
-  // 256-tiles: the ping-pong kernel, 8 waves, 64-wide K slices in a two-slot ring; 128-tiles:
-  // 4 waves, two blocks per CU, or, when every tile has a CU to itself, one block per CU with a
-  // four-slot ring (128 KiB). Measured and not kept: 32-wide slices in a four-slot ring for the
-  // ping-pong kernel (7-12% slower: twice the phases and barriers), the in-phase 8-wave schedule
-  // it replaced (3-11% slower on the c5 product shapes), 256-tiles of 4 waves with 128x128 per
-  // wave, and 32x32x16 MFMAs (identical results; 5-15% slower under the board power limit).
-  const int cus = current_device_cus();
-  if (tile == 128 && a.M % 256 == 0 && a.N % 256 == 0 && cus > 0) {
-    // A launch of more than two 128-tiles per CU whose result also splits into 256-tiles runs
-    // on the ping-pong kernel when that takes fewer units of work per CU, by the cost model of
-    // the planner (a wave of 256-tiles: 4 units; a wave of two 128-tiles per CU: 2.7). With
-    // both sides multiples of 256 the two kernels give the same bits, so only the time changes
-    // (e.g. Q X of one 1024 x 16384 matrix: 256 tiles in one wave instead of 1024 in two).
-    const int mt2 = a.M / 256, nt2 = a.N / 256;
-    const long long n256 = (long long)(a.tri ? mt2 * (mt2 + 1) / 2 : mt2 * nt2) * a.L;
-    const double c256 = 4.0 * (double)((n256 + cus - 1) / cus);
-    const double c128 = 2.7 * (double)((nb + 2LL * cus - 1) / (2LL * cus));
-    if (nb > 2LL * cus && c256 < c128) {
-      NtArgs s = a;
-      s.mt = mt2;
-      s.nt = nt2;
-      s.tiles_per_mat = (int)(n256 / a.L);
-      return launch_nt(s, 256, stream);
-    }
-  }
-  if (tile == 128) {
-    // The same products on 64x64 tiles (4 waves of 64x16, an eight-slot ring of 16 KiB slots,
-    // one block per CU) when those still fit one wave of blocks on the device: four times the
-    // CUs on a launch that waits on load latency. Every value keeps its K order -- the slice
-    // rotation depends only on the 256-aligned block of the tile's columns -- so the bits match
-    // the 128-tile kernel's. A k-major B is one 64-value block of 128-byte k-rows per slice.
-    NtArgs s = a;
-    s.mt = 2 * a.mt;
-    s.nt = 2 * a.nt;
-    s.tiles_per_mat = a.tri ? s.mt * (s.mt + 1) / 2 : s.mt * s.nt;
-    const long long nb64 = (long long)s.tiles_per_mat * a.L;
-    if (nb64 <= cus) {
-      dim3 g64((unsigned)nb64), b64(64 * kT64WN);
-#define DMUON_NT64K(E, KM)                                                                     \
-  do {                                                                                         \
-    if (s.mode == EPI_SYM)                                                                     \
-      hipLaunchKernelGGL((nt_mfma_kernel<64, 64, 64, kT64S, 1, kT64WN, EPI_SYM, E, KM>), g64, b64, 0,    \
-                         stream, s);                                                           \
-    else if (s.mode == EPI_NS)                                                                 \
-      hipLaunchKernelGGL((nt_mfma_kernel<64, 64, 64, kT64S, 1, kT64WN, EPI_NS, E, KM>), g64, b64, 0,     \
-                         stream, s);                                                           \
-    else                                                                                       \
-      hipLaunchKernelGGL((nt_mfma_kernel<64, 64, 64, kT64S, 1, kT64WN, EPI_FINAL, E, KM>), g64, b64, 0,  \
-                         stream, s);                                                           \
-  } while (0)
-#define DMUON_NT64(E)                                                                          \
-  do {                                                                                         \
-    if (s.b_kmajor) DMUON_NT64K(E, true);                                                      \
-    else DMUON_NT64K(E, false);                                                                \
-  } while (0)
-      if (a.elt == ELT_F16) DMUON_NT64(ELT_F16);
-      else DMUON_NT64(ELT_BF16);
-#undef DMUON_NT64
-#undef DMUON_NT64K
-      return hipGetLastError();
-    }
-  }
-  const bool deep = tile != 256 && nb <= cus;
-  if (a.elt == ELT_F16) {
-    if (tile == 256) DMUON_PP(ELT_F16);
-    else if (deep) DMUON_NT(128, 64, kT128S, 2, kT128WN, ELT_F16);
-    else DMUON_NT(128, 64, 2, 2, 2, ELT_F16);
-  } else {
-    if (tile == 256) DMUON_PP(ELT_BF16);
-    else if (deep) DMUON_NT(128, 64, kT128S, 2, kT128WN, ELT_BF16);
-    else DMUON_NT(128, 64, 2, 2, 2, ELT_BF16);
-  }
+    return false;
+  return true;
+}
+
+// The tile grid of a product on `tile` x `tile` tiles (M and N are multiples of it).
+void set_tiles(NtArgs& a, int tile) {
+  a.mt = a.M / tile;
+  a.nt = a.N / tile;
+  a.tiles_per_mat = a.tri ? a.mt * (a.mt + 1) / 2 : a.mt * a.nt;
+}
+
+// One launch of `nb` blocks: p is the one product, or the table of several.
+template <int BM, int S, int WM, int WN, int E, class ARGS>
+void launch_mfma(const ARGS& p, int mode, bool kmajor, long long nb, hipStream_t stream) {
+  const dim3 grid((unsigned)nb), block(64 * WM * WN);
+#define DMUON_NT(MODE, KM)                                                                     \
+  hipLaunchKernelGGL((nt_mfma_kernel<BM, BM, 64, S, WM, WN, MODE, E, KM, ARGS>), grid, block,  \
+                     0, stream, p)
+  if (mode == EPI_SYM) { if (kmajor) DMUON_NT(EPI_SYM, true); else DMUON_NT(EPI_SYM, false); }
+  else if (mode == EPI_NS) { if (kmajor) DMUON_NT(EPI_NS, true); else DMUON_NT(EPI_NS, false); }
+  else { if (kmajor) DMUON_NT(EPI_FINAL, true); else DMUON_NT(EPI_FINAL, false); }
 #undef DMUON_NT
-#undef DMUON_NT3
+}
+template <int E, class ARGS>
+void launch_pp(const ARGS& p, int mode, bool kmajor, long long nb, hipStream_t stream) {
+  const dim3 grid((unsigned)nb), block(512);
+#define DMUON_PP(MODE, KM)                                                                     \
+  hipLaunchKernelGGL((nt_pp_kernel<64, 2, MODE, E, KM, ARGS>), grid, block, 0, stream, p)
+  if (mode == EPI_SYM) { if (kmajor) DMUON_PP(EPI_SYM, true); else DMUON_PP(EPI_SYM, false); }
+  else if (mode == EPI_NS) { if (kmajor) DMUON_PP(EPI_NS, true); else DMUON_PP(EPI_NS, false); }
+  else { if (kmajor) DMUON_PP(EPI_FINAL, true); else DMUON_PP(EPI_FINAL, false); }
 #undef DMUON_PP
-#undef DMUON_PP3
+}
+
+// Which kernel runs a launch of a 128- or 256-tile plan.
+enum NtKernel { NT_PP256, NT_128, NT_128_DEEP, NT_64 };
+
+template <int E, class ARGS>
+void launch_kernel(NtKernel k, const ARGS& p, int mode, bool kmajor, long long nb,
+                   hipStream_t stream) {
+  if (k == NT_PP256) launch_pp<E>(p, mode, kmajor, nb, stream);
+  else if (k == NT_64) launch_mfma<64, kT64S, 1, kT64WN, E>(p, mode, kmajor, nb, stream);
+  else if (k == NT_128_DEEP) launch_mfma<128, kT128S, 2, kT128WN, E>(p, mode, kmajor, nb, stream);
+  else launch_mfma<128, 2, 2, 2, E>(p, mode, kmajor, nb, stream);
+}
+
+}  // namespace
+
+// 256-tiles: the ping-pong kernel, 8 waves, 64-wide K slices in a two-slot ring; 128-tiles:
+// 4 waves, two blocks per CU, or, when every tile has a CU to itself, one block per CU with a
+// four-slot ring (128 KiB). Measured and not kept: 32-wide slices in a four-slot ring for the
+// ping-pong kernel (7-12% slower: twice the phases and barriers), the in-phase 8-wave schedule
+// it replaced (3-11% slower on the c5 product shapes), 256-tiles of 4 waves with 128x128 per
+// wave, and 32x32x16 MFMAs (identical results; 5-15% slower under the board power limit).
+//
+// A 128-tile launch takes, over all of its products (every choice gives the same bits):
+//  - the ping-pong kernel, when it has more than two 128-tiles per CU, every result also splits
+//    into 256-tiles and that takes fewer units of work per CU by the cost model of the planner
+//    (a wave of 256-tiles: 4 units; a wave of two 128-tiles per CU: 2.7), e.g. Q X of one
+//    1024 x 16384 matrix: 256 tiles in one wave instead of 1024 in two;
+//  - 64x64 tiles (4 waves of 64x16, an eight-slot ring of 16 KiB slots, one block per CU) when
+//    those still fit one wave of blocks on the device: four times the CUs on a launch that
+//    waits on load latency. Every value keeps its K order -- the slice rotation depends only on
+//    the 256-aligned block of the tile's columns. A k-major B is one 64-value block of 128-byte
+//    k-rows per slice;
+//  - else 128-tiles.
+hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream) {
+  if (n < 1 || n > kMaxGroups) return hipErrorInvalidValue;
+  // the longest K loops first: their tiles must not start last
+  int order[kMaxGroups], cnt = 0;
+  for (int g = 0; g < n; ++g) {
+    if ((long long)a[g].tiles_per_mat * a[g].L <= 0) continue;
+    if (!nt_args_ok(a[g])) return hipErrorInvalidValue;
+    if (a[g].mode != a[0].mode || a[g].b_kmajor != a[0].b_kmajor || a[g].elt != a[0].elt)
+      return hipErrorInvalidValue;
+    const int k = a[g].k_loop > 0 ? a[g].k_loop : a[g].K;
+    int at = cnt++;
+    for (; at > 0; --at) {
+      const NtArgs& o = a[order[at - 1]];
+      if ((o.k_loop > 0 ? o.k_loop : o.K) >= k) break;
+      order[at] = order[at - 1];
+    }
+    order[at] = g;
+  }
+  if (cnt == 0) return hipSuccess;
+  if (cnt > 1 && a[order[0]].elt != ELT_F16) return hipErrorInvalidValue;
+  const int cus = current_device_cus();
+  long long nb = 0, nb256 = 0, nb64 = 0;
+  bool split256 = true;
+  for (int i = 0; i < cnt; ++i) {
+    const NtArgs& p = a[order[i]];
+    const long long t2 = p.M / 256, u2 = p.N / 256, t4 = p.M / 64, u4 = p.N / 64;
+    nb += (long long)p.tiles_per_mat * p.L;
+    nb256 += (p.tri ? t2 * (t2 + 1) / 2 : t2 * u2) * p.L;
+    nb64 += (p.tri ? t4 * (t4 + 1) / 2 : t4 * u4) * p.L;
+    split256 = split256 && p.M % 256 == 0 && p.N % 256 == 0;
+  }
+  NtKernel kernel = tile == 256 ? NT_PP256 : NT_128;
+  if (tile != 256 && cus > 0) {
+    const double c256 = 4.0 * (double)((nb256 + cus - 1) / cus);
+    const double c128 = 2.7 * (double)((nb + 2LL * cus - 1) / (2LL * cus));
+    if (split256 && nb > 2LL * cus && c256 < c128) kernel = NT_PP256, nb = nb256;
+    else if (nb64 <= cus) kernel = NT_64, nb = nb64;
+    else if (nb <= cus) kernel = NT_128_DEEP;
+  }
+  const int t = kernel == NT_PP256 ? 256 : kernel == NT_64 ? 64 : 128;
+  if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
+  const int mode = a[order[0]].mode;
+  const bool km = a[order[0]].b_kmajor != 0;
+  if (cnt == 1) {
+    NtArgs p = a[order[0]];
+    if (t != tile) set_tiles(p, t);
+    if (p.elt == ELT_F16) launch_kernel<ELT_F16>(kernel, p, mode, km, nb, stream);
+    else launch_kernel<ELT_BF16>(kernel, p, mode, km, nb, stream);
+    return hipGetLastError();
+  }
+  NtBatch b;
+  b.n = cnt;
+  b.first[0] = 0;
+  for (int i = 0; i < cnt; ++i) {
+    b.a[i] = a[order[i]];
+    if (t != tile) set_tiles(b.a[i], t);
+    b.first[i + 1] = b.first[i] + b.a[i].tiles_per_mat * b.a[i].L;
+  }
+  launch_kernel<ELT_F16>(kernel, b, mode, km, nb, stream);
   return hipGetLastError();
+}
+
+hipError_t launch_nt(const NtArgs& a, int tile, hipStream_t stream) {
+  return launch_nt_batch(&a, 1, tile, stream);
 }
 
 }  // namespace dmuon

@@ -9,8 +9,8 @@ Constructor, ``step()`` and ``zero_grad()`` keep the reference's signature and e
     U = NS(ns_in)                                                   muon.py:1704
     W *= 1 - lr*wd  (wd > 0);  W += -lr*0.2*sqrt(max(m, n)) * U     muon.py:1728-1740
 
-runs on the GPU as one C-ABI call per bucket of same-shape parameters
-(``dmuon_muon_step_group``): a fused momentum/Nesterov/staging kernel, a norm finalise, and
+runs on the GPU as one C-ABI call pair per set of same-shape buckets
+(``dmuon_muon_stage_groups``, ``dmuon_muon_apply_groups``): a fused momentum/Nesterov/staging kernel, a norm finalise, and
 the fp16 MFMA products of the chosen NS form (``ns_backend``: "gram", the default, or
 "direct"), the last product applying the weight update in its epilogue. The momentum buffer is fp32 and lives in
 ``optimizer.state[id(dp)]["momentum_buffer"]`` shaped ``(rows, cols)`` like the reference's.
@@ -140,6 +140,7 @@ class Muon(torch.optim.Optimizer):
         self._record_step_profile = bool(record_step_profile)
         self._workspace_limit = int(workspace_limit_bytes)
         self._workspaces: list = [None, None]
+        self._call_plans: dict = {}
         self._ptr_tables: dict = {}
         self._captured_tables: dict = {}      # tables a graph capture has read (kept alive)
         self._overlap_staging = bool(overlap_staging)
@@ -358,57 +359,112 @@ class Muon(torch.optim.Optimizer):
                                                            "ns_scale", dp.param_name)
                     if not dp._owned_data.is_contiguous():
                         raise RuntimeError(f"{dp.param_name}: Muon needs a contiguous weight")
-                tile, _, _, nbytes = _C.plan(rows, cols, len(part), 0, num_cus, backend)
-                chunks.append((rows, cols, n_t, dev, first, pdt is not None, part, tile, nbytes))
+                chunks.append((rows, cols, n_t, dev, first, pdt is not None, part))
                 count += len(part)
                 numel += len(part) * rows * cols
         if not chunks:
             return 0, 0
         dev = chunks[0][3]
         main = torch.cuda.current_stream(dev)
-        self._run_pipeline(chunks, dev, main, (lr, mu, wd, coeffs, T, backend, rst, n_rst))
+        self._run_pipeline(self._call_sets(chunks, backend), dev, main,
+                           (lr, mu, wd, coeffs, T, backend, rst, n_rst))
         for c in chunks:
             for dp, _, _ in c[6]:
                 dp._reduced_grad = None
         return count, numel
 
-    def _stage_chunk(self, chunk, ws, stream, args) -> None:
-        """Momentum, norm and NS operands of one chunk into ``ws``, on ``stream`` (the pointer
-        arrays and any contiguous gradient copies are made on that stream too)."""
-        rows, cols, n_t, dev, first, _, part, tile, _ = chunk
-        _, mu, _, _, _, backend, _, _ = args
-        L = len(part)
-        with torch.cuda.stream(stream):
-            gs = [g if g.is_contiguous() else g.contiguous() for _, g, _ in part]
-            ests = ([self.state[id(dp)]["ns_scale"].data_ptr() for dp, _, _ in part]
-                    if self._single_pass else [])
-            ptrs = self._ptr_table(("stage",) + tuple(id(dp) for dp, _, _ in part),
-                                   [t.data_ptr() for t in gs]
-                                   + [self.state[id(dp)]["momentum_buffer"].data_ptr()
-                                      for dp, _, _ in part] + ests, dev)
-            _C.call("dmuon_muon_stage_group", ptrs.data_ptr(), _float_dtype_code(gs[0]),
-                    ptrs.data_ptr() + 8 * L,
-                    ptrs.data_ptr() + 16 * L if ests else None, rows, cols, L, n_t, mu,
-                    int(self._nesterov), int(first), backend, self._ns_eps, ws.data_ptr(),
-                    ws.numel(), tile, stream.cuda_stream)
+    def _call_sets(self, chunks: list, backend: int) -> list:
+        """The chunks as calls: ``[(chunks, tile, workspace bytes), ...]``. Chunks of different
+        shapes join one call -- one launch per product over all of them -- when the library's
+        estimate of the joined products is below that of separate ones and their workspaces fit
+        ``workspace_limit_bytes`` together. With ``overlap_staging`` every chunk stays a call of
+        its own (the pipeline needs a next chunk to stage)."""
+        sets: list = []            # [chunks, sizes, tile, bytes, estimate]
+        for c in chunks:
+            num_cus = torch.cuda.get_device_properties(c[3]).multi_processor_count
+            size = (c[0], c[1], len(c[6]))
+            tile, nbytes, us = self._plan_call((size,), num_cus, backend)
+            best = None
+            for s in sets:
+                if self._overlap_staging or len(s[0]) >= _C.MAX_GROUPS or s[0][0][3] != c[3] or \
+                        s[3] + nbytes > self._workspace_limit:
+                    continue
+                joined = self._plan_call(s[1] + (size,), num_cus, backend)
+                saved = s[4] + us - joined[2]
+                if saved > 0 and joined[1] <= self._workspace_limit and \
+                        (best is None or saved > best[0]):
+                    best = (saved, s, joined)
+            if best is None:
+                sets.append([[c], (size,), tile, nbytes, us])
+            else:
+                _, s, joined = best
+                s[0].append(c)
+                s[1] += (size,)
+                s[2:] = joined
+        return [(s[0], s[2], s[3]) for s in sets]
 
-    def _apply_chunk(self, chunk, ws, stream, args) -> None:
-        """NS products and the fused weight update of one staged chunk, on ``stream``."""
-        rows, cols, n_t, dev, _, has_pub, part, tile, _ = chunk
-        lr, _, wd, coeffs, T, backend, rst, n_rst = args
-        L = len(part)
+    def _plan_call(self, sizes: tuple, num_cus: int, backend: int) -> tuple:
+        """``_C.plan_groups`` of ``sizes``, kept: it depends on nothing else."""
+        key = (sizes, num_cus, backend)
+        got = self._call_plans.get(key)
+        if got is None:
+            if len(self._call_plans) >= 4096:
+                self._call_plans.clear()
+            got = self._call_plans[key] = _C.plan_groups(sizes, 0, num_cus, backend)
+        return got
+
+    @staticmethod
+    def _descriptors(chunks: list):
+        descs = (_C.MuonGroup * len(chunks))()
+        for d, (rows, cols, n_t, _, first, _, part) in zip(descs, chunks):
+            d.rows, d.cols, d.batch, d.n_transposed = rows, cols, len(part), n_t
+            d.first_step = int(first)
+        return descs
+
+    def _stage_set(self, chunks, tile, ws, stream, args) -> None:
+        """Momentum, norm and NS operands of one call's chunks into ``ws``, on ``stream`` (the
+        pointer arrays and any contiguous gradient copies are made on that stream too)."""
+        _, mu, _, _, _, backend, _, _ = args
         with torch.cuda.stream(stream):
-            W = [dp._owned_data for dp, _, _ in part]
-            pubs = [dp.publish_target() for dp, _, _ in part] if has_pub else []
-            wptrs = self._ptr_table(("apply",) + tuple(id(dp) for dp, _, _ in part),
-                                    [t.data_ptr() for t in W] + [t.data_ptr() for t in pubs],
-                                    dev)
-            # the forward copies (master != parameter) are written by the same epilogue
-            _C.call("dmuon_muon_apply_group", wptrs.data_ptr(), _float_dtype_code(W[0]),
-                    wptrs.data_ptr() + 8 * L if pubs else None,
-                    _float_dtype_code(pubs[0]) if pubs else 0, rows, cols, L, n_t, lr, wd,
-                    coeffs, T, backend, rst, n_rst, ws.data_ptr(), ws.numel(), tile,
-                    stream.cuda_stream)
+            descs = self._descriptors(chunks)
+            keep = []
+            for d, (_, _, _, dev, _, _, part) in zip(descs, chunks):
+                L = len(part)
+                gs = [g if g.is_contiguous() else g.contiguous() for _, g, _ in part]
+                ests = ([self.state[id(dp)]["ns_scale"].data_ptr() for dp, _, _ in part]
+                        if self._single_pass else [])
+                ptrs = self._ptr_table(("stage",) + tuple(id(dp) for dp, _, _ in part),
+                                       [t.data_ptr() for t in gs]
+                                       + [self.state[id(dp)]["momentum_buffer"].data_ptr()
+                                          for dp, _, _ in part] + ests, dev)
+                base = ptrs.data_ptr()
+                d.g_ptrs, d.buf_ptrs, d.g_dtype = base, base + 8 * L, _float_dtype_code(gs[0])
+                d.est_ptrs = base + 16 * L if ests else None
+                keep.append((gs, ptrs))
+            _C.call("dmuon_muon_stage_groups", descs, len(chunks), mu, int(self._nesterov),
+                    backend, self._ns_eps, ws.data_ptr(), ws.numel(), tile, stream.cuda_stream)
+
+    def _apply_set(self, chunks, tile, ws, stream, args) -> None:
+        """NS products and the fused weight update of one staged call, on ``stream``."""
+        lr, _, wd, coeffs, T, backend, rst, n_rst = args
+        with torch.cuda.stream(stream):
+            descs = self._descriptors(chunks)
+            keep = []
+            for d, (_, _, _, dev, _, has_pub, part) in zip(descs, chunks):
+                L = len(part)
+                W = [dp._owned_data for dp, _, _ in part]
+                pubs = [dp.publish_target() for dp, _, _ in part] if has_pub else []
+                wptrs = self._ptr_table(("apply",) + tuple(id(dp) for dp, _, _ in part),
+                                        [t.data_ptr() for t in W] + [t.data_ptr() for t in pubs],
+                                        dev)
+                # the forward copies (master != parameter) are written by the same epilogue
+                base = wptrs.data_ptr()
+                d.w_ptrs, d.w_dtype = base, _float_dtype_code(W[0])
+                d.pub_ptrs = base + 8 * L if pubs else None
+                d.pub_dtype = _float_dtype_code(pubs[0]) if pubs else 0
+                keep.append((W, pubs, wptrs))
+            _C.call("dmuon_muon_apply_groups", descs, len(chunks), lr, wd, coeffs, T, backend,
+                    rst, n_rst, ws.data_ptr(), ws.numel(), tile, stream.cuda_stream)
 
     def _ptr_table(self, slot: tuple, ptrs: list, device: torch.device) -> Tensor:
         """The device array of ``ptrs`` (int64 addresses) that a group entry point reads, kept
@@ -439,33 +495,33 @@ class Muon(torch.optim.Optimizer):
         self._ptr_tables[slot] = (key, table)
         return table
 
-    def _run_pipeline(self, chunks, dev, main, args) -> None:
-        """The chunks one after another on ``main``; with ``overlap_staging`` chunk k+1 is
-        staged on a side stream into the other workspace while chunk k's NS runs."""
-        overlap = self._overlap_staging and len(chunks) > 1
+    def _run_pipeline(self, sets, dev, main, args) -> None:
+        """The calls one after another on ``main``; with ``overlap_staging`` call k+1 is staged
+        on a side stream into the other workspace while call k's NS runs."""
+        overlap = self._overlap_staging and len(sets) > 1
         side = self._side_stream(dev) if overlap else main
         # both workspaces exist before the hand-over event, so no block the side stream writes
         # can still be in use by later work on `main`
         nslots = 2 if overlap else 1
-        wss = [self._get_workspace(dev, max(c[8] for k, c in enumerate(chunks)
+        wss = [self._get_workspace(dev, max(c[2] for k, c in enumerate(sets)
                                             if k % nslots == sl), sl)
-               for sl in range(min(nslots, len(chunks)))]
+               for sl in range(min(nslots, len(sets)))]
         if overlap:
             start = torch.cuda.Event()
             start.record(main)           # gradients, buffers and weights are ready on `main`
             side.wait_event(start)
         free = [None, None]
-        for k, chunk in enumerate(chunks):
+        for k, (chunks, tile, _) in enumerate(sets):
             slot = k % nslots
             ws = wss[slot]
             if free[slot] is not None:
                 side.wait_event(free[slot])
-            self._stage_chunk(chunk, ws, side, args)
+            self._stage_set(chunks, tile, ws, side, args)
             if overlap:
                 staged = torch.cuda.Event()
                 staged.record(side)
                 main.wait_event(staged)
-            self._apply_chunk(chunk, ws, main, args)
+            self._apply_set(chunks, tile, ws, main, args)
             if overlap:
                 done = torch.cuda.Event()
                 done.record(main)

@@ -72,7 +72,7 @@ extern "C" {
 const char* dmuon_last_error(void);
 
 /* ABI version (major*100 + minor): DMUON_ABI_VERSION of the header the library was built with. */
-#define DMUON_ABI_VERSION 108
+#define DMUON_ABI_VERSION 109
 int dmuon_abi_version(void);
 
 /*
@@ -320,6 +320,36 @@ int dmuon_muon_step_group_noalloc(void* const* g_ptrs, int g_dtype, float* const
  * allocation-free step. Allocates no device memory besides the array itself, which the loader
  * reserves on this GPU with its code object at the first resolution. */
 int dmuon_noalloc_init(void** scratch_out, int64_t* scratch_bytes);
+
+/* Several groups of different oriented shapes in one sequence of launches: every product of the
+ * iteration is one launch over all of them (a model with a few small shapes fills the GPU and
+ * pays one launch chain instead of one per shape). The groups share lr, mu, wd, the coefficients
+ * and restarts; each matrix gets the bits its own dmuon_muon_stage_group / _apply_group calls
+ * give it at the same tile. At most DMUON_MAX_GROUPS groups a call; est_ptrs is given for every
+ * group or for none. The workspace is the groups' workspaces one after another.
+ *   dmuon_muon_plan_groups: the tile to pass on (0 lets it choose; one group: the tile
+ *     dmuon_ns_plan gives it), the workspace, and optionally an estimate of the products' time,
+ *     by which a caller decides whether to join groups (reads only the sizes of the groups). */
+#define DMUON_MAX_GROUPS 8
+typedef struct dmuon_muon_group {
+  void* const* g_ptrs;            /* DEVICE arrays of `batch` pointers, as above; stage: */
+  float* const* buf_ptrs;
+  float* const* est_ptrs;
+  void* const* w_ptrs;            /* apply: */
+  void* const* pub_ptrs;
+  int g_dtype, w_dtype, pub_dtype;
+  int rows, cols, batch, n_transposed, first_step;
+} dmuon_muon_group;
+int dmuon_muon_plan_groups(const dmuon_muon_group* groups, int n, int tile, int num_cus,
+                           int backend, int* tile_out, int64_t* workspace_bytes,
+                           double* cost_us);
+int dmuon_muon_stage_groups(const dmuon_muon_group* groups, int n, double mu, int nesterov,
+                            int backend, float eps, void* workspace, int64_t workspace_bytes,
+                            int tile, void* stream);
+int dmuon_muon_apply_groups(const dmuon_muon_group* groups, int n, double lr, double wd,
+                            const float* coeffs, int T, int backend, const int* restarts,
+                            int n_restarts, void* workspace, int64_t workspace_bytes, int tile,
+                            void* stream);
 
 /* direct_newton_schulz / gram_newton_schulz (by `backend`, as above) for `batch` matrices of one
  * oriented shape (the last n_transposed are cols x rows, as above): out[l] <- NS(g[l]). */
