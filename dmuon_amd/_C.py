@@ -103,6 +103,11 @@ _SIGNATURES = {
                                           c_int, c_vp]),
     "dmuon_adamw_multi": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_i64, c_int, c_int,
                                   c_int, c_int, c_f, c_f, c_f, c_f, c_f, c_f, c_f, c_f, c_vp]),
+    "dmuon_adamw_tensors": (c_int, [ctypes.POINTER(c_i64), c_int, c_int, c_int, c_int, c_int, c_f,
+                                    c_f, c_f, c_f, c_f, c_f, c_f, c_f, c_vp]),
+    "dmuon_newton_schulz_matrices": (c_int, [ctypes.POINTER(c_vp), c_int, ctypes.POINTER(c_vp),
+                                             c_int, c_int, c_int, c_int, c_fp, c_int, c_int, c_ip,
+                                             c_int, c_f, c_vp, c_i64, c_int, c_vp]),
     "dmuon_segmented_l2_norm_sq": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_vp,
                                            c_vp]),
     "dmuon_segmented_scale": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_vp,

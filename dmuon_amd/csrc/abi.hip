@@ -1212,6 +1212,33 @@ int dmuon_muon_update(void* const* w_ptrs, int w_dtype, const void* const* u_ptr
   return check_launch(launch_update(u, static_cast<hipStream_t>(stream)), who);
 }
 
+}  // extern "C"
+
+namespace {
+
+int adamw_checks(const char* who, int n, int64_t total, int p_dtype, int g_dtype, bool pub,
+                 int pub_dtype, float bc2_sqrt) {
+  if (n < 0 || total < 0) return fail("%s: negative tensor count or size", who);
+  if ((p_dtype != DMUON_DTYPE_F32 && p_dtype != DMUON_DTYPE_BF16) ||
+      (g_dtype != DMUON_DTYPE_F32 && g_dtype != DMUON_DTYPE_BF16))
+    return fail("%s: unsupported dtype (p %d, g %d)", who, p_dtype, g_dtype);
+  if (pub && pub_dtype != DMUON_DTYPE_F32 && pub_dtype != DMUON_DTYPE_BF16)
+    return fail("%s: unsupported publish dtype %d", who, pub_dtype);
+  if (!(bc2_sqrt > 0.f)) return fail("%s: bias correction must be positive", who);
+  return 0;
+}
+
+// read p, g, m, v; write p, m, v and the forward copy
+double adamw_bytes(int64_t total, int p_dtype, int g_dtype, bool pub, int pub_dtype) {
+  const int pb = p_dtype == DMUON_DTYPE_F32 ? 4 : 2, gb = g_dtype == DMUON_DTYPE_F32 ? 4 : 2;
+  const double qb = pub ? (pub_dtype == DMUON_DTYPE_F32 ? 4 : 2) : 0;
+  return (double)total * (6.0 * pb + gb + qb);
+}
+
+}  // namespace
+
+extern "C" {
+
 int dmuon_adamw_multi(const int64_t* p_ptrs, const int64_t* g_ptrs, const int64_t* m_ptrs,
                       const int64_t* v_ptrs, const int64_t* pub_ptrs, const int64_t* offsets,
                       int n, int64_t total, int p_dtype, int g_dtype, int pub_dtype, int apply_wd,
@@ -1222,12 +1249,8 @@ int dmuon_adamw_multi(const int64_t* p_ptrs, const int64_t* g_ptrs, const int64_
   if (n < 0 || total < 0) return fail("%s: negative tensor count or size", who);
   if (!p_ptrs || !g_ptrs || !m_ptrs || !v_ptrs || !offsets)
     return fail("%s: pointer arrays must be non-NULL", who);
-  if ((p_dtype != DMUON_DTYPE_F32 && p_dtype != DMUON_DTYPE_BF16) ||
-      (g_dtype != DMUON_DTYPE_F32 && g_dtype != DMUON_DTYPE_BF16))
-    return fail("%s: unsupported dtype (p %d, g %d)", who, p_dtype, g_dtype);
-  if (pub_ptrs && pub_dtype != DMUON_DTYPE_F32 && pub_dtype != DMUON_DTYPE_BF16)
-    return fail("%s: unsupported publish dtype %d", who, pub_dtype);
-  if (!(bc2_sqrt > 0.f)) return fail("%s: bias correction must be positive", who);
+  if (adamw_checks(who, n, total, p_dtype, g_dtype, pub_ptrs != nullptr, pub_dtype, bc2_sqrt))
+    return 1;
   AdamWArgs a{};
   a.p_ptrs = p_ptrs; a.g_ptrs = g_ptrs; a.m_ptrs = m_ptrs; a.v_ptrs = v_ptrs;
   a.pub_ptrs = pub_ptrs; a.pub_dtype = pub_dtype;
@@ -1235,11 +1258,47 @@ int dmuon_adamw_multi(const int64_t* p_ptrs, const int64_t* g_ptrs, const int64_
   a.p_dtype = p_dtype; a.g_dtype = g_dtype; a.apply_wd = apply_wd != 0;
   a.wd_scale = wd_scale; a.beta1 = beta1; a.alpha1 = alpha1; a.beta2 = beta2; a.alpha2 = alpha2;
   a.bc2_sqrt = bc2_sqrt; a.eps = eps; a.neg_step = neg_step;
-  const int pb = p_dtype == DMUON_DTYPE_F32 ? 4 : 2, gb = g_dtype == DMUON_DTYPE_F32 ? 4 : 2;
-  const double qb = pub_ptrs ? (pub_dtype == DMUON_DTYPE_F32 ? 4 : 2) : 0;
-  const double bytes = (double)total * (6.0 * pb + gb + qb);   // read p,g,m,v; write p,m,v(,q)
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return timed(PC_ADAMW, 0.0, bytes, st, who, [&] { return launch_adamw(a, st); });
+  return timed(PC_ADAMW, 0.0, adamw_bytes(total, p_dtype, g_dtype, pub_ptrs != nullptr, pub_dtype),
+               st, who, [&] { return launch_adamw(a, st); });
+}
+
+int dmuon_adamw_tensors(const int64_t* table, int n, int p_dtype, int g_dtype, int pub_dtype,
+                        int apply_wd, float wd_scale, float beta1, float alpha1, float beta2,
+                        float alpha2, float bc2_sqrt, float eps, float neg_step, void* stream) {
+  const char* who = "dmuon_adamw_tensors";
+  if (n == 0) return 0;
+  if (n < 0 || !table) return fail("%s: negative tensor count or NULL table", who);
+  bool pub = false;
+  for (int t = 0; t < n; ++t) {
+    const int64_t* r = table + 6 * (int64_t)t;
+    if (r[5] < 0) return fail("%s: tensor %d has a negative size", who, t);
+    if (r[5] > 0 && (!r[0] || !r[1] || !r[2] || !r[3]))
+      return fail("%s: tensor %d has a NULL address", who, t);
+    pub = pub || r[4] != 0;
+  }
+  if (adamw_checks(who, n, 0, p_dtype, g_dtype, pub, pub_dtype, bc2_sqrt)) return 1;
+  AdamWArgs a{};
+  a.pub_dtype = pub_dtype;
+  a.p_dtype = p_dtype; a.g_dtype = g_dtype; a.apply_wd = apply_wd != 0;
+  a.wd_scale = wd_scale; a.beta1 = beta1; a.alpha1 = alpha1; a.beta2 = beta2; a.alpha2 = alpha2;
+  a.bc2_sqrt = bc2_sqrt; a.eps = eps; a.neg_step = neg_step;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  AdamWTable tab;
+  for (int t0 = 0; t0 < n; t0 += kAdamWTable) {
+    a.n = n - t0 < kAdamWTable ? n - t0 : kAdamWTable;
+    tab.off[0] = 0;
+    for (int t = 0; t < a.n; ++t) {
+      const int64_t* r = table + 6 * (int64_t)(t0 + t);
+      tab.p[t] = r[0]; tab.g[t] = r[1]; tab.m[t] = r[2]; tab.v[t] = r[3]; tab.q[t] = r[4];
+      tab.off[t + 1] = tab.off[t] + r[5];
+    }
+    a.total = tab.off[a.n];
+    if (timed(PC_ADAMW, 0.0, adamw_bytes(a.total, p_dtype, g_dtype, pub, pub_dtype), st, who,
+              [&] { return launch_adamw_table(a, tab, st); }))
+      return 1;
+  }
+  return 0;
 }
 
 static int clip_common(const int64_t* ptrs, const int64_t* numels, const int32_t* dtypes,
@@ -1383,6 +1442,38 @@ int dmuon_newton_schulz_group(void* const* g_ptrs, int g_dtype, void* const* out
   Call c{&g, 1, 0, static_cast<hipStream_t>(stream), who};
   return run_groups(c, 0.f, 0, 1.f, coeffs, T, backend, restarts, n_restarts, eps, workspace,
                     workspace_bytes, tile);
+}
+
+int dmuon_newton_schulz_matrices(const void* const* g, int g_dtype, void* const* out,
+                                 int out_dtype, int rows, int cols, int batch,
+                                 const float* coeffs, int T, int backend, const int* restarts,
+                                 int n_restarts, float eps, void* workspace,
+                                 int64_t workspace_bytes, int tile, void* stream) {
+  const char* who = "dmuon_newton_schulz_matrices";
+  if (batch == 0) return 0;
+  if (batch < 0 || !g || !out) return fail("%s: NULL address table or negative batch", who);
+  const int64_t words = align256(16 * (int64_t)batch);
+  if (!workspace || !aligned16(workspace) || workspace_bytes < words)
+    return fail("%s: workspace NULL, misaligned or too small", who);
+  for (int l = 0; l < batch; ++l)
+    if (!g[l] || !out[l]) return fail("%s: NULL matrix address", who);
+  int64_t* dev = static_cast<int64_t*>(workspace);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  TableWords t;
+  for (int w0 = 0; w0 < 2 * batch; w0 += kTableWords) {
+    const int nw = 2 * batch - w0 < kTableWords ? 2 * batch - w0 : kTableWords;
+    for (int w = 0; w < nw; ++w) {
+      const int l = w0 + w;
+      t.w[w] = (int64_t)(l < batch ? reinterpret_cast<intptr_t>(g[l])
+                                   : reinterpret_cast<intptr_t>(out[l - batch]));
+    }
+    if (check_launch(launch_write_table(t, nw, dev + w0, st), who)) return 1;
+  }
+  return dmuon_newton_schulz_group(reinterpret_cast<void* const*>(dev), g_dtype,
+                                   reinterpret_cast<void* const*>(dev + batch), out_dtype, rows,
+                                   cols, batch, 0, coeffs, T, backend, restarts, n_restarts, eps,
+                                   static_cast<char*>(workspace) + words, workspace_bytes - words,
+                                   tile, stream);
 }
 
 int dmuon_muon_stage_group(void* const* g_ptrs, int g_dtype, float* const* buf_ptrs,

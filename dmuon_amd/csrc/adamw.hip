@@ -141,30 +141,66 @@ __device__ __forceinline__ void adamw_elt2(float* p, const float* g, float* m, f
   rnd2<D>(p[0], p[1]);
 }
 
-template <int PD, int GD>
-__global__ __launch_bounds__(256) void adamw_kernel(const AdamWArgs a) {
+// Where a block finds the bucket's tensors: device arrays (AdamWArgs), or, for a short table
+// that a host caller holds, the launch's own arguments -- no copy to the device, which for a few
+// norm vectors costs more than the update (pinned staging and a copy launch). `first` is the
+// last tensor whose start is <= lo.
+struct DeviceTable {
+  __device__ static int first(const AdamWArgs& a, const DeviceTable&, long long lo) {
+    int t = 0, r = a.n - 1;
+    while (t < r) {
+      const int mid = (t + r + 1) >> 1;
+      if (a.offsets[mid] <= lo) t = mid; else r = mid - 1;
+    }
+    return t;
+  }
+  __device__ static int64_t off(const AdamWArgs& a, const DeviceTable&, int t) { return a.offsets[t]; }
+  __device__ static int64_t p(const AdamWArgs& a, const DeviceTable&, int t) { return a.p_ptrs[t]; }
+  __device__ static int64_t g(const AdamWArgs& a, const DeviceTable&, int t) { return a.g_ptrs[t]; }
+  __device__ static int64_t m(const AdamWArgs& a, const DeviceTable&, int t) { return a.m_ptrs[t]; }
+  __device__ static int64_t v(const AdamWArgs& a, const DeviceTable&, int t) { return a.v_ptrs[t]; }
+  __device__ static int64_t q(const AdamWArgs& a, const DeviceTable&, int t) {
+    return a.pub_ptrs ? a.pub_ptrs[t] : 0;
+  }
+};
+struct ArgTable {
+  AdamWTable d;
+  // the starts are compared by the lanes of a wave at once: one load each instead of a chain of
+  // log2(n) scalar loads
+  __device__ static int first(const AdamWArgs& a, const ArgTable& tab, long long lo) {
+    static_assert(kAdamWTable <= 128, "two starts per lane");
+    const int lane = threadIdx.x & 63;
+    const bool b0 = lane < a.n && tab.d.off[lane] <= lo;
+    const bool b1 = lane + 64 < a.n && tab.d.off[lane + 64] <= lo;
+    return __popcll(__ballot(b0)) + __popcll(__ballot(b1)) - 1;
+  }
+  __device__ static int64_t off(const AdamWArgs&, const ArgTable& tab, int t) { return tab.d.off[t]; }
+  __device__ static int64_t p(const AdamWArgs&, const ArgTable& tab, int t) { return tab.d.p[t]; }
+  __device__ static int64_t g(const AdamWArgs&, const ArgTable& tab, int t) { return tab.d.g[t]; }
+  __device__ static int64_t m(const AdamWArgs&, const ArgTable& tab, int t) { return tab.d.m[t]; }
+  __device__ static int64_t v(const AdamWArgs&, const ArgTable& tab, int t) { return tab.d.v[t]; }
+  __device__ static int64_t q(const AdamWArgs&, const ArgTable& tab, int t) { return tab.d.q[t]; }
+};
+
+template <int PD, int GD, class TAB>
+__global__ __launch_bounds__(256) void adamw_kernel(const AdamWArgs a, const TAB tab) {
   const long long lo = (long long)blockIdx.x * a.per_block;
   if (lo >= a.total) return;
   const long long hi = min(lo + a.per_block, a.total);
-  // last tensor whose start is <= lo
-  int t = 0, r = a.n - 1;
-  while (t < r) {
-    const int mid = (t + r + 1) >> 1;
-    if (a.offsets[mid] <= lo) t = mid; else r = mid - 1;
-  }
+  int t = __builtin_amdgcn_readfirstlane(TAB::first(a, tab, lo));
   const int tid = threadIdx.x;
-  for (; t < a.n && a.offsets[t] < hi; ++t) {
-    const long long t0 = a.offsets[t];
-    const long long s = max(lo, t0) - t0, e = min(hi, a.offsets[t + 1]) - t0;
+  for (; t < a.n && TAB::off(a, tab, t) < hi; ++t) {
+    const long long t0 = TAB::off(a, tab, t);
+    const long long s = max(lo, t0) - t0, e = min(hi, (long long)TAB::off(a, tab, t + 1)) - t0;
     if (s >= e) continue;
-    void* P = reinterpret_cast<void*>(a.p_ptrs[t]);
-    const void* G = reinterpret_cast<const void*>(a.g_ptrs[t]);
-    void* M = reinterpret_cast<void*>(a.m_ptrs[t]);
-    void* V = reinterpret_cast<void*>(a.v_ptrs[t]);
-    const int64_t pub_addr = a.pub_ptrs ? a.pub_ptrs[t] : 0;
-    void* Q = reinterpret_cast<void*>(pub_addr);           // forward copy of p, or null
-    const bool aligned =
-        ((a.p_ptrs[t] | a.g_ptrs[t] | a.m_ptrs[t] | a.v_ptrs[t] | pub_addr) & 15) == 0;
+    const int64_t pa = TAB::p(a, tab, t), ga = TAB::g(a, tab, t), ma = TAB::m(a, tab, t),
+                  va = TAB::v(a, tab, t), qa = TAB::q(a, tab, t);
+    void* P = reinterpret_cast<void*>(pa);
+    const void* G = reinterpret_cast<const void*>(ga);
+    void* M = reinterpret_cast<void*>(ma);
+    void* V = reinterpret_cast<void*>(va);
+    void* Q = reinterpret_cast<void*>(qa);                 // forward copy of p, or null
+    const bool aligned = ((pa | ga | ma | va | qa) & 15) == 0;
     long long vs = e, ve = e;
     if (aligned) {
       vs = min((s + 7) & ~7LL, e);
@@ -205,24 +241,40 @@ __global__ __launch_bounds__(256) void adamw_kernel(const AdamWArgs a) {
 
 }  // namespace
 
-hipError_t launch_adamw(AdamWArgs a, hipStream_t stream) {
+namespace {
+
+template <class TAB>
+hipError_t launch_tables(AdamWArgs a, const TAB& tab, hipStream_t stream) {
   if (a.total <= 0 || a.n <= 0) return hipSuccess;
   // 4096 elements per block (a multiple of the 8-element vector), more when the grid would
-  // exceed 2^31 blocks
-  long long per = 4096;
+  // exceed 2^31 blocks; 2048 (one vector per thread) while that leaves at most two blocks per
+  // CU of a 256-CU device: such an update waits on latency, not bandwidth (65 norm vectors of
+  // 4096 bf16: 7.2 -> 4.7 us with the table as arguments)
+  long long per = a.total <= 512 * 2048 ? 2048 : 4096;
   if ((a.total + per - 1) / per > 0x7fffffffLL) per = ((a.total + 0x7ffffffeLL) / 0x7fffffffLL + 7) & ~7LL;
   a.per_block = per;
   const long long blocks = (a.total + per - 1) / per;
   const dim3 grid((unsigned)blocks), block(256);
   if (a.p_dtype == DT_F32 && a.g_dtype == DT_F32)
-    hipLaunchKernelGGL((adamw_kernel<DT_F32, DT_F32>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((adamw_kernel<DT_F32, DT_F32, TAB>), grid, block, 0, stream, a, tab);
   else if (a.p_dtype == DT_F32)
-    hipLaunchKernelGGL((adamw_kernel<DT_F32, DT_BF16>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((adamw_kernel<DT_F32, DT_BF16, TAB>), grid, block, 0, stream, a, tab);
   else if (a.g_dtype == DT_F32)
-    hipLaunchKernelGGL((adamw_kernel<DT_BF16, DT_F32>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((adamw_kernel<DT_BF16, DT_F32, TAB>), grid, block, 0, stream, a, tab);
   else
-    hipLaunchKernelGGL((adamw_kernel<DT_BF16, DT_BF16>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((adamw_kernel<DT_BF16, DT_BF16, TAB>), grid, block, 0, stream, a, tab);
   return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_adamw(const AdamWArgs& a, hipStream_t stream) {
+  return launch_tables(a, DeviceTable{}, stream);
+}
+
+hipError_t launch_adamw_table(const AdamWArgs& a, const AdamWTable& tab, hipStream_t stream) {
+  if (a.n > kAdamWTable) return hipErrorInvalidValue;
+  return launch_tables(a, ArgTable{tab}, stream);
 }
 
 }  // namespace dmuon

@@ -173,7 +173,24 @@ struct AdamWArgs {
   float wd_scale, beta1, alpha1, beta2, alpha2, bc2_sqrt, eps, neg_step;
   long long per_block;                    // set by launch_adamw
 };
-hipError_t launch_adamw(AdamWArgs a, hipStream_t stream);
+hipError_t launch_adamw(const AdamWArgs& a, hipStream_t stream);
+// The same with the tensors' addresses and starts as launch arguments (a's own arrays unused);
+// 80 tensors with AdamWArgs fit the 4 KiB a launch may carry.
+constexpr int kAdamWTable = 80;
+struct AdamWTable {
+  int64_t p[kAdamWTable], g[kAdamWTable], m[kAdamWTable], v[kAdamWTable], q[kAdamWTable];
+  int64_t off[kAdamWTable + 1];
+};
+static_assert(sizeof(AdamWTable) + sizeof(AdamWArgs) <= 4096, "launch arguments");
+hipError_t launch_adamw_table(const AdamWArgs& a, const AdamWTable& tab, hipStream_t stream);
+
+// dst[i] = values[i] for i < n (n <= kTableWords), the values being launch arguments: a short
+// table from the host in stream order, without a pinned buffer or a copy.
+constexpr int kTableWords = 480;
+struct TableWords {
+  int64_t w[kTableWords];
+};
+hipError_t launch_write_table(const TableWords& t, int n, int64_t* dst, hipStream_t stream);
 
 // Segmented clip job table (device arrays, the reference's fast-clip layout).
 struct ClipArgs {

@@ -1,4 +1,4 @@
-"""Fused decoupled AdamW on the HIP kernel ``dmuon_adamw_multi``.
+"""Fused decoupled AdamW on the HIP kernel ``dmuon_adamw_tensors``.
 
 ``fused_adamw_`` updates one bucket of the reference's ``_adamw_update_batch``
 (``dmuon/optim/muon.py:1857-1916``): tensors that share the post-increment step count, the
@@ -16,6 +16,7 @@ from torch import Tensor
 
 from .. import _C
 
+_device_index = Tensor.get_device          # -1 for a CPU tensor
 _CODES = {torch.float32: _C.DTYPE_F32, torch.bfloat16: _C.DTYPE_BF16}
 
 
@@ -59,27 +60,28 @@ def fused_adamw_(params: Sequence[Tensor], grads: Sequence[Tensor], exp_avgs: Se
     if dev.type != "cuda":
         raise RuntimeError("fused_adamw_: tensors must live on the GPU (HIP kernel only)")
     if torch.cuda.is_current_stream_capturing():
-        # the bias correction follows the host step count and the job table is copied from a
-        # temporary host buffer: a replay would repeat a stale step from freed memory
-        raise RuntimeError("fused_adamw_ cannot be captured into a graph (host step count and "
-                           "per-call job table); step AdamW-routed parameters eagerly")
+        # the bias correction follows the host step count: a replay would repeat a stale step
+        raise RuntimeError("fused_adamw_ cannot be captured into a graph (host step count); step "
+                           "AdamW-routed parameters eagerly")
     pdt, gdt = params[0].dtype, grads[0].dtype
     if pdt not in _CODES or gdt not in _CODES:
         raise ValueError(f"fused_adamw_: unsupported dtypes param {pdt}, grad {gdt}")
-    gs = []
-    for p, g, m, v in zip(params, grads, exp_avgs, exp_avg_sqs):
-        for t in (p, g, m, v):
-            if t.device != dev:
-                raise RuntimeError("fused_adamw_: all tensors must be on one device")
-        if p.dtype != pdt or m.dtype != pdt or v.dtype != pdt or g.dtype != gdt:
-            raise ValueError("fused_adamw_: a bucket shares one param/state dtype and one grad "
-                             "dtype")
-        if not (p.numel() == g.numel() == m.numel() == v.numel()):
-            raise ValueError("fused_adamw_: param, grad and state sizes differ")
-        for t in (p, m, v):
-            if not t.is_contiguous():
-                raise RuntimeError("fused_adamw_: params and AdamW state must be contiguous")
-        gs.append(g if g.is_contiguous() else g.contiguous())
+    # each property over all tensors at once: a Python loop over the tensors costs more than the
+    # update of a model's norm vectors
+    owned = [*params, *exp_avgs, *exp_avg_sqs]
+    index = dev.index if dev.index is not None else params[0].get_device()
+    if not all(map(index.__eq__, map(_device_index, [*owned, *grads]))):
+        raise RuntimeError("fused_adamw_: all tensors must be on one device")
+    if {t.dtype for t in owned} != {pdt} or {g.dtype for g in grads} != {gdt}:
+        raise ValueError("fused_adamw_: a bucket shares one param/state dtype and one grad dtype")
+    numels = list(map(Tensor.numel, params))
+    if not all(list(map(Tensor.numel, ts)) == numels for ts in (grads, exp_avgs, exp_avg_sqs)):
+        raise ValueError("fused_adamw_: param, grad and state sizes differ")
+    if not all(map(Tensor.is_contiguous, owned)):
+        raise RuntimeError("fused_adamw_: params and AdamW state must be contiguous")
+    gs = grads
+    if not all(map(Tensor.is_contiguous, grads)):
+        gs = [g.contiguous() for g in grads]
     qdt = None
     if publish is not None:
         if len(publish) != n:
@@ -94,19 +96,14 @@ def fused_adamw_(params: Sequence[Tensor], grads: Sequence[Tensor], exp_avgs: Se
                 raise ValueError("fused_adamw_: publish targets must match the params in size "
                                  "and share one dtype")
             qdt = q.dtype
-    offsets = [0]
-    for p in params:
-        offsets.append(offsets[-1] + p.numel())
     pubs = [0] * n if qdt is None else [0 if q is None else q.data_ptr() for q in publish]
-    table = ([p.data_ptr() for p in params] + [g.data_ptr() for g in gs]
-             + [m.data_ptr() for m in exp_avgs] + [v.data_ptr() for v in exp_avg_sqs] + pubs
-             + offsets)
-    dtab = torch.tensor(table, dtype=torch.int64, pin_memory=True).to(dev, non_blocking=True)
-    base = dtab.data_ptr()
+    table = (_C.c_i64 * (6 * n))()
+    for k, ts in enumerate((params, gs, exp_avgs, exp_avg_sqs)):
+        table[k::6] = list(map(Tensor.data_ptr, ts))
+    table[4::6] = pubs
+    table[5::6] = numels
     s = adamw_scalars(step, lr, betas, weight_decay, eps)
     stream = torch.cuda.current_stream(dev).cuda_stream
-    _C.call("dmuon_adamw_multi", base, base + 8 * n, base + 16 * n, base + 24 * n,
-            None if qdt is None else base + 32 * n, base + 40 * n, n, offsets[-1], _CODES[pdt],
-            _CODES[gdt], 0 if qdt is None else _CODES[qdt], s["apply_wd"], s["wd_scale"],
-            s["beta1"], s["alpha1"], s["beta2"], s["alpha2"], s["bc2_sqrt"], s["eps"],
-            s["neg_step"], stream)
+    _C.call("dmuon_adamw_tensors", table, n, _CODES[pdt], _CODES[gdt],
+            0 if qdt is None else _CODES[qdt], s["apply_wd"], s["wd_scale"], s["beta1"],
+            s["alpha1"], s["beta2"], s["alpha2"], s["bc2_sqrt"], s["eps"], s["neg_step"], stream)

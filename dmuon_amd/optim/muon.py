@@ -17,7 +17,7 @@ the fp16 MFMA products of the chosen NS form (``ns_backend``: "gram", the defaul
 
 Parameters that are not dedicated (and 1-D dedicated ones) get the reference's decoupled AdamW
 (``muon.py:1857-1916``): its (step, dtype) buckets, each updated by one fused HIP pass
-(``dmuon_adamw_multi``) with the rounding points of the reference's ``torch._foreach`` sequence.
+(``dmuon_adamw_tensors``) with the rounding points of the reference's ``torch._foreach`` sequence.
 """
 from __future__ import annotations
 

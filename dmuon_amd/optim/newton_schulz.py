@@ -125,9 +125,8 @@ def _restarts(restart_iterations) -> list:
     return out
 
 
-def _ptr_array(tensors: Sequence[Tensor], device: torch.device) -> Tensor:
-    host = torch.tensor([t.data_ptr() for t in tensors], dtype=torch.int64, pin_memory=True)
-    return host.to(device, non_blocking=True)
+def _address_array(tensors: Sequence[Tensor]):
+    return (_C.c_vp * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
 # NS scratch of the stand-alone functions, one buffer per (device, stream): calls on two
@@ -175,13 +174,11 @@ def newton_schulz_batched(
     num_cus = torch.cuda.get_device_properties(G0.device).multi_processor_count
     t, _mp, _np, nbytes = _C.plan(rows, cols, L, tile, num_cus, code)
     cur = torch.cuda.current_stream(G0.device)
-    ws = _WORKSPACE.get(G0.device, cur, nbytes)
-    gp = _ptr_array(ins, G0.device)
-    op = _ptr_array(outs, G0.device)
-    stream = cur.cuda_stream
-    _C.call("dmuon_newton_schulz_group", gp.data_ptr(), _float_dtype_code(ins[0]), op.data_ptr(),
-            _float_dtype_code(outs[0]), rows, cols, L, 0, coeff, T, code, rst, n_rst, float(eps),
-            ws.data_ptr(), ws.numel(), t, stream)
+    # the matrices' addresses sit in front of the planned workspace
+    ws = _WORKSPACE.get(G0.device, cur, nbytes + (16 * L + 255) // 256 * 256)
+    _C.call("dmuon_newton_schulz_matrices", _address_array(ins), _float_dtype_code(ins[0]),
+            _address_array(outs), _float_dtype_code(outs[0]), rows, cols, L, coeff, T, code, rst,
+            n_rst, float(eps), ws.data_ptr(), ws.numel(), t, cur.cuda_stream)
     if out is None and G0.dtype != work_dtype:
         return [o.to(G0.dtype) for o in outs]
     return outs

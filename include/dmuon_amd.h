@@ -359,6 +359,16 @@ int dmuon_newton_schulz_group(void* const* g_ptrs, int g_dtype, void* const* out
                               int T, int backend, const int* restarts, int n_restarts, float eps,
                               void* workspace, int64_t workspace_bytes, int tile, void* stream);
 
+/* The same for matrices whose addresses the host holds: g and out are HOST arrays of `batch`
+ * device addresses, all rows x cols. They reach the device as arguments of a small kernel in
+ * stream order (no pinned buffer, no copy). The workspace is the one dmuon_ns_plan sizes plus
+ * 16 * batch bytes rounded up to 256. */
+int dmuon_newton_schulz_matrices(const void* const* g, int g_dtype, void* const* out,
+                                 int out_dtype, int rows, int cols, int batch,
+                                 const float* coeffs, int T, int backend, const int* restarts,
+                                 int n_restarts, float eps, void* workspace,
+                                 int64_t workspace_bytes, int tile, void* stream);
+
 /*
  * Decoupled AdamW over n tensors in one pass (one bucket of the reference's
  * _adamw_update_batch: same step count, same param dtype, same grad dtype).
@@ -379,6 +389,13 @@ int dmuon_adamw_multi(const int64_t* p_ptrs, const int64_t* g_ptrs, const int64_
                       int n, int64_t total, int p_dtype, int g_dtype, int pub_dtype, int apply_wd,
                       float wd_scale, float beta1, float alpha1, float beta2, float alpha2,
                       float bc2_sqrt, float eps, float neg_step, void* stream);
+
+/* The same update with the tensors described by a HOST table of n rows of six int64: the
+ * addresses of param, grad, exp_avg, exp_avg_sq and forward copy (0: none), and the number of
+ * elements. The rows travel as launch arguments, 80 tensors a launch; nothing is copied. */
+int dmuon_adamw_tensors(const int64_t* table, int n, int p_dtype, int g_dtype, int pub_dtype,
+                        int apply_wd, float wd_scale, float beta1, float alpha1, float beta2,
+                        float alpha2, float bc2_sqrt, float eps, float neg_step, void* stream);
 
 /*
  * Segmented gradient clipping, the two device operations of the reference's fast-clip path,
