@@ -112,6 +112,9 @@ _SIGNATURES = {
                                            c_vp]),
     "dmuon_segmented_scale": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_vp,
                                       c_vp]),
+    "dmuon_clip_workspace_size": (c_int, [c_i64, c_i64, c_int, ctypes.POINTER(c_i64)]),
+    "dmuon_clip_norms": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_int,
+                                 c_int, c_d, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)

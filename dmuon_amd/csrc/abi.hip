@@ -1347,6 +1347,49 @@ int dmuon_segmented_scale(const int64_t* ptrs, const int64_t* numels, const int3
   return timed(PC_CLIP, 0.0, 0.0, st, who, [&] { return launch_clip_scale(a, st); });
 }
 
+static int64_t clip_workspace(int64_t n_jobs, int64_t chunk_size, int n_tensors) {
+  return 8 * (int64_t)n_tensors + 4 * n_jobs * clip_pieces(n_jobs, chunk_size);
+}
+
+int dmuon_clip_workspace_size(int64_t n_jobs, int64_t chunk_size, int n_tensors,
+                              int64_t* workspace_bytes) {
+  if (!workspace_bytes || n_jobs < 0 || n_jobs > 0x7fffffff || chunk_size <= 0 || n_tensors < 0)
+    return fail("dmuon_clip_workspace_size: bad sizes or NULL output");
+  *workspace_bytes = clip_workspace(n_jobs, chunk_size, n_tensors);
+  return 0;
+}
+
+int dmuon_clip_norms(const int64_t* ptrs, const int64_t* numels, const int32_t* dtypes,
+                     const int32_t* segments, const int32_t* job_tensor_ids,
+                     const int64_t* job_offsets, const int32_t* first_job, int64_t n_jobs,
+                     int64_t chunk_size, int n_tensors, int n_segments, double max_norm,
+                     float* norms, float* coefs, uint8_t* clipped, uint8_t* found_inf,
+                     void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* who = "dmuon_clip_norms";
+  ClipArgs a{};
+  if (clip_common(ptrs, numels, dtypes, segments, job_tensor_ids, job_offsets, n_jobs, chunk_size,
+                  who, &a))
+    return 1;
+  if (n_tensors <= 0 || n_segments < 0) return fail("%s: needs tensors", who);
+  if (!dtypes || !segments || !first_job || !norms || !coefs || !clipped || !found_inf)
+    return fail("%s: NULL argument", who);
+  const int64_t need = clip_workspace(n_jobs, chunk_size, n_tensors);
+  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 7) || workspace_bytes < need)
+    return fail("%s: workspace NULL, misaligned or smaller than %lld bytes", who, (long long)need);
+  ClipFinishArgs f{};
+  f.tensor_sq = static_cast<double*>(workspace);
+  f.partials = reinterpret_cast<const float*>(f.tensor_sq + n_tensors);
+  f.first_job = first_job; f.dtypes = dtypes; f.segments = segments;
+  f.n = n_tensors; f.n_segments = n_segments;
+  f.pieces = clip_pieces(n_jobs, chunk_size);
+  f.global = n_segments == 0;
+  f.has_max = max_norm == max_norm;            // NaN: no limit
+  f.max_norm = f.has_max ? (float)max_norm : 0.f;
+  f.norms = norms; f.coefs = coefs; f.clipped = clipped; f.found_inf = found_inf;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return timed(PC_CLIP, 0.0, 0.0, st, who, [&] { return launch_clip_norms(a, f, st); });
+}
+
 int dmuon_ns_plan(int rows, int cols, int batch, int tile_req, int num_cus, int backend,
                   int* tile, int* m_pad, int* n_pad, int64_t* workspace_bytes) {
   if (!tile || !m_pad || !n_pad || !workspace_bytes) return fail("dmuon_ns_plan: NULL output");

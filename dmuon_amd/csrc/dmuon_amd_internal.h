@@ -204,4 +204,19 @@ struct ClipArgs {
 hipError_t launch_clip_sumsq(const ClipArgs& a, hipStream_t stream);
 hipError_t launch_clip_scale(ClipArgs a, hipStream_t stream);
 
+// Norms, coefficients and flags of a job table's tensors in two launches. Tensor t's jobs are
+// first_job[t] .. first_job[t + 1] - 1, each split into `pieces` pieces (clip_pieces) whose sums
+// go to partials[job * pieces + piece].
+struct ClipFinishArgs {
+  const float* partials; double* tensor_sq;
+  const int32_t* first_job; const int32_t* dtypes; const int32_t* segments;
+  int n, n_segments, pieces;
+  int global, has_max;
+  float max_norm;
+  float* norms; float* coefs;             // [n_segments] (+ the norm of the norms), global: [1]
+  uint8_t* clipped; uint8_t* found_inf;
+};
+int clip_pieces(long long n_jobs, long long chunk);
+hipError_t launch_clip_norms(ClipArgs a, const ClipFinishArgs& f, hipStream_t stream);
+
 }  // namespace dmuon

@@ -21,6 +21,7 @@ stays rank-uniform.
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from collections import OrderedDict
 from dataclasses import dataclass
@@ -124,7 +125,7 @@ def _job_lists(numels, chunk: int):
 
 class _JobTable:
     """Device-resident job table of the kernel-eligible tensors: int64 [ptrs | numels |
-    job_offsets] and int32 [dtypes | segments | job_tensor_ids | zeros]."""
+    job_offsets] and int32 [dtypes | segments | job_tensor_ids | zeros | first job of each]."""
 
     def __init__(self, tensors, segments, device, chunk):
         n = len(tensors)
@@ -135,7 +136,8 @@ class _JobTable:
                               job_off])
         i32 = np.concatenate([np.array([_DTYPE_CODES[g.dtype] for g in tensors], dtype=np.int32),
                               np.asarray(segments, dtype=np.int32), job_t.astype(np.int32),
-                              np.zeros(n, dtype=np.int32)])
+                              np.zeros(n + 1, dtype=np.int32),
+                              np.cumsum((numels + chunk - 1) // chunk).astype(np.int32)])
         self._d64 = torch.from_numpy(i64).pin_memory().to(device, non_blocking=True)
         self._d32 = torch.from_numpy(i32).pin_memory().to(device, non_blocking=True)
         b64, b32 = self._d64.data_ptr(), self._d32.data_ptr()
@@ -143,6 +145,7 @@ class _JobTable:
         self.dtypes, self.segments = b32, b32 + 4 * n
         self.job_tensor_ids = b32 + 8 * n
         self.zero_segments = b32 + 8 * n + 4 * self.n_jobs
+        self.first_job = self.zero_segments + 4 * n     # its first entry, 0, ends the zeros
         self.device = device
         self._dtypes = [g.dtype for g in tensors]
         self._dtype_groups = None
@@ -167,6 +170,25 @@ class _JobTable:
         _C.call("dmuon_segmented_l2_norm_sq", self.ptrs, self.numels, self.dtypes,
                 self.segments if segments is None else segments, self.job_tensor_ids,
                 self.job_offsets, self.n_jobs, self.chunk, local_sq.data_ptr(), self._stream())
+
+    def norms(self, n_segments: int, max_norm: Optional[float]):
+        """``(norms, coefs, clipped, found_inf)`` of the table's segments, or of all its tensors
+        as one (``n_segments=0``, per-tensor norms rounded to their dtype): float32 and bool
+        device tensors. With segments ``norms`` has one more entry, the norm of the norms."""
+        k = max(n_segments, 1)
+        need = ctypes.c_int64()
+        _C.call("dmuon_clip_workspace_size", self.n_jobs, self.chunk, self.n, ctypes.byref(need))
+        need = need.value
+        ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+        out = torch.empty(4 * (2 * k + 1) + 2 * k, dtype=torch.uint8, device=self.device)
+        base, at = out.data_ptr(), 4 * (2 * k + 1)
+        _C.call("dmuon_clip_norms", self.ptrs, self.numels, self.dtypes, self.segments,
+                self.job_tensor_ids, self.job_offsets, self.first_job, self.n_jobs, self.chunk,
+                self.n, n_segments, float("nan") if max_norm is None else float(max_norm), base,
+                base + 4 * (k + 1), base + at, base + at + k, ws.data_ptr(), need,
+                self._stream())
+        floats, flags = out[:at].view(torch.float32), out[at:].view(torch.bool)
+        return floats[:k + 1], floats[k + 1:], flags[:k], flags[k:]
 
     def scale(self, coefs: torch.Tensor, segments=None) -> None:
         _C.call("dmuon_segmented_scale", self.ptrs, self.numels, self.dtypes,
@@ -211,9 +233,13 @@ def _split(buckets, device, ext):
     return kt, ks, rest
 
 
+def _needs_collective(reduce_flags) -> bool:
+    return dist.is_available() and dist.is_initialized() and any(reduce_flags)
+
+
 def _apply_segment_reductions(local_sq: torch.Tensor, reduce_flags, process_group=None):
     """The one rank-uniform collective over the reduce=True segments (fast_clip.py:313-339)."""
-    if not (dist.is_available() and dist.is_initialized() and any(reduce_flags)):
+    if not _needs_collective(reduce_flags):
         return local_sq
     mask = torch.tensor(reduce_flags, device=local_sq.device, dtype=torch.bool)
     red = torch.where(mask, local_sq, torch.zeros_like(local_sq))
@@ -248,6 +274,22 @@ def clip_grad_norm_buckets_(buckets: Sequence[GradClipBucket], max_norm: Optiona
     chunk = _resolve_chunk_size(chunk_size)
     reduce_flags = [1 if b.reduce else 0 for b in buckets]
     kt, ks, rest = _split(buckets, device, ext)
+
+    if kt and not rest and not _needs_collective(reduce_flags):
+        # every gradient on the kernels, nothing to reduce across ranks: norms, coefficients and
+        # flags in one pass, then the scaling
+        table = _job_table(kt, ks, device, chunk)
+        norms, coefs, clipped, found_inf = table.norms(len(buckets), max_norm)
+        if max_norm is not None:
+            table.scale(coefs)
+        limit = None if max_norm is None else float(max_norm)
+        stats = tuple(
+            GradClipBucketStats(name=b.name, total_norm=n, max_norm=limit, clip_coef=c, clipped=cl,
+                                param_count=sum(1 for g in b.grads if g is not None),
+                                found_inf=f, fastpath=True)
+            for b, n, c, cl, f in zip(buckets, norms.unbind(), coefs.unbind(), clipped.unbind(),
+                                      found_inf.unbind()))
+        return SegmentedGradClipResult(norms[len(buckets)], stats, fastpath=True)
 
     local_sq = torch.zeros(len(buckets), device=device, dtype=torch.float32)
     for g, s in rest:

@@ -83,18 +83,15 @@ class GlobalNormMuonClipStrategy:
         eligible = [t for t in tensors if ext is not None and _kernel_eligible(t, device)]
         table = (_job_table(eligible, list(range(len(eligible))), device, _resolve_chunk_size(None))
                  if eligible and context.norm_type == 2.0 else None)
+        if table is not None and len(eligible) == len(tensors) and not (
+                dist.is_available() and dist.is_initialized()):
+            return self._on_kernels(context, table)
         total = _total_norm(tensors, eligible, table, context.norm_type, device)
-        if context.error_if_nonfinite and bool(torch.logical_or(total.isnan(), total.isinf())):
-            raise RuntimeError(
-                f"The total norm of order {context.norm_type} for DMuon Muon gradients is "
-                "non-finite, so it cannot be clipped. To disable this error and scale the "
-                "gradients by the non-finite norm anyway, set `error_if_nonfinite=False`.")
+        _check_total(context, total)
         max_norm = context.max_norm
         clip_coef: Union[torch.Tensor, float] = 1.0
         clipped: Union[torch.Tensor, bool] = False
         if max_norm is not None:
-            if max_norm < 0:
-                raise ValueError(f"max_norm must be non-negative, got {max_norm}")
             coef = float(max_norm) / (total + 1e-6)
             coef_c = torch.clamp(coef, max=1.0)
             _scale_all(tensors, eligible, table, coef_c, device)
@@ -105,6 +102,31 @@ class GlobalNormMuonClipStrategy:
                                  norm_type=context.norm_type, clip_coef=clip_coef,
                                  clipped=clipped, param_count=len(entries),
                                  found_inf=~torch.isfinite(total), strategy=self.name)
+
+
+    def _on_kernels(self, context: MuonGradClipContext, table) -> MuonGradClipStats:
+        """Every gradient on the kernels, one rank: norms, coefficient and flags in one pass over
+        the gradients, then the scaling."""
+        max_norm = context.max_norm
+        norms, coefs, clipped, found_inf = table.norms(0, max_norm)
+        _check_total(context, norms[0])
+        if max_norm is not None:
+            table.scale(coefs, segments=table.zero_segments)
+        return MuonGradClipStats(
+            total_norm=norms[0], max_norm=max_norm, norm_type=context.norm_type,
+            clip_coef=1.0 if max_norm is None else coefs[0],
+            clipped=False if max_norm is None else clipped[0],
+            param_count=len(context.entries), found_inf=found_inf[0], strategy=self.name)
+
+
+def _check_total(context: MuonGradClipContext, total: torch.Tensor) -> None:
+    if context.error_if_nonfinite and bool(torch.logical_or(total.isnan(), total.isinf())):
+        raise RuntimeError(
+            f"The total norm of order {context.norm_type} for DMuon Muon gradients is "
+            "non-finite, so it cannot be clipped. To disable this error and scale the "
+            "gradients by the non-finite norm anyway, set `error_if_nonfinite=False`.")
+    if context.max_norm is not None and context.max_norm < 0:
+        raise ValueError(f"max_norm must be non-negative, got {context.max_norm}")
 
 
 def _total_norm(tensors, eligible, table, p, device) -> torch.Tensor:

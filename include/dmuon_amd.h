@@ -421,6 +421,28 @@ int dmuon_segmented_scale(const int64_t* ptrs, const int64_t* numels, const int3
                           const int64_t* job_offsets, int64_t n_jobs, int64_t chunk_size,
                           const float* coefs, void* stream);
 
+/*
+ * Norms, clip coefficients and flags of the tensors of such a job table, in two launches and
+ * without atomics (the same bits on every call). Tensor t's jobs are first_job[t] ..
+ * first_job[t + 1] - 1 (DEVICE array of n_tensors + 1).
+ *   n_segments > 0: norms[s] = sqrt of segment s's sum of squares, coefs[s] = min(max_norm /
+ *     (norms[s] + 1e-6), 1), clipped[s] = norms[s] finite and > max_norm, found_inf[s] = not
+ *     finite; norms[n_segments] = the 2-norm of the segments' norms.
+ *   n_segments == 0: one norm over all tensors, each tensor's norm first rounded to its dtype
+ *     (as torch._foreach_norm returns it): norms[0], coefs[0], clipped[0] (coefficient < 1 and
+ *     the norm finite), found_inf[0].
+ * max_norm NaN: no limit (coefficients 1, clipped 0). A coefficient of a non-finite norm is what
+ * the division gives. The workspace (8-byte aligned) has dmuon_clip_workspace_size bytes.
+ */
+int dmuon_clip_workspace_size(int64_t n_jobs, int64_t chunk_size, int n_tensors,
+                              int64_t* workspace_bytes);
+int dmuon_clip_norms(const int64_t* ptrs, const int64_t* numels, const int32_t* dtypes,
+                     const int32_t* segments, const int32_t* job_tensor_ids,
+                     const int64_t* job_offsets, const int32_t* first_job, int64_t n_jobs,
+                     int64_t chunk_size, int n_tensors, int n_segments, double max_norm,
+                     float* norms, float* coefs, uint8_t* clipped, uint8_t* found_inf,
+                     void* workspace, int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

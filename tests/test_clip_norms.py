@@ -1,0 +1,83 @@
+"""``dmuon_clip_norms``: norms, coefficients and flags of a job table in two launches."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+from dmuon_amd import _C, fast_clip
+from dmuon_amd.fast_clip import GradClipBucket, clip_grad_norm_buckets_
+
+
+def test_workspace_and_refusals():
+    lib, need = _C.lib(), ctypes.c_int64()
+    size = lambda *a: lib.dmuon_clip_workspace_size(*a, ctypes.byref(need))  # noqa: E731
+    assert size(1, 262144, 1) == 0 and need.value == 8 + 4 * 32     # pieces of at least 8192
+    assert size(10000, 262144, 3) == 0 and need.value == 24 + 4 * 10000
+    assert size(0, 16, 2) == 0 and need.value == 16
+    assert size(-1, 16, 2) != 0 and size(1, 0, 2) != 0
+    q, ws = 4096, 1 << 20
+    call = lambda **k: lib.dmuon_clip_norms(  # noqa: E731
+        q, q, q, q, q, q, k.get("first", q), 1, 16, k.get("n", 1), 1, 1.0, q, k.get("coefs", q), q,
+        q, k.get("ws", 8), k.get("bytes", ws), None)
+    for bad in (dict(n=0), dict(first=None), dict(coefs=None), dict(ws=None), dict(ws=12),
+                dict(bytes=4)):
+        assert call(**bad) != 0, bad
+
+
+def _grads(sizes, dtypes, gpu, seed):
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    return [torch.randn(n, device=gpu, generator=gen).to(dt) for n, dt in zip(sizes, dtypes)]
+
+
+DT = [torch.float32, torch.bfloat16, torch.float16]
+# empty and single-element tensors, sizes around a piece and a job, more tensors and segments than
+# the finishing block has waves, jobs enough that a piece is a whole job
+CASES = [([1], None), ([0, 5], None), ([8191, 8192, 8193, 262144, 262145], None),
+         (list(range(1, 40)), None), ([3_000_000, 17, 70_001], None),
+         ([4096 * 257], 256)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,chunk", CASES)
+@pytest.mark.parametrize("max_norm", [None, 0.5, 1e6])
+def test_segments_against_float64(gpu, sizes, chunk, max_norm):
+    dts = [DT[i % 3] for i in range(len(sizes))]
+    grads = _grads(sizes, dts, gpu, len(sizes))
+    before = [g.double() for g in grads]
+    buckets = tuple(GradClipBucket(str(i), [g], reduce=False) for i, g in enumerate(grads))
+    first = [s.total_norm.clone() for s in
+             clip_grad_norm_buckets_(buckets, None, chunk_size=chunk).bucket_stats]
+    res = clip_grad_norm_buckets_(buckets, max_norm, chunk_size=chunk)
+    total = 0.0
+    for s, f, g, b in zip(res.bucket_stats, first, grads, before):
+        norm = float(b.norm())
+        total += norm * norm
+        assert torch.equal(s.total_norm, f)                     # the same bits on every call
+        assert float(s.total_norm) == pytest.approx(norm, rel=1e-6, abs=1e-30)
+        coef = 1.0 if max_norm is None else min(1.0, max_norm / (norm + 1e-6))
+        assert float(s.clip_coef) == pytest.approx(coef, rel=1e-6)
+        assert bool(s.clipped) == (max_norm is not None and norm > max_norm)
+        assert not bool(s.found_inf)
+        want = b if max_norm is None else b.float() * s.clip_coef
+        assert torch.equal(g, want.to(g.dtype))
+    assert float(res.total_norm) == pytest.approx(math.sqrt(total), rel=1e-6, abs=1e-30)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_one_norm_over_all_rounds_each_to_its_dtype(gpu, bad):
+    sizes = [70_001, 33, 262_145, 8192] * 5
+    grads = _grads(sizes, [DT[i % 3] for i in range(len(sizes))], gpu, 3)
+    table = fast_clip._JobTable(grads, list(range(len(grads))), gpu, 262144)
+    norms, coefs, clipped, found = table.norms(0, 1.0)
+    want = math.sqrt(sum(float(g.double().norm().to(g.dtype)) ** 2 for g in grads))
+    assert float(norms[0]) == pytest.approx(want, rel=1e-6)
+    assert float(coefs[0]) == pytest.approx(1.0 / (want + 1e-6), rel=1e-6)
+    assert bool(clipped[0]) and not bool(found[0])
+    assert float(table.norms(0, None)[1][0]) == 1.0 and not bool(table.norms(0, None)[2][0])
+    grads[3][5] = bad
+    norms, coefs, clipped, found = table.norms(0, 1.0)
+    assert not math.isfinite(float(norms[0])) and bool(found[0]) and not bool(clipped[0])
+    want = 0.0 if bad == float("inf") else bad
+    assert float(coefs[0]) == want or math.isnan(want) and math.isnan(float(coefs[0]))
