@@ -211,10 +211,11 @@ int plan(int rows, int cols, int batch, int tile_req, int num_cus, int gram, int
 
 // Estimated time (us) of the Newton-Schulz products of a call's groups on `tile`-tiles: each
 // product is one launch over all of them, whose time is that of its longest tile or of its
-// work spread over the machine, whichever is more, plus a fixed part per launch. A tile's time is
-// fixed + slices of K (64 wide) at the kernel's rate, measured on MI355X as K sweeps of triangle
-// products (us): 256-tiles 13 + 1.0 per slice, 128-tiles one per CU 6 + 0.39, two per CU
-// 6 + 0.68 for the pair, 64-tiles 5 + 0.18. Only the comparison of two splits matters.
+// work spread over the machine, whichever is more, plus 2 us from launch to launch. A tile's time
+// is fixed + slices of K (64 wide) at its kernel's rate, measured on MI355X as K sweeps (64 ..
+// 8192) of triangle products with 36 .. 1020 tiles: 256-tiles 13 us + 1.0 per slice on a third of
+// the CUs and 1.4 on all of them, 128-tiles one per CU 6 + 0.39 .. 0.46, two per CU 8 + 0.93 for
+// the pair, 64-tiles 5 + 0.18. Only the comparison of two splits matters.
 double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, bool gram) {
   // launches of one NS run of five steps: X X^T, m x m triangle products, Q updates, P X
   const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_full = gram ? 3 : 0,
@@ -226,12 +227,12 @@ double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, b
       return tiles;
     };
     int t = tile;
-    double fixed = 13.0, slice = 1.0, slots = num_cus;
-    if (tile == 128) {
-      if (total(64) <= num_cus) t = 64, fixed = 5.0, slice = 0.18;
-      else if (total(128) <= num_cus) fixed = 6.0, slice = 0.39;
-      else fixed = 6.0, slice = 0.68, slots = 2.0 * num_cus;
-    }
+    double fixed = 13.0, slice = 0, slots = num_cus;
+    auto busy = [&](double tiles) { return tiles < num_cus ? tiles / num_cus : 1.0; };
+    if (tile == 256) slice = 0.85 + 0.55 * busy(total(256));
+    else if (total(64) <= num_cus) t = 64, fixed = 5.0, slice = 0.18;
+    else if (total(128) <= num_cus) fixed = 6.0, slice = 0.35 + 0.11 * busy(total(128));
+    else fixed = 8.0, slice = 0.93, slots = 2.0 * num_cus;
     double longest = 0, sum = 0;
     for (int i = 0; i < n; ++i) {
       const std::pair<double, double> d = dims(g[i], t);
@@ -243,6 +244,7 @@ double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, b
     const double spread = sum / slots + (total(t) > slots ? 0.5 * longest : 0.0);
     return (spread > longest ? spread : longest) + 2.0;
   };
+  // tiles along m and n: of the padded sides, 64-tiles of the sides rounded up to 64
   auto sides = [](const dmuon_muon_group& q, int t) {
     const int64_t m = q.rows < q.cols ? q.rows : q.cols, w = q.rows < q.cols ? q.cols : q.rows;
     return std::pair<double, double>((double)((m + t - 1) / t), (double)((w + t - 1) / t));

@@ -1283,11 +1283,15 @@ bool nt_args_ok(const NtArgs& a) {
   return true;
 }
 
-// The tile grid of a product on `tile` x `tile` tiles (M and N are multiples of it).
+// Tiles of a product on `tile` x `tile` tiles (M and N are multiples of it). On 64-tiles the
+// padding that no later product reads (live_rows / live_cols, multiples of 64) has none.
+long long tiles_of(const NtArgs& a, int tile, int* mt, int* nt) {
+  *mt = (tile == 64 && a.live_rows > 0 ? a.live_rows : a.M) / tile;
+  *nt = (tile == 64 && a.live_cols > 0 ? a.live_cols : a.N) / tile;
+  return a.tri ? (long long)*mt * (*mt + 1) / 2 : (long long)*mt * *nt;
+}
 void set_tiles(NtArgs& a, int tile) {
-  a.mt = a.M / tile;
-  a.nt = a.N / tile;
-  a.tiles_per_mat = a.tri ? a.mt * (a.mt + 1) / 2 : a.mt * a.nt;
+  a.tiles_per_mat = (int)tiles_of(a, tile, &a.mt, &a.nt);
 }
 
 // One launch of `nb` blocks: p is the one product, or the table of several.
@@ -1370,10 +1374,10 @@ hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream)
   bool split256 = true;
   for (int i = 0; i < cnt; ++i) {
     const NtArgs& p = a[order[i]];
-    const long long t2 = p.M / 256, u2 = p.N / 256, t4 = p.M / 64, u4 = p.N / 64;
+    int mt, nt;
     nb += (long long)p.tiles_per_mat * p.L;
-    nb256 += (p.tri ? t2 * (t2 + 1) / 2 : t2 * u2) * p.L;
-    nb64 += (p.tri ? t4 * (t4 + 1) / 2 : t4 * u4) * p.L;
+    nb256 += tiles_of(p, 256, &mt, &nt) * p.L;
+    nb64 += tiles_of(p, 64, &mt, &nt) * p.L;
     split256 = split256 && p.M % 256 == 0 && p.N % 256 == 0;
   }
   NtKernel kernel = tile == 256 ? NT_PP256 : NT_128;

@@ -391,7 +391,8 @@ class Muon(torch.optim.Optimizer):
                     continue
                 joined = self._plan_call(s[1] + (size,), num_cus, backend)
                 saved = s[4] + us - joined[2]
-                if saved > 0 and joined[1] <= self._workspace_limit and \
+                # by more than the estimates' own error on near ties
+                if saved > 0.01 * joined[2] and joined[1] <= self._workspace_limit and \
                         (best is None or saved > best[0]):
                     best = (saved, s, joined)
             if best is None:
