@@ -65,6 +65,10 @@ struct NtArgs {
   // sub-tile lies wholly in it does no MFMA work and stores nothing; the padding then holds
   // whatever it held.
   int live_rows, live_cols;
+  // EPI_SYM, tri: the operands are the caller's own, m_real x k_real inside the M x K of the tile
+  // grid and slices (multiples of 8 elements, 16-byte aligned rows): loads past them give 0,
+  // nothing past m_real is stored and the addend is read inside it only
+  int edge, k_real;
 };
 enum { DIAG_SKIP_NONE = 0, DIAG_SKIP_WAVES = 1, DIAG_SKIP_BLOCKS = 2 };
 enum { C_NONE = 0, C_IS_A = 1, C_IS_B = 2 };

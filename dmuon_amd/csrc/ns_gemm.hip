@@ -352,7 +352,9 @@ __device__ __forceinline__ TilePos decode_tile(const NtArgs& a, int lb) {
 // Epilogue of a finished tile: the accumulators of this wave (rows iw.., columns jw.. of
 // matrix l) through the MODE-specific staging and stores. Uses the per-wave LDS area
 // smem + wave * EPI_REGION; the caller guarantees no operand slice is still in use there.
-template <class T, int MODE, int E, class Acc>
+// EDGE (EPI_SYM): the operands end at m_real x k_real inside the last tiles (NtArgs::edge); whole
+// 8-value chunks lie in or out.
+template <class T, int MODE, int E, bool EDGE, class Acc>
 __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const Acc& acc, int l,
                                             int bi, int bj, int i0, int j0, int lane, int wave,
                                             int wi, int wj) {
@@ -373,8 +375,13 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
     const uint16_t* crow =
         Cb + (long long)(iw + 32 * x + lane / CLR) * a.ldc + jw + 4 * (lane % CLR);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-      dst[q] = *reinterpret_cast<const u32x2_t*>(crow + (long long)(CRI * q) * a.ldc);
+    for (int q = 0; q < NQ; ++q) {
+      if (EDGE && (iw + 32 * x + lane / CLR + CRI * q >= a.m_real ||
+                   jw + 4 * (lane % CLR) >= a.m_real))
+        dst[q] = u32x2_t{0, 0};
+      else
+        dst[q] = *reinterpret_cast<const u32x2_t*>(crow + (long long)(CRI * q) * a.ldc);
+    }
   };
   float s = a.alpha;
   if (a.alpha_dev) s *= a.alpha_dev[l];
@@ -491,9 +498,12 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
           // non-temporal: the outputs of a launch exceed L2 and the next product streams them
           // back from HBM / Infinity Cache anyway (measured 0.9% on the c5 step)
 #pragma unroll
-          for (int k = 0; k < NR; ++k)
+          for (int k = 0; k < NR; ++k) {
+            if (EDGE && (iw + 32 * x + cr + k * RPIT >= a.m_real || jw + 8 * cc >= a.m_real))
+              continue;
             __builtin_nontemporal_store(
                 dv[k], reinterpret_cast<u32x4_t*>(Db + doff + (long long)k * RPIT * a.ldd));
+          }
           if (D2b) {
 #pragma unroll
             for (int k = 0; k < NR; ++k)
@@ -551,6 +561,7 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
           const u32x4_t v = *reinterpret_cast<const u32x4_t*>(regt + (r0 + cr) * T::EPT + 16 * cc);
           // diagonal tile: output row j keeps columns i < j (chunk i0 .. i0+7)
           const int dj = jw + r0 + cr, di = ip + 8 * cc;
+          if (EDGE && (dj >= a.m_real || di >= a.m_real)) continue;
           if (!diag || di + 7 < dj) {
             __builtin_nontemporal_store(v,
                                         reinterpret_cast<u32x4_t*>(dst + (long long)r0 * ldt));
@@ -770,7 +781,8 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
   }
 }
 
-template <int BM, int BN, int BK, int S, int WM, int WN, int MODE, int E, bool BKM, class ARGS>
+template <int BM, int BN, int BK, int S, int WM, int WN, int MODE, int E, bool BKM, bool EDGE,
+          class ARGS>
 __global__ __launch_bounds__(64 * WM * WN)
 __attribute__((amdgpu_waves_per_eu(Occupancy<BM, BN, BK, S, WM, WN>::WPE,
                                    Occupancy<BM, BN, BK, S, WM, WN>::WPE)))
@@ -830,17 +842,38 @@ void nt_mfma_kernel(const ARGS args) {
       offb[q] = (unsigned)(r * a.ldb + T::slot(lsl, r) * 8) * 2u;
     }
   }
+  // EDGE: a lane whose row ends past the operand always reads 0 (an offset past any buffer range),
+  // and one whose chunk lies past k_real does in the last slice (the value ORed in there)
+  constexpr unsigned kOutside = 0x80000000u;
+  unsigned taila[8], tailb[8];
+  if constexpr (EDGE) {
+    static_assert(!BKM && MODE == EPI_SYM, "edges of a symmetric product");
+    const int ktail = a.k_real - (a.K - BK);        // values of the last slice
+#pragma unroll
+    for (int q = 0; q < T::A_INST; ++q) {
+      const int r = (T::NW * q + wave) * T::RPI + lrow;
+      if (i0 + r >= a.m_real) offa[q] = kOutside;
+      taila[q] = T::slot(lsl, r) * 8 >= ktail ? kOutside : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < T::B_INST; ++q) {
+      const int r = (T::NW * q + wave) * T::RPI + lrow;
+      if (j0 + r >= a.m_real) offb[q] = kOutside;
+      tailb[q] = T::slot(lsl, r) * 8 >= ktail ? kOutside : 0u;
+    }
+  }
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // The loads are MUBUF buffer loads into LDS (buffer_load_dwordx4 ... lds): one resource per
   // operand panel of this tile (SGPR base, range = the panel's rows), 32-bit lane offsets, the
   // slice offset in soffset. Cheaper to issue than 64-bit-address global loads (measured 1-3%
   // on the full kernel) and range-checked by the hardware: an offset past the panel reads 0.
   // Word 3 0x00020000: 32-bit data format, as gfx9 raw buffers use.
+  const int rowsA = EDGE ? min(BM, a.m_real - i0) : BM, rowsB = EDGE ? min(BN, a.m_real - j0) : BN;
   const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(Ab), (short)0, (int)((long long)BM * a.lda * 2), 0x00020000);
+      const_cast<uint16_t*>(Ab), (short)0, (int)((long long)rowsA * a.lda * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(Bb), (short)0,
-      (int)((long long)(BKM ? a.K : BN) * a.ldb * 2), 0x00020000);
+      (int)((long long)(BKM ? a.K : rowsB) * a.ldb * 2), 0x00020000);
   const unsigned kstepB = BKM ? (unsigned)a.ldb : 1u;   // B slice offset: k-rows or k values
   // slice sl_ of A and B into ring slot slot_ (this wave's share)
 #define DMUON_ISSUE(slice_, slot_)                                                             \
@@ -848,12 +881,15 @@ void nt_mfma_kernel(const ARGS args) {
     char* st_ = smem + (slot_) * T::STAGE + wave * 1024;                                       \
     const unsigned so_ = (unsigned)((slice_) * BK * 2);                                        \
     const unsigned sob_ = so_ * kstepB;                                                        \
+    const unsigned tl_ = EDGE && (slice_) == a.K / BK - 1 ? kOutside : 0u;                     \
     _Pragma("unroll") for (int q = 0; q < T::A_INST; ++q)                                      \
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_ptr_t)(st_ + q * 1024 * T::NW), 16, \
-                                                 offa[q], so_, 0, 0);                          \
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(                                              \
+            rsA, (lds_ptr_t)(st_ + q * 1024 * T::NW), 16,                                      \
+            EDGE ? offa[q] | (taila[q] & tl_) : offa[q], so_, 0, 0);                           \
     _Pragma("unroll") for (int q = 0; q < T::B_INST; ++q)                                      \
         __builtin_amdgcn_raw_ptr_buffer_load_lds(                                              \
-            rsB, (lds_ptr_t)(st_ + T::A_BYTES + q * 1024 * T::NW), 16, offb[q], sob_, 0, 0);   \
+            rsB, (lds_ptr_t)(st_ + T::A_BYTES + q * 1024 * T::NW), 16,                         \
+            EDGE ? offb[q] | (tailb[q] & tl_) : offb[q], sob_, 0, 0);                          \
   } while (0)
 
   // the wave sub-tile as BI x BJ blocks of 16x16 (v_mfma_f32_16x16x32)
@@ -953,8 +989,8 @@ void nt_mfma_kernel(const ARGS args) {
   wait_vmcnt<0>();
   bare_barrier();
 
-  nt_epilogue<T, MODE, E>(a, smem, Acc16<BI, BJ>{acc, lane}, l, bi, bj, i0, j0, lane, wave, wi,
-                          wj);
+  nt_epilogue<T, MODE, E, EDGE>(a, smem, Acc16<BI, BJ>{acc, lane}, l, bi, bj, i0, j0, lane, wave,
+                                wi, wj);
 }
 
 // Ping-pong schedule of the 256x256 tile with 8 waves of 128x64 (wave w and w + 4 share a SIMD).
@@ -1174,8 +1210,8 @@ __device__ __forceinline__ void pp_tile(const NtArgs& a, char* smem, int l, int 
   wait_vmcnt<0>();
   // a diagonal-tile wave whose values all lie below the diagonal has nothing to store
   if constexpr (LIM >= -3)
-    nt_epilogue<T, MODE, E>(a, smem, Acc16<8, 4>{acc, lane}, l, bi, bj, i0, j0, lane, wave, wi,
-                            wj);
+    nt_epilogue<T, MODE, E, false>(a, smem, Acc16<8, 4>{acc, lane}, l, bi, bj, i0, j0, lane, wave,
+                                   wi, wj);
 }
 
 template <int BK, int S, int MODE, int E, bool BKM, class ARGS>
@@ -1277,6 +1313,13 @@ bool nt_args_ok(const NtArgs& a) {
     return false;
   if (a.c_in != C_NONE && a.c_in != C_IS_A && a.c_in != C_IS_B) return false;
   if (a.k_loop < 0 || a.k_loop > a.K || a.k_loop % 64 != 0) return false;
+  // operands that end inside the last tiles: whole 16-byte chunks of a symmetric product whose
+  // last tile row and last slice hold something
+  if (a.edge && !(a.mode == EPI_SYM && a.tri && !a.sym_exact && !a.b_kmajor && !a.D2 &&
+                  a.M == a.N && a.k_loop == 0 && a.m_real % 8 == 0 && a.k_real % 8 == 0 &&
+                  a.m_real > a.M - 128 && a.m_real <= a.M && a.k_real > a.K - 64 &&
+                  a.k_real <= a.K && a.lda >= a.k_real && a.ldb >= a.k_real))
+    return false;
   if (a.live_rows < 0 || a.live_rows % 64 != 0 || a.live_cols < 0 || a.live_cols % 64 != 0 ||
       (a.tri && a.live_rows != a.live_cols))
     return false;
@@ -1299,8 +1342,15 @@ template <int BM, int S, int WM, int WN, int E, class ARGS>
 void launch_mfma(const ARGS& p, int mode, bool kmajor, long long nb, hipStream_t stream) {
   const dim3 grid((unsigned)nb), block(64 * WM * WN);
 #define DMUON_NT(MODE, KM)                                                                     \
-  hipLaunchKernelGGL((nt_mfma_kernel<BM, BM, 64, S, WM, WN, MODE, E, KM, ARGS>), grid, block,  \
-                     0, stream, p)
+  hipLaunchKernelGGL((nt_mfma_kernel<BM, BM, 64, S, WM, WN, MODE, E, KM, false, ARGS>), grid,  \
+                     block, 0, stream, p)
+  if constexpr (std::is_same<ARGS, NtArgs>::value) {
+    if (p.edge) {                       // nt_args_ok: a symmetric product, B not k-major
+      hipLaunchKernelGGL((nt_mfma_kernel<BM, BM, 64, S, WM, WN, EPI_SYM, E, false, true, ARGS>),
+                         grid, block, 0, stream, p);
+      return;
+    }
+  }
   if (mode == EPI_SYM) { if (kmajor) DMUON_NT(EPI_SYM, true); else DMUON_NT(EPI_SYM, false); }
   else if (mode == EPI_NS) { if (kmajor) DMUON_NT(EPI_NS, true); else DMUON_NT(EPI_NS, false); }
   else { if (kmajor) DMUON_NT(EPI_FINAL, true); else DMUON_NT(EPI_FINAL, false); }
@@ -1380,11 +1430,13 @@ hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream)
     nb64 += tiles_of(p, 64, &mt, &nt) * p.L;
     split256 = split256 && p.M % 256 == 0 && p.N % 256 == 0;
   }
+  const bool edge = a[order[0]].edge != 0;       // runs on the 128- and 64-tile kernels only
+  if (edge && (cnt > 1 || tile != 128)) return hipErrorInvalidValue;
   NtKernel kernel = tile == 256 ? NT_PP256 : NT_128;
   if (tile != 256 && cus > 0) {
     const double c256 = 4.0 * (double)((nb256 + cus - 1) / cus);
     const double c128 = 2.7 * (double)((nb + 2LL * cus - 1) / (2LL * cus));
-    if (split256 && nb > 2LL * cus && c256 < c128) kernel = NT_PP256, nb = nb256;
+    if (!edge && split256 && nb > 2LL * cus && c256 < c128) kernel = NT_PP256, nb = nb256;
     else if (nb64 <= cus) kernel = NT_64, nb = nb64;
     else if (nb <= cus) kernel = NT_128_DEEP;
   }
