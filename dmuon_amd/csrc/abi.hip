@@ -338,27 +338,35 @@ double update_bytes(const Group& g) {
                   (g.pub_ptrs ? width(g.pub_dtype) : 0.0));
 }
 
-// One product of the iteration over the groups of a call: fill(group, args) sets a group's
-// operands, work(group) its useful FLOPs.
+// The args of one product for each group of a call: fill(group, args) sets a group's operands.
 template <class Fill>
-int nt_product(const Call& c, int cls, double (*work)(const Group&), Fill&& fill) {
-  NtArgs a[kMaxGroups];
-  double flops = 0.0, bytes = 0.0;
+void product_args(const Call& c, NtArgs* a, Fill&& fill) {
   for (int i = 0; i < c.n; ++i) {
-    Group& g = c.g[i];
     NtArgs& s = a[i];
     s = NtArgs{};
     s.elt = ELT_F16;
-    s.L = g.batch;
-    fill(g, s);
+    s.L = c.g[i].batch;
+    fill(c.g[i], s);
     s.mt = s.M / c.tile;
     s.nt = s.N / c.tile;
     s.tiles_per_mat = s.tri ? tri_tiles(s.M, c.tile) : s.mt * s.nt;
-    flops += work(g);
-    if (cls == PC_FINAL) bytes += update_bytes(g);
+  }
+}
+
+// One product of the iteration over the groups of a call, work(group) its useful FLOPs; with
+// `more`, tiles of that product too (launch_nt_fill).
+template <class Fill>
+int nt_product(const Call& c, int cls, double (*work)(const Group&), Fill&& fill,
+               NtFill* more = nullptr, bool all = false) {
+  NtArgs a[kMaxGroups];
+  product_args(c, a, fill);
+  double flops = 0.0, bytes = 0.0;
+  for (int i = 0; i < c.n; ++i) {
+    flops += work(c.g[i]) + (more && all ? square_flops(c.g[i]) : 0.0);
+    if (cls == PC_FINAL) bytes += update_bytes(c.g[i]);
   }
   return timed(cls, flops, bytes, c.stream, c.who,
-               [&] { return launch_nt_batch(a, c.n, c.tile, c.stream); });
+               [&] { return launch_nt_fill(a, c.n, more, all, c.tile, c.stream); });
 }
 
 // K loop lengths: the operands are zero past m (n), so the products multiply only m (n) rounded
@@ -492,17 +500,26 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
   // that consumes Q, which writes only its transposed output, the row form Q that Q X reads.
   // A Q that is still P itself (after a start or restart) is symmetric and serves as either
   // form. Two slots, used in turn.
-  auto q_update = [&](int from, float a_, bool last) -> int {
+  auto q_args = [&](Group& g, NtArgs& s, int from, float a_, bool last) {
     const int to = 1 - from;
-    return nt_product(c, PC_POLY, square_flops, [&](Group& g, NtArgs& s) {
-      square_operands(g, s, g.qslot[from], g.w.Pm, g.qslot[from]);
-      s.mode = EPI_NS; s.alpha = 1.f; s.beta = a_;
-      s.c_in = C_IS_A;                           // the addend is the A panel's last slices
-      if (last) s.DT = g.qslot[to];              // Q, the row form
-      else s.D = g.qslot[to];                    // Q^T
-      g.qbuf[to] = g.qslot[to];
-    });
+    square_operands(g, s, g.qslot[from], g.w.Pm, g.qslot[from]);
+    s.mode = EPI_NS; s.alpha = 1.f; s.beta = a_;
+    s.c_in = C_IS_A;                           // the addend is the A panel's last slices
+    if (last) s.DT = g.qslot[to];              // Q, the row form
+    else s.D = g.qslot[to];                    // Q^T
+    g.qbuf[to] = g.qslot[to];
   };
+  auto q_update = [&](int from, float a_, bool last) -> int {
+    return nt_product(c, PC_POLY, square_flops,
+                      [&](Group& g, NtArgs& s) { q_args(g, s, from, a_, last); });
+  };
+  // A Q update with R's update and another step behind it: W, R and the next Z do not read Q, so
+  // its tiles go where these triangle launches leave CUs idle, and what is left runs with the
+  // last of them. One 4096^2 matrix: 136 tiles each on 256 CUs, so the 256 tiles of the update
+  // cost no launch of their own. As a D-only product it is EPI_SYM's arithmetic without a
+  // triangle (alpha = 1: the same bits). Needs a table entry per group.
+  NtFill fill;
+  bool filling = false;
   // iterations from it up to the next restart (or T): the Q updates the segment has left
   auto updates_left = [&](int it) {
     int end = it + 1;
@@ -531,28 +548,40 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
     // Z = c R^2 + b R; after a (re)start also Q = Z + a I, as the epilogue's second output, or,
     // when R is not updated afterwards (Z itself is not needed), as the only one
     const bool fresh = qs < 0, only_q = fresh && !evolve;
+    if (filling)   // the update still reads the old Z: the new one goes where W was
+      for (int i = 0; i < c.n; ++i) std::swap(c.g[i].w.Pm, c.g[i].w.Wm);
     if (nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
           uint16_t* R = g.w.Am;
           symmetric_square(g, s, R, R, R, only_q ? g.qslot[0] : g.w.Pm, cc / (g.rs * g.rs),
                            cb / g.rs, only_q ? ca : 0.f, fresh && evolve ? g.qslot[0] : nullptr,
                            fresh && evolve ? ca : 0.f);
           if (fresh) g.qbuf[0] = g.qslot[0];
-        }))
+        }, filling ? &fill : nullptr, true))
       return 1;
+    filling = false;
     if (fresh) {
       qs = 0;
+    } else if (evolve && 2 * c.n <= kMaxGroups) {
+      fill.next = 0;
+      product_args(c, fill.a, [&](Group& g, NtArgs& s) {
+        q_args(g, s, qs, ca, false);
+        s.mode = EPI_SYM;
+      });
+      filling = true;
+      qs = 1 - qs;
     } else {
       if (q_update(qs, ca, updates_left(it) == 1)) return 1;   // Q <- Z Q + a Q
       qs = 1 - qs;
     }
     if (evolve) {
       // W = Z R + a R (the stored R is rs times R), then R = P R P = W Z + a W
+      NtFill* more = filling ? &fill : nullptr;
       if (nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
             symmetric_square(g, s, g.w.Pm, g.w.Am, g.w.Am, g.w.Wm, 1.f, ca, 0.f);
-          }) ||
+          }, more) ||
           nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
             symmetric_square(g, s, g.w.Wm, g.w.Pm, g.w.Wm, g.w.Am, 1.f / g.rs, ca / g.rs, 0.f);
-          }))
+          }, more))
         return 1;
       for (int i = 0; i < c.n; ++i) c.g[i].rs = 1.f;
     }

@@ -29,6 +29,8 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # no a*b+c contraction: the momentum and weight updates round each op like the reference
     "-ffp-contract=off",
+    # leading scalar kernel arguments arrive in SGPRs instead of by a load from memory
+    "-mllvm", "-amdgpu-kernarg-preload-count=8",
     "-Wall",
     "-Wno-unused-function",
 ]

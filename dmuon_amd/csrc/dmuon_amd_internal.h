@@ -69,6 +69,8 @@ struct NtArgs {
   // grid and slices (multiples of 8 elements, 16-byte aligned rows): loads past them give 0,
   // nothing past m_real is stored and the addend is read inside it only
   int edge, k_real;
+  // first tile of the launch (a product whose tiles are spread over several launches)
+  int tile0;
 };
 enum { DIAG_SKIP_NONE = 0, DIAG_SKIP_WAVES = 1, DIAG_SKIP_BLOCKS = 2 };
 enum { C_NONE = 0, C_IS_A = 1, C_IS_B = 2 };
@@ -88,6 +90,15 @@ hipError_t launch_nt(const NtArgs& a, int tile, hipStream_t stream);
 // The same for n (1 .. kMaxGroups) fp16 products of one mode and B layout, in one launch. A
 // value's bits do not depend on what else the launch holds.
 hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream);
+// The same with tiles of a further product over the same shapes (as many args, of the same mode
+// and layout) in the CUs the launch would leave idle: `next` counts the tiles already done, of
+// all of them in order; `all` takes the rest. n + n <= kMaxGroups.
+struct NtFill {
+  NtArgs a[kMaxGroups];
+  long long next;
+};
+hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int tile,
+                          hipStream_t stream);
 // The logical tile the NT kernels give hardware block b of a launch of nb blocks (host copy of
 // the device mapping, for tests: it must be a permutation of 0 .. nb - 1).
 int nt_block_tile(int b, int nb);

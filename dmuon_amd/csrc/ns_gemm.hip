@@ -290,17 +290,25 @@ struct TilePos {
 
 // The product this block works on, and its tile among that product's tiles. A launch holds one
 // product (NtArgs) or several of different shapes (NtBatch); the XCD windows run over all of
-// the launch's tiles.
-__device__ __forceinline__ const NtArgs& block_args(const NtArgs& p, int& lb) {
+// the launch's tiles. The groups' first tiles are scalar arguments in front, which arrive in
+// registers with the wave (kernarg preload, see the build flags): the block then waits for its
+// own product's arguments only, as in a launch of one. Read from the table first, they cost every
+// joined launch a second trip to the argument memory (1.5 us of an 8-9 us launch).
+struct Firsts {
+  int f[kMaxGroups - 1];              // first tile of groups 1 .. 7 (INT_MAX past the last)
+};
+__device__ __forceinline__ const NtArgs& block_args(const NtArgs& p, const Firsts&, int& lb) {
   lb = xcd_remap(blockIdx.x, gridDim.x);
   return p;
 }
-__device__ __forceinline__ const NtArgs& block_args(const NtBatch& p, int& lb) {
+__device__ __forceinline__ const NtArgs& block_args(const NtBatch& p, const Firsts& s, int& lb) {
   const int t = xcd_remap(blockIdx.x, gridDim.x);
-  int g = 0;
-  while (g + 1 < p.n && t >= p.first[g + 1]) ++g;
+  int g = 0, base = 0;
+#pragma unroll
+  for (int i = 0; i < kMaxGroups - 1; ++i)
+    if (t >= s.f[i]) g = i + 1, base = s.f[i];
   g = __builtin_amdgcn_readfirstlane(g);
-  lb = t - p.first[g];
+  lb = t - __builtin_amdgcn_readfirstlane(base) + p.a[g].tile0;
   return p.a[g];
 }
 
@@ -781,12 +789,13 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
   }
 }
 
+#define DMUON_FIRSTS int f1, int f2, int f3, int f4, int f5, int f6, int f7
 template <int BM, int BN, int BK, int S, int WM, int WN, int MODE, int E, bool BKM, bool EDGE,
           class ARGS>
 __global__ __launch_bounds__(64 * WM * WN)
 __attribute__((amdgpu_waves_per_eu(Occupancy<BM, BN, BK, S, WM, WN>::WPE,
                                    Occupancy<BM, BN, BK, S, WM, WN>::WPE)))
-void nt_mfma_kernel(const ARGS args) {
+void nt_mfma_kernel(DMUON_FIRSTS, const ARGS args) {
   using T = Tile<BM, BN, BK, S, WM, WN>;
   __shared__ __attribute__((aligned(16))) char smem[T::LDS_BYTES];
   static_assert(T::LDS_BYTES <= 160 * 1024, "LDS budget");
@@ -802,7 +811,7 @@ void nt_mfma_kernel(const ARGS args) {
   // the decode is the same for every lane; readfirstlane states it, so the buffer descriptors
   // and offsets built from it stay scalar whatever the compiler's uniformity analysis proves
   int lb;
-  const NtArgs& a = block_args(args, lb);
+  const NtArgs& a = block_args(args, Firsts{{f1, f2, f3, f4, f5, f6, f7}}, lb);
   const TilePos tp = decode_tile(a, lb);
   const int l = __builtin_amdgcn_readfirstlane(tp.l);
   const int bi = __builtin_amdgcn_readfirstlane(tp.bi), bj = __builtin_amdgcn_readfirstlane(tp.bj);
@@ -1216,14 +1225,14 @@ __device__ __forceinline__ void pp_tile(const NtArgs& a, char* smem, int l, int 
 
 template <int BK, int S, int MODE, int E, bool BKM, class ARGS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void nt_pp_kernel(const ARGS args) {
+void nt_pp_kernel(DMUON_FIRSTS, const ARGS args) {
   using T = Tile<256, 256, BK, S, 2, 4>;
   __shared__ __attribute__((aligned(16))) char smem[T::LDS_BYTES];
   static_assert(T::LDS_BYTES <= 160 * 1024, "LDS budget");
   // the decode is the same for every lane; readfirstlane states it, so the buffer descriptors
   // and offsets built from it stay scalar whatever the compiler's uniformity analysis proves
   int lb;
-  const NtArgs& a = block_args(args, lb);
+  const NtArgs& a = block_args(args, Firsts{{f1, f2, f3, f4, f5, f6, f7}}, lb);
   const TilePos tp = decode_tile(a, lb);
   const int l = __builtin_amdgcn_readfirstlane(tp.l);
   const int bi = __builtin_amdgcn_readfirstlane(tp.bi), bj = __builtin_amdgcn_readfirstlane(tp.bj);
@@ -1338,29 +1347,39 @@ void set_tiles(NtArgs& a, int tile) {
 }
 
 // One launch of `nb` blocks: p is the one product, or the table of several.
+Firsts firsts_of(const NtArgs&) { return Firsts{}; }
+Firsts firsts_of(const NtBatch& p) {
+  Firsts s;
+  for (int g = 1; g < kMaxGroups; ++g) s.f[g - 1] = g < p.n ? p.first[g] : 0x7fffffff;
+  return s;
+}
+template <class... P, class ARGS>
+void launch_args(void (*kernel)(P...), long long nb, int threads, hipStream_t stream,
+                 const ARGS& p) {
+  const Firsts s = firsts_of(p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(threads), 0, stream, s.f[0], s.f[1], s.f[2],
+                     s.f[3], s.f[4], s.f[5], s.f[6], p);
+}
 template <int BM, int S, int WM, int WN, int E, class ARGS>
 void launch_mfma(const ARGS& p, int mode, bool kmajor, long long nb, hipStream_t stream) {
-  const dim3 grid((unsigned)nb), block(64 * WM * WN);
-#define DMUON_NT(MODE, KM)                                                                     \
-  hipLaunchKernelGGL((nt_mfma_kernel<BM, BM, 64, S, WM, WN, MODE, E, KM, false, ARGS>), grid,  \
-                     block, 0, stream, p)
+#define DMUON_NT(MODE, KM, EDGE)                                                               \
+  launch_args(nt_mfma_kernel<BM, BM, 64, S, WM, WN, MODE, E, KM, EDGE, ARGS>, nb,              \
+              64 * WM * WN, stream, p)
   if constexpr (std::is_same<ARGS, NtArgs>::value) {
     if (p.edge) {                       // nt_args_ok: a symmetric product, B not k-major
-      hipLaunchKernelGGL((nt_mfma_kernel<BM, BM, 64, S, WM, WN, EPI_SYM, E, false, true, ARGS>),
-                         grid, block, 0, stream, p);
+      DMUON_NT(EPI_SYM, false, true);
       return;
     }
   }
-  if (mode == EPI_SYM) { if (kmajor) DMUON_NT(EPI_SYM, true); else DMUON_NT(EPI_SYM, false); }
-  else if (mode == EPI_NS) { if (kmajor) DMUON_NT(EPI_NS, true); else DMUON_NT(EPI_NS, false); }
-  else { if (kmajor) DMUON_NT(EPI_FINAL, true); else DMUON_NT(EPI_FINAL, false); }
+  if (mode == EPI_SYM) { if (kmajor) DMUON_NT(EPI_SYM, true, false); else DMUON_NT(EPI_SYM, false, false); }
+  else if (mode == EPI_NS) { if (kmajor) DMUON_NT(EPI_NS, true, false); else DMUON_NT(EPI_NS, false, false); }
+  else { if (kmajor) DMUON_NT(EPI_FINAL, true, false); else DMUON_NT(EPI_FINAL, false, false); }
 #undef DMUON_NT
 }
 template <int E, class ARGS>
 void launch_pp(const ARGS& p, int mode, bool kmajor, long long nb, hipStream_t stream) {
-  const dim3 grid((unsigned)nb), block(512);
 #define DMUON_PP(MODE, KM)                                                                     \
-  hipLaunchKernelGGL((nt_pp_kernel<64, 2, MODE, E, KM, ARGS>), grid, block, 0, stream, p)
+  launch_args(nt_pp_kernel<64, 2, MODE, E, KM, ARGS>, nb, 512, stream, p)
   if (mode == EPI_SYM) { if (kmajor) DMUON_PP(EPI_SYM, true); else DMUON_PP(EPI_SYM, false); }
   else if (mode == EPI_NS) { if (kmajor) DMUON_PP(EPI_NS, true); else DMUON_PP(EPI_NS, false); }
   else { if (kmajor) DMUON_PP(EPI_FINAL, true); else DMUON_PP(EPI_FINAL, false); }
@@ -1399,67 +1418,126 @@ void launch_kernel(NtKernel k, const ARGS& p, int mode, bool kmajor, long long n
 //    the 256-aligned block of the tile's columns. A k-major B is one 64-value block of 128-byte
 //    k-rows per slice;
 //  - else 128-tiles.
-hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream) {
-  if (n < 1 || n > kMaxGroups) return hipErrorInvalidValue;
-  // the longest K loops first: their tiles must not start last
-  int order[kMaxGroups], cnt = 0;
+namespace {
+
+// The products of a launch, the longest K loops first (their tiles must not start last).
+// Fails on a product the kernels may not run.
+hipError_t order_products(const NtArgs* a, int n, const NtArgs** out, int* cnt) {
+  *cnt = 0;
   for (int g = 0; g < n; ++g) {
     if ((long long)a[g].tiles_per_mat * a[g].L <= 0) continue;
     if (!nt_args_ok(a[g])) return hipErrorInvalidValue;
     if (a[g].mode != a[0].mode || a[g].b_kmajor != a[0].b_kmajor || a[g].elt != a[0].elt)
       return hipErrorInvalidValue;
     const int k = a[g].k_loop > 0 ? a[g].k_loop : a[g].K;
-    int at = cnt++;
+    int at = (*cnt)++;
     for (; at > 0; --at) {
-      const NtArgs& o = a[order[at - 1]];
+      const NtArgs& o = *out[at - 1];
       if ((o.k_loop > 0 ? o.k_loop : o.K) >= k) break;
-      order[at] = order[at - 1];
+      out[at] = out[at - 1];
     }
-    order[at] = g;
+    out[at] = &a[g];
   }
-  if (cnt == 0) return hipSuccess;
-  if (cnt > 1 && a[order[0]].elt != ELT_F16) return hipErrorInvalidValue;
+  return hipSuccess;
+}
+
+// The kernel of a launch of a `tile` plan, its tile, its blocks, and the blocks resident at once.
+struct NtChoice {
+  NtKernel kernel;
+  int tile;
+  long long nb, slots;
+};
+NtChoice choose_kernel(const NtArgs* const* a, int cnt, int tile) {
   const int cus = current_device_cus();
   long long nb = 0, nb256 = 0, nb64 = 0;
   bool split256 = true;
   for (int i = 0; i < cnt; ++i) {
-    const NtArgs& p = a[order[i]];
+    const NtArgs& p = *a[i];
     int mt, nt;
     nb += (long long)p.tiles_per_mat * p.L;
     nb256 += tiles_of(p, 256, &mt, &nt) * p.L;
     nb64 += tiles_of(p, 64, &mt, &nt) * p.L;
     split256 = split256 && p.M % 256 == 0 && p.N % 256 == 0;
   }
-  const bool edge = a[order[0]].edge != 0;       // runs on the 128- and 64-tile kernels only
-  if (edge && (cnt > 1 || tile != 128)) return hipErrorInvalidValue;
-  NtKernel kernel = tile == 256 ? NT_PP256 : NT_128;
-  if (tile != 256 && cus > 0) {
+  if (tile == 256) return {NT_PP256, 256, nb, cus};
+  if (cus > 0) {
     const double c256 = 4.0 * (double)((nb256 + cus - 1) / cus);
     const double c128 = 2.7 * (double)((nb + 2LL * cus - 1) / (2LL * cus));
-    if (!edge && split256 && nb > 2LL * cus && c256 < c128) kernel = NT_PP256, nb = nb256;
-    else if (nb64 <= cus) kernel = NT_64, nb = nb64;
-    else if (nb <= cus) kernel = NT_128_DEEP;
+    if (!a[0]->edge && split256 && nb > 2LL * cus && c256 < c128) return {NT_PP256, 256, nb256, cus};
+    if (nb64 <= cus) return {NT_64, 64, nb64, cus};
+    if (nb <= cus) return {NT_128_DEEP, 128, nb, cus};
   }
-  const int t = kernel == NT_PP256 ? 256 : kernel == NT_64 ? 64 : 128;
-  if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
-  const int mode = a[order[0]].mode;
-  const bool km = a[order[0]].b_kmajor != 0;
-  if (cnt == 1) {
-    NtArgs p = a[order[0]];
-    if (t != tile) set_tiles(p, t);
-    if (p.elt == ELT_F16) launch_kernel<ELT_F16>(kernel, p, mode, km, nb, stream);
-    else launch_kernel<ELT_BF16>(kernel, p, mode, km, nb, stream);
-    return hipGetLastError();
-  }
+  return {NT_128, 128, nb, 2LL * cus};
+}
+
+}  // namespace
+
+hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream) {
+  return launch_nt_fill(a, n, nullptr, false, tile, stream);
+}
+
+hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int tile,
+                          hipStream_t stream) {
+  if (n < 1 || n > kMaxGroups || (fill && 2 * n > kMaxGroups)) return hipErrorInvalidValue;
+  const NtArgs* list[kMaxGroups];
+  int cnt;
+  hipError_t e = order_products(a, n, list, &cnt);
+  if (e != hipSuccess) return e;
+  if (cnt == 0) return hipSuccess;
+  if ((cnt > 1 || fill) && a[0].elt != ELT_F16) return hipErrorInvalidValue;
+  // an edge product runs on the 128- and 64-tile kernels only
+  if (a[0].edge && (cnt > 1 || fill || tile != 128)) return hipErrorInvalidValue;
+  const NtChoice k = choose_kernel(list, cnt, tile);
+  long long nb = k.nb;
   NtBatch b;
-  b.n = cnt;
+  b.n = 0;
   b.first[0] = 0;
-  for (int i = 0; i < cnt; ++i) {
-    b.a[i] = a[order[i]];
-    if (t != tile) set_tiles(b.a[i], t);
-    b.first[i + 1] = b.first[i] + b.a[i].tiles_per_mat * b.a[i].L;
+  auto put = [&](const NtArgs& p, long long tile0, long long tiles) {
+    NtArgs& q = b.a[b.n];
+    q = p;
+    if (k.tile != tile) set_tiles(q, k.tile);
+    q.tile0 = (int)tile0;
+    const long long whole = (long long)q.tiles_per_mat * q.L;
+    b.first[b.n + 1] = b.first[b.n] + (int)(tiles < 0 ? whole : tiles);
+    ++b.n;
+    return whole;
+  };
+  if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
+  for (int i = 0; i < cnt; ++i) put(*list[i], 0, -1);
+  if (fill) {
+    const NtArgs* more[kMaxGroups];
+    int fcnt;
+    e = order_products(fill->a, n, more, &fcnt);
+    if (e != hipSuccess || fcnt != cnt || fill->a[0].mode != a[0].mode ||
+        fill->a[0].b_kmajor != a[0].b_kmajor || fill->a[0].elt != a[0].elt)
+      return hipErrorInvalidValue;
+    // as many tiles as the last wave leaves room for, or all that are left
+    long long room = k.slots > 0 ? (k.slots - nb % k.slots) % k.slots : 0;
+    if (all) room = 0x7fffffffLL - nb;
+    long long before = 0;             // tiles of the groups in front
+    for (int i = 0; i < fcnt && room > 0; ++i) {
+      int mt, nt;
+      const long long whole = tiles_of(*more[i], k.tile, &mt, &nt) * more[i]->L;
+      const long long from = fill->next > before ? fill->next - before : 0;
+      if (from < whole) {
+        const long long take = whole - from < room ? whole - from : room;
+        put(*more[i], from, take);
+        nb += take;
+        room -= take;
+        fill->next += take;
+      }
+      before += whole;
+    }
+    if (all && fill->next < before) return hipErrorInvalidValue;
   }
-  launch_kernel<ELT_F16>(kernel, b, mode, km, nb, stream);
+  const int mode = a[0].mode;
+  const bool km = a[0].b_kmajor != 0;
+  if (b.n == 1) {
+    if (b.a[0].elt == ELT_F16) launch_kernel<ELT_F16>(k.kernel, b.a[0], mode, km, nb, stream);
+    else launch_kernel<ELT_BF16>(k.kernel, b.a[0], mode, km, nb, stream);
+  } else {
+    launch_kernel<ELT_F16>(k.kernel, b, mode, km, nb, stream);
+  }
   return hipGetLastError();
 }
 

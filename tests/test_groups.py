@@ -66,6 +66,10 @@ CASES = [
     ([(512, 1024, 12, 4), (384, 640, 4, 4), (130, 250, 2, 1)], 128),
     ([(512, 1024, 24, 8), (1024, 1024, 8, 0), (256, 512, 8, 3)], 128),
     ([(256, 1024, 2, 1), (700, 500, 1, 0), (512, 768, 2, 1)], 256),
+    # five groups: too many to spread a Q update over other launches, which their own calls do
+    ([(256, 768, 3, 1), (300, 1000, 2, 1), (512, 512, 2, 0), (128, 128, 1, 0), (64, 640, 1, 0)], 128),
+    ([(512, 2048, 12, 4), (1024, 1024, 3, 0), (384, 640, 4, 4), (130, 250, 2, 1), (64, 64, 1, 0)], 128),
+    ([(512, 768, 2, 1), (256, 1024, 2, 1), (700, 500, 1, 0), (300, 300, 1, 0), (256, 256, 3, 0)], 256),
 ]
 
 
