@@ -602,9 +602,16 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
     // the last n_flip matrices of the batch are stored in the other orientation
     const bool tr = (a.transposed != 0) != (l >= a.L - a.n_flip);
     const long long pitch = tr ? a.m_real : a.n_real;
-    // 16-byte vectors need 16-byte aligned bases (torch allocations are; views may not be)
-    const bool valign = ((reinterpret_cast<uintptr_t>(wp) | reinterpret_cast<uintptr_t>(outp) |
-                          reinterpret_cast<uintptr_t>(pp)) & 15) == 0;
+    // The tensors' rows may start at any element (a pitch of 3001, a view's base): the vectors
+    // state the element's own alignment, which global memory takes.
+    typedef u32x4_t v16_t __attribute__((aligned(2)));
+    typedef u32x4_t v32_t __attribute__((aligned(4)));
+    auto at16 = [](void* p, long long i) {
+      return (__attribute__((address_space(1))) v16_t*)(static_cast<uint16_t*>(p) + i);
+    };
+    auto at32 = [](void* p, long long i) {
+      return (__attribute__((address_space(1))) v32_t*)(static_cast<float*>(p) + i);
+    };
 #pragma unroll
     for (int x = 0; x < Acc::SLABS; ++x) {
       u32x2_t cfin[NQ];
@@ -641,9 +648,10 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
       // normal orientation: vector = 8 consecutive j of one row i (8 lanes per 64-column row);
       // transposed: vector = 8 consecutive i of one original row j (4 lanes per 32-row column).
       // All weight loads of the slab are issued before any store. Vectors that cross the real
-      // extent, or rows whose pitch breaks 16-byte alignment, take the per-element path.
+      // extent take the per-element path. (So did every row whose pitch is no multiple of 8:
+      // the final product of two 1555x3001 matrices took 125 us against 54 for the same product
+      // without the update; 74 this way.)
       constexpr int NV = 32 * T::WTN / 8 / 64;
-      const bool vpitch = (pitch & 7) == 0 && valign;
       long long voff[NV];
       bool vfull[NV];
       int vr[NV], vc[NV];
@@ -656,21 +664,21 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
           vc[v] = (idx % (T::WTN / 8)) * 8;
           const int i = ibase + vr[v], j = jw + vc[v];
           voff[v] = (long long)i * pitch + j;
-          vfull[v] = vpitch && i < a.m_real && j + 7 < a.n_real;
+          vfull[v] = i < a.m_real && j + 7 < a.n_real;
         } else {
           vc[v] = idx / 4;
           vr[v] = (idx % 4) * 8;
           const int i = ibase + vr[v], j = jw + vc[v];
           voff[v] = (long long)j * pitch + i;
-          vfull[v] = vpitch && j < a.n_real && i + 7 < a.m_real;
+          vfull[v] = j < a.n_real && i + 7 < a.m_real;
         }
         if (wp && vfull[v]) {
           if (a.w_dtype == DT_F32) {
-            const u32x4_t* q = reinterpret_cast<const u32x4_t*>(static_cast<const float*>(wp) + voff[v]);
+            const auto q = at32(wp, voff[v]);
             wraw[v][0] = q[0];
             wraw[v][1] = q[1];
           } else {
-            wraw[v][0] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(wp) + voff[v]);
+            wraw[v][0] = *at16(wp, voff[v]);
           }
         }
       }
@@ -683,7 +691,7 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
         if (vfull[v]) {
           if (outp) {
             if (a.out_dtype == DT_F32) {
-              u32x4_t* q = reinterpret_cast<u32x4_t*>(static_cast<float*>(outp) + voff[v]);
+              const auto q = at32(outp, voff[v]);
               q[0] = u32x4_t{__float_as_uint(u[0]), __float_as_uint(u[1]), __float_as_uint(u[2]),
                              __float_as_uint(u[3])};
               q[1] = u32x4_t{__float_as_uint(u[4]), __float_as_uint(u[5]), __float_as_uint(u[6]),
@@ -694,7 +702,7 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
               o.y = (unsigned)f2bf(u[2]) | ((unsigned)f2bf(u[3]) << 16);
               o.z = (unsigned)f2bf(u[4]) | ((unsigned)f2bf(u[5]) << 16);
               o.w = (unsigned)f2bf(u[6]) | ((unsigned)f2bf(u[7]) << 16);
-              *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(outp) + voff[v]) = o;
+              *at16(outp, voff[v]) = o;
             }
           }
           if (wp) {
@@ -714,7 +722,7 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
                 wn[t] = __builtin_fmaf(-a.lrs, u[t], wv);
                 r[t] = __float_as_uint(wn[t]);
               }
-              u32x4_t* q = reinterpret_cast<u32x4_t*>(static_cast<float*>(wp) + voff[v]);
+              const auto q = at32(wp, voff[v]);
               q[0] = u32x4_t{r[0], r[1], r[2], r[3]};
               q[1] = u32x4_t{r[4], r[5], r[6], r[7]};
             } else {
@@ -727,20 +735,20 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
                 r[t] = f2bf(__builtin_fmaf(-a.lrs, u[t], wv));
                 wn[t] = bf2f(r[t]);
               }
-              *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(wp) + voff[v]) =
+              *at16(wp, voff[v]) =
                   u32x4_t{r[0] | (r[1] << 16), r[2] | (r[3] << 16), r[4] | (r[5] << 16),
                           r[6] | (r[7] << 16)};
             }
             if (pp) {
               // publish: the forward copy in its own dtype, same layout as W
               if (a.pub_dtype == DT_BF16) {
-                *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(pp) + voff[v]) =
+                *at16(pp, voff[v]) =
                     u32x4_t{(unsigned)f2bf(wn[0]) | ((unsigned)f2bf(wn[1]) << 16),
                             (unsigned)f2bf(wn[2]) | ((unsigned)f2bf(wn[3]) << 16),
                             (unsigned)f2bf(wn[4]) | ((unsigned)f2bf(wn[5]) << 16),
                             (unsigned)f2bf(wn[6]) | ((unsigned)f2bf(wn[7]) << 16)};
               } else {
-                u32x4_t* q = reinterpret_cast<u32x4_t*>(static_cast<float*>(pp) + voff[v]);
+                const auto q = at32(pp, voff[v]);
                 q[0] = u32x4_t{__float_as_uint(wn[0]), __float_as_uint(wn[1]),
                                __float_as_uint(wn[2]), __float_as_uint(wn[3])};
                 q[1] = u32x4_t{__float_as_uint(wn[4]), __float_as_uint(wn[5]),
@@ -749,7 +757,7 @@ __device__ __forceinline__ void nt_epilogue(const NtArgs& a, char* smem, const A
             }
           }
         } else {
-          // ragged edges and unaligned bases, one element at a time (kept rolled, re-reading U
+          // ragged edges, one element at a time (kept rolled, re-reading U
           // from the slab, so the unrolled slab loop around it stays small)
 #pragma unroll 1
           for (int t = 0; t < 8; ++t) {
