@@ -268,7 +268,15 @@ double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, b
     const std::pair<double, double> s = sides(q, t);
     return dims_t(s.first * s.second, m_of(q));
   });
-  return n_xx * tri_n + n_tri * tri_m + n_full * full + n_px * px;
+  bool small = gram && tile == kGramSmallSide;     // run_gram's one-workgroup form
+  double matrices = 0;
+  for (int i = 0; i < n; ++i) {
+    small = small && m_of(g[i]) <= kGramSmallSide;
+    matrices += g[i].batch;
+  }
+  const double squares = small ? 2 * (4.0 + 13.0 * ceil(matrices / num_cus))
+                               : n_tri * tri_m + n_full * full;
+  return n_xx * tri_n + squares + n_px * px;
 }
 
 // Tile, workspace and estimated time of several groups in one call. One group takes the tile
@@ -533,6 +541,15 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
   };
   int qs = -1;               // slot of the current Q, -1: none since the last (re)start
   if (gram()) return 1;
+  // Matrices of at most 128 rows: a segment's m x m products in one launch, one workgroup per
+  // matrix with everything in LDS (the same bits). All groups of the call, and segments of at
+  // most kGramSmallSteps steps.
+  bool small = c.tile == kGramSmallSide;
+  for (int i = 0; i < c.n; ++i) small = small && c.g[i].m_pad == kGramSmallSide;
+  for (int it = 0, end; small && it < T; it = end) {
+    for (end = it + 1; end < T && !is_restart(end);) ++end;
+    small = end - it <= kGramSmallSteps;
+  }
   for (int it = 0; it < T; ++it) {
     if (it != 0 && is_restart(it) && qs >= 0) {
       if (nt_product(c, PC_GEMM, gemm_flops,
@@ -542,6 +559,27 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
       for (int i = 0; i < c.n; ++i) c.g[i].rs = 1.f;
       if (gram()) return 1;
       qs = -1;
+    }
+    if (small) {
+      GramSmallArgs a;
+      a.n = c.n;
+      a.steps = updates_left(it);
+      for (int k = 0; k < 3 * a.steps; ++k) a.coeff[k] = coeffs[3 * it + k];
+      int matrices = 0;
+      double flops = 0.0;
+      for (int i = 0; i < c.n; ++i) {
+        Group& g = c.g[i];
+        a.g[i] = GramSmallGroup{g.w.Am, g.qslot[0], matrices, g.km, g.rs};
+        g.qbuf[0] = g.qslot[0];
+        matrices += g.batch;
+        flops += (3 * a.steps - 2) * poly_flops(g) + (a.steps - 1) * square_flops(g);
+      }
+      if (timed(PC_POLY, flops, 0.0, c.stream, c.who,
+                [&] { return launch_gram_small(a, matrices, c.stream); }))
+        return 1;
+      qs = 0;
+      it += a.steps - 1;
+      continue;
     }
     const float ca = coeffs[3 * it], cb = coeffs[3 * it + 1], cc = coeffs[3 * it + 2];
     const bool evolve = it + 1 < T && !is_restart(it + 1);

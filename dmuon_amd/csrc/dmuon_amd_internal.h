@@ -103,6 +103,22 @@ hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int ti
 // the device mapping, for tests: it must be a permutation of 0 .. nb - 1).
 int nt_block_tile(int b, int nb);
 
+// The m x m products of one Gram segment (`steps` NS steps from R on, `coeff` their (a, b, c)) for
+// matrices padded to 128 x 128, one workgroup per matrix: reads R (rs times R), writes Q. Rows and
+// columns from km (64 or 128) on are neither read nor written.
+constexpr int kGramSmallSteps = 16, kGramSmallSide = 128;
+struct GramSmallGroup {
+  const uint16_t* R; uint16_t* Q;         // fp16 [L][128][128]
+  int first, km;                          // first matrix of the group among the launch's
+  float rs;
+};
+struct GramSmallArgs {
+  int n, steps;
+  float coeff[3 * kGramSmallSteps];
+  GramSmallGroup g[kMaxGroups];
+};
+hipError_t launch_gram_small(const GramSmallArgs& a, int matrices, hipStream_t stream);
+
 // What one launch of the pre kernel does:
 //   PRE_BF16  momentum update, bf16 ns_in into Y / YT, norm partials (direct NS staging)
 //   PRE_NORM  momentum update and norm partials only
