@@ -75,7 +75,7 @@ struct Workspace {
   uint16_t *X, *X2, *Am, *Pm;
   // Gram backend only: the two slots of the accumulated polynomial Q (or its transpose), P R
   uint16_t *Q0, *Q1, *Wm;
-  float *partials, *scale, *scale_sq;
+  float *partials, *scale, *est_old;
   // correction of a copy staged with an estimated scale (1 when staged exactly), and the
   // per-matrix "stage again" flags
   float *ratio, *ratio_sq;
@@ -110,7 +110,7 @@ Workspace carve(char* base, int m_pad, int n_pad, int Rp, int Cp, int batch, int
   w.nparts = pre_blocks_per_mat(Rp, Cp);
   w.partials = reinterpret_cast<float*>(take(L * w.nparts * 4));
   w.scale = reinterpret_cast<float*>(take(L * 4));
-  w.scale_sq = reinterpret_cast<float*>(take(L * 4));
+  w.est_old = reinterpret_cast<float*>(take(L * 4));
   w.ratio = reinterpret_cast<float*>(take(L * 4));
   w.ratio_sq = reinterpret_cast<float*>(take(L * 4));
   w.restage = reinterpret_cast<int*>(take(L * 4));
@@ -637,7 +637,7 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
 int run_stage(const Call& c, float mu, int nesterov, float eps) {
   PreArgs p[2 * kMaxGroups];
   int np = 0;
-  bool est = false, exact = false;
+  bool est = false, exact = false, few_parts = true;
   double pre_bytes = 0.0, st_bytes = 0.0, norm_bytes = 0.0;
   NormArgs na[kMaxGroups];
   for (int i = 0; i < c.n; ++i) {
@@ -670,6 +670,9 @@ int run_stage(const Call& c, float mu, int nesterov, float eps) {
       q.kx = kNsKx;
       q.scale = g.w.scale + l0;
       q.restage = g.est_ptrs ? g.w.restage + l0 : nullptr;
+      q.est_old = g.w.est_old + l0;
+      q.norm_group = i;
+      q.norm_l0 = l0;
       // the NS products read X k-major, so only X is staged: by the direct write for a wide
       // orientation, by the transposed one for a tall orientation
       q.skip_y = tall_ ? 1 : 0;
@@ -684,8 +687,9 @@ int run_stage(const Call& c, float mu, int nesterov, float eps) {
                             (g.est_ptrs ? 2.0 : 0.0));
       if (!g.est_ptrs) st_bytes += elems * 2.0;
     }
-    na[i] = NormArgs{g.w.partials, g.w.nparts, g.batch, g.w.scale, g.w.scale_sq, g.est_ptrs,
+    na[i] = NormArgs{g.w.partials, g.w.nparts, g.batch, g.w.scale, g.w.est_old, g.est_ptrs,
                      g.w.ratio, g.w.ratio_sq, g.w.restage};
+    few_parts = few_parts && g.w.nparts <= kNormStageParts;
     norm_bytes += (double)g.batch * g.w.nparts * 4;
   }
   if (est && exact)
@@ -707,6 +711,12 @@ int run_stage(const Call& c, float mu, int nesterov, float eps) {
   if (timed(PC_PRE, 0.0, pre_bytes, c.stream, c.who,
             [&] { return launch_pre_batch(p, np, c.stream); }))
     return 1;
+  // small matrices: the norm and the exact staging in one launch
+  if (few_parts) {
+    stage(PRE_F16, false);
+    return timed(PC_NORM, 0.0, norm_bytes + st_bytes, c.stream, c.who,
+                 [&] { return launch_norm_stage(na, c.n, p, np, eps, c.stream); });
+  }
   if (timed(PC_NORM, 0.0, norm_bytes, c.stream, c.who,
             [&] { return launch_norm_finalize_est(na, c.n, eps, c.stream); }))
     return 1;

@@ -143,6 +143,10 @@ struct PreArgs {
   const int* restage;                     // PRE_F16: optional per-matrix "copy needed" flags
   // copies not written (the consumer reads the other one): skip_y -- Y, skip_yt -- YT
   int skip_y, skip_yt;
+  float* est_old;                         // PRE_EST: [L], the estimates as they were used
+  // launch_norm_stage: the norm group these matrices belong to, the first one's place in it
+  int norm_group, norm_l0;
+  int stage_blocks;                       // blocks per matrix, set by launch_norm_stage
 };
 hipError_t launch_pre(const PreArgs& a, hipStream_t stream);
 // The same stage over n (1 .. 2 kMaxGroups) sets of matrices: one launch per kernel that some of
@@ -160,14 +164,15 @@ int pre_blocks_per_mat(int Rp, int Cp);
 hipError_t launch_norm_finalize(const float* partials, int nparts, int L, float eps,
                                 float* scale, float* scale_sq, hipStream_t stream);
 
-// The same, plus the correction of a copy staged with an estimated scale: with est_ptrs and
-// est = *est_ptrs[l] > 0 and r = scale / est in [1/4, 4], ratio[l] = r, ratio_sq[l] = r^2 and
-// restage[l] = 0 (the staged copy times r is the exactly scaled one); otherwise ratio = 1,
-// ratio_sq = 1, restage = 1 (stage again with the exact scale). *est_ptrs[l] becomes scale.
+// The same for groups of matrices, plus the correction of a copy staged with an estimated scale:
+// with est_ptrs and est = est_old[l] > 0 (what PRE_EST staged with) and r = scale / est in
+// [1/4, 4], ratio[l] = r, ratio_sq[l] = r^2 and restage[l] = 0 (the staged copy times r is the
+// exactly scaled one); otherwise ratio = 1, ratio_sq = 1, restage = 1 (stage again with the exact
+// scale). *est_ptrs[l] becomes scale.
 // One launch for up to kMaxGroups groups of matrices.
 struct NormArgs {
   const float* partials; int nparts, L;
-  float* scale; float* scale_sq; float* const* est_ptrs;
+  float* scale; const float* est_old; float* const* est_ptrs;
   float* ratio; float* ratio_sq; int* restage;
 };
 struct NormBatch {
@@ -176,6 +181,11 @@ struct NormBatch {
   NormArgs a[kMaxGroups];
 };
 hipError_t launch_norm_finalize_est(const NormArgs* a, int n, float eps, hipStream_t stream);
+// The same with the PRE_F16 pass over the sets that need it, in one launch (restage[] is not
+// written): every block sums its matrix's partials, so only where those are few.
+constexpr int kNormStageParts = 4096;
+hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np, float eps,
+                             hipStream_t stream);
 
 // dst[l][r][c] = r < rows && c < cols ? src[l][r][c] : 0 over rows_out x cols_out (16-bit)
 // dst = src, n16 chunks of 16 bytes (both 16-byte aligned, not overlapping)

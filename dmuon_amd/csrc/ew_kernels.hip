@@ -69,6 +69,13 @@ __device__ __forceinline__ void stg_nt(V* p, V v) {
   __builtin_nontemporal_store(v, (__attribute__((address_space(1))) V*)p);
 }
 
+// The scale PRE_EST stages matrix l with; the matrix's first block leaves it for the norm.
+__device__ __forceinline__ float staged_scale(const PreArgs& a, int l, bool first) {
+  const float est = *a.est_ptrs[l];
+  if (first && threadIdx.x == 0) a.est_old[l] = est;
+  return est;
+}
+
 // Four values of a row whose pitch may be any number of elements: vector accesses that state the
 // element's own alignment (global memory takes them; a row of 3001 columns is never 8-byte
 // aligned).
@@ -86,9 +93,11 @@ __device__ __forceinline__ void stg_nt_any(float* p, f32x4_t v) {
 
 // One 64x64 tile (rows r0.., columns c0..) of matrix l; returns this thread's share of the
 // tile's sum of squares of ns_in. The caller synchronises before tileT is used again.
+// `scale`: the exact scale of PRE_F16, when the caller has it (otherwise a.scale[l]).
 template <int ST>
 __device__ __forceinline__ float pre_tile(const PreArgs& a, int l, int r0, int c0,
-                                          uint16_t (*tileT)[kTile + kPad]) {
+                                          uint16_t (*tileT)[kTile + kPad],
+                                          const float* scale = nullptr) {
   const int tid = threadIdx.x;
   const int tc = tid & 15, tr = tid >> 4;
 
@@ -100,8 +109,8 @@ __device__ __forceinline__ float pre_tile(const PreArgs& a, int l, int r0, int c
   // PRE_F16 reads the buffer PRE_NORM left (the new momentum) and only recomputes ns_in
   const bool read_buf = buf && (ST == PRE_F16 || !a.first_step);
   float sc = 1.f;
-  if constexpr (ST == PRE_F16) sc = a.scale[l] * a.kx;
-  if constexpr (ST == PRE_EST) sc = *a.est_ptrs[l] * a.kx;
+  if constexpr (ST == PRE_F16) sc = (scale ? *scale : a.scale[l]) * a.kx;
+  if constexpr (ST == PRE_EST) sc = staged_scale(a, l, r0 == 0 && c0 == 0) * a.kx;
   // PRE_EST without a usable estimate: momentum and partials only (the copy is staged later)
   const bool copy = ST != PRE_NORM && (ST != PRE_EST || sc > 0.f);
 
@@ -305,10 +314,10 @@ __device__ __forceinline__ void pre_unpack(const GradWords<GF>& t, const f32x4_t
 // Copy scale of this launch for matrix l (1 for PRE_BF16 / PRE_NORM), and whether it writes one
 // (PRE_EST without a usable estimate writes momentum and partials only).
 template <int ST>
-__device__ __forceinline__ float pre_scale(const PreArgs& a, int l, bool& copy) {
+__device__ __forceinline__ float pre_scale(const PreArgs& a, int l, bool first, bool& copy) {
   float sc = 1.f;
   if constexpr (ST == PRE_F16) sc = a.scale[l] * a.kx;
-  if constexpr (ST == PRE_EST) sc = *a.est_ptrs[l] * a.kx;
+  if constexpr (ST == PRE_EST) sc = staged_scale(a, l, first) * a.kx;
   copy = ST != PRE_NORM && (ST != PRE_EST || sc > 0.f);
   return sc;
 }
@@ -331,7 +340,7 @@ __global__ __launch_bounds__(256) void muon_pre_wide_kernel(const ARGS args) {
   float* buf = a.buf_ptrs ? a.buf_ptrs[l] : nullptr;
   const bool read_buf = buf && (ST == PRE_F16 || !a.first_step);
   bool copy;
-  const float sc = pre_scale<ST>(a, l, copy);
+  const float sc = pre_scale<ST>(a, l, blk == l * per, copy);
   const GradWords<GF> gw = pre_load_g<GF>(g, i);
   const f32x4_t bw = read_buf ? ldg_nt(reinterpret_cast<const f32x4_t*>(buf + i))
                               : f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -381,7 +390,7 @@ __global__ __launch_bounds__(256) void muon_pre_tall_kernel(const ARGS args) {
   float* buf = a.buf_ptrs ? a.buf_ptrs[l] : nullptr;
   const bool read_buf = buf && (ST == PRE_F16 || !a.first_step);
   bool copy;
-  const float sc = pre_scale<ST>(a, l, copy);
+  const float sc = pre_scale<ST>(a, l, blk == l * per, copy);
   float ss[TR / 16] = {0.f, 0.f, 0.f, 0.f};   // one per four rows of this wave
 #pragma unroll
   for (int rb = 0; rb < TR / 4; rb += RB) {
@@ -461,28 +470,48 @@ __global__ __launch_bounds__(256) void muon_restage_kernel(const ARGS args) {
   }
 }
 
-// Sum of matrix l's partials in fp64, in a fixed order (the same bits on every call): thread t
-// adds groups of four consecutive partials t, t + 1024, ..., then a tree over the 1024 threads.
-// One block per matrix; 1024 threads with four loads per step keep ~57K partials of a
-// 4096 x 14336 matrix from being a long chain of dependent load latencies. Result in red[0].
+// Sum of matrix l's partials in fp64, in a fixed order (the same bits on every call and from
+// every kernel): 1024 lanes, lane v adding groups of four consecutive partials v, v + 1024, ...,
+// then a tree over the lanes. A block of TH threads takes 1024 / TH lanes per thread. With 1024
+// threads and four loads per step ~57K partials of a 4096 x 14336 matrix are no long chain of
+// dependent load latencies. Result in red[0] (TH doubles).
 constexpr int kFinThreads = 1024;
+template <int TH>
 __device__ __forceinline__ void sum_partials(const float* partials, int nparts, int l,
                                              double* red) {
+  constexpr int V = kFinThreads / TH;
   const float* p = partials + (long long)l * nparts;
   const int t = threadIdx.x;
-  double s = 0.0;
+  double s[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) s[k] = 0.0;
   if ((nparts & 3) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
     const f32x4_t* p4 = reinterpret_cast<const f32x4_t*>(p);
-    for (int q = t; q < nparts / 4; q += kFinThreads) {
-      const f32x4_t v = p4[q];
-      s += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+    for (int q0 = 0; q0 < nparts / 4; q0 += kFinThreads) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const int q = q0 + k * TH + t;
+        if (q >= nparts / 4) continue;
+        const f32x4_t v = p4[q];
+        s[k] += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+      }
     }
   } else {
-    for (int q = t; q < nparts; q += kFinThreads) s += (double)p[q];
+    for (int q0 = 0; q0 < nparts; q0 += kFinThreads) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const int q = q0 + k * TH + t;
+        if (q < nparts) s[k] += (double)p[q];
+      }
+    }
   }
-  red[t] = s;
+#pragma unroll
+  for (int w = V / 2; w > 0; w >>= 1)
+#pragma unroll
+    for (int k = 0; k < w; ++k) s[k] += s[k + w];
+  red[t] = s[0];
   __syncthreads();
-  for (int w = kFinThreads / 2; w > 0; w >>= 1) {
+  for (int w = TH / 2; w > 0; w >>= 1) {
     if (t < w) red[t] += red[t + w];
     __syncthreads();
   }
@@ -494,7 +523,7 @@ __global__ __launch_bounds__(kFinThreads) void norm_finalize_kernel(const float*
                                                                     float* scale_sq) {
   __shared__ double red[kFinThreads];
   const int l = blockIdx.x;
-  sum_partials(partials, nparts, l, red);
+  sum_partials<kFinThreads>(partials, nparts, l, red);
   if (threadIdx.x == 0) {
     const float nrm = (float)sqrt(red[0]);
     const float sc = 1.0f / (nrm + eps);
@@ -524,6 +553,29 @@ __global__ __launch_bounds__(256) void muon_update_kernel(const UpdateArgs a) {
   }
 }
 
+__device__ __forceinline__ float norm_scale(double sumsq, float eps) {
+  return 1.0f / ((float)sqrt(sumsq) + eps);
+}
+// sc over the scale the copy was staged with, when that lies within [1/4, 4]; otherwise, or with
+// none, 0. PRE_EST left the staged scale in est_old (the kept one may be overwritten meanwhile).
+__device__ __forceinline__ float norm_ratio(const NormArgs& a, int l, float sc) {
+  if (!a.est_ptrs) return 0.f;
+  const float est = a.est_old[l];
+  if (!(est > 0.f)) return 0.f;
+  const float r = sc / est;
+  return r >= 0.25f && r <= 4.f ? r : 0.f;         // 0 for NaN / inf too
+}
+__device__ __forceinline__ void norm_outputs(const NormArgs& a, int l, double sumsq, float eps,
+                                             bool flag) {
+  const float sc = norm_scale(sumsq, eps);
+  a.scale[l] = sc;
+  const float r = norm_ratio(a, l, sc);
+  if (a.est_ptrs) *a.est_ptrs[l] = sc;
+  a.ratio[l] = r > 0.f ? r : 1.f;
+  a.ratio_sq[l] = r > 0.f ? r * r : 1.f;
+  if (flag) a.restage[l] = r > 0.f ? 0 : 1;
+}
+
 __global__ __launch_bounds__(kFinThreads) void norm_finalize_est_kernel(const NormBatch b,
                                                                         float eps) {
   __shared__ double red[kFinThreads];
@@ -532,26 +584,34 @@ __global__ __launch_bounds__(kFinThreads) void norm_finalize_est_kernel(const No
   g = __builtin_amdgcn_readfirstlane(g);
   const NormArgs& a = b.a[g];
   const int l = blockIdx.x - b.first[g];
-  sum_partials(a.partials, a.nparts, l, red);
-  if (threadIdx.x == 0) {
-    const float nrm = (float)sqrt(red[0]);
-    const float sc = 1.0f / (nrm + eps);
-    a.scale[l] = sc;
-    a.scale_sq[l] = sc * sc;
-    float r = 1.f;
-    bool ok = false;
-    if (a.est_ptrs) {
-      const float est = *a.est_ptrs[l];
-      if (est > 0.f) {
-        r = sc / est;
-        ok = r >= 0.25f && r <= 4.f;   // false for NaN / inf too
-      }
-      *a.est_ptrs[l] = sc;
-    }
-    if (!ok) r = 1.f;
-    a.ratio[l] = r;
-    a.ratio_sq[l] = r * r;
-    a.restage[l] = ok ? 0 : 1;
+  sum_partials<kFinThreads>(a.partials, a.nparts, l, red);
+  if (threadIdx.x == 0) norm_outputs(a, l, red[0], eps, true);
+}
+
+// Norm and exact staging of small matrices in one launch: every block of a matrix sums its (few)
+// partials itself, the first one writes the outputs, and the matrix's blocks stage its tiles if
+// its kept scale does not do (or there is none). One launch less on every step of a small model
+// (twelve 512x2048 matrices 293.1 -> 290.3 us, one 1024x1024 155.1 -> 154.0, ragged ones 258.4 ->
+// 255.1, one 128x512 Newton-Schulz 67.3 -> 65.8).
+template <class ARGS>
+__global__ __launch_bounds__(256) void norm_stage_kernel(const NormBatch b, const ARGS args,
+                                                         float eps) {
+  __shared__ double red[256];
+  __shared__ __attribute__((aligned(16))) uint16_t tileT[kTile][kTile + kPad];
+  unsigned blk;
+  const PreArgs& p = block_args(args, blk);
+  const int per_mat = p.stage_blocks, ls = blk / per_mat, first = blk - ls * per_mat;
+  const NormArgs& a = b.a[p.norm_group];
+  const int l = ls + p.norm_l0;                    // the set's matrix among the group's
+  sum_partials<256>(a.partials, a.nparts, l, red);
+  const float sc = norm_scale(red[0], eps);
+  const bool ok = norm_ratio(a, l, sc) > 0.f;
+  if (first == 0 && threadIdx.x == 0) norm_outputs(a, l, red[0], eps, false);
+  if (ok) return;                                  // block-uniform
+  const int tx = p.Cp / kTile, per = tx * (p.Rp / kTile);
+  for (int t = first; t < per; t += per_mat) {
+    __syncthreads();   // the previous tile's transposed read of tileT is done
+    pre_tile<PRE_F16>(p, ls, (t / tx) * kTile, (t % tx) * kTile, tileT, &sc);
   }
 }
 
@@ -714,6 +774,49 @@ hipError_t launch_pre_batch(const PreArgs* a, int n, hipStream_t stream) {
 }
 
 hipError_t launch_pre(const PreArgs& a, hipStream_t stream) { return launch_pre_batch(&a, 1, stream); }
+
+hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np, float eps,
+                             hipStream_t stream) {
+  if (n < 1 || n > kMaxGroups || np < 1 || np > 2 * kMaxGroups) return hipErrorInvalidValue;
+  NormBatch b;
+  b.n = n;
+  long long matrices = 0;
+  for (int g = 0; g < n; ++g) {
+    b.a[g] = a[g];
+    matrices += a[g].L;
+  }
+  PreBatch q;
+  q.n = 0;
+  long long blocks = 0;
+  for (int i = 0; i < np; ++i) {
+    if (p[i].L <= 0) continue;
+    if (p[i].norm_group < 0 || p[i].norm_group >= n || p[i].norm_l0 < 0 ||
+        p[i].norm_l0 + p[i].L > a[p[i].norm_group].L)
+      return hipErrorInvalidValue;
+    PreArgs& s = q.a[q.n];
+    s = p[i];
+    s.restage = nullptr;
+    // Staged again only now and then: 2048 blocks over the call's matrices (8 at least each), of
+    // which the usual step runs the sums only. Without kept scales every tile has its block.
+    const long long tiles = (long long)(s.Rp / kTile) * (s.Cp / kTile);
+    const long long few = std::max(8LL, 2048 / matrices);
+    s.stage_blocks = (int)(a[s.norm_group].est_ptrs ? std::min(tiles, few) : tiles);
+    q.first[q.n++] = (unsigned)blocks;
+    blocks += (long long)s.stage_blocks * s.L;
+  }
+  if (blocks == 0) return hipSuccess;
+  if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (sizeof(NormBatch) + sizeof(PreBatch) + 64 > 4096 || q.n == 1) {
+    for (int i = 0; i < q.n; ++i)
+      hipLaunchKernelGGL(norm_stage_kernel<PreArgs>,
+                         dim3((unsigned)((long long)q.a[i].stage_blocks * q.a[i].L)), dim3(256), 0,
+                         stream, b, q.a[i], eps);
+  } else {
+    hipLaunchKernelGGL(norm_stage_kernel<PreBatch>, dim3((unsigned)blocks), dim3(256), 0, stream,
+                       b, q, eps);
+  }
+  return hipGetLastError();
+}
 
 hipError_t launch_norm_finalize_est(const NormArgs* a, int n, float eps, hipStream_t stream) {
   if (n < 1 || n > kMaxGroups) return hipErrorInvalidValue;
