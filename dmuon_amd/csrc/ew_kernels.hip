@@ -796,10 +796,10 @@ hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np,
     PreArgs& s = q.a[q.n];
     s = p[i];
     s.restage = nullptr;
-    // Staged again only now and then: 2048 blocks over the call's matrices (8 at least each), of
+    // Staged again only now and then: 1024 blocks over the call's matrices (8 at least each), of
     // which the usual step runs the sums only. Without kept scales every tile has its block.
     const long long tiles = (long long)(s.Rp / kTile) * (s.Cp / kTile);
-    const long long few = std::max(8LL, 2048 / matrices);
+    const long long few = std::max(8LL, 1024 / matrices);
     s.stage_blocks = (int)(a[s.norm_group].est_ptrs ? std::min(tiles, few) : tiles);
     q.first[q.n++] = (unsigned)blocks;
     blocks += (long long)s.stage_blocks * s.L;

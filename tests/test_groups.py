@@ -70,6 +70,8 @@ CASES = [
     ([(256, 768, 3, 1), (300, 1000, 2, 1), (512, 512, 2, 0), (128, 128, 1, 0), (64, 640, 1, 0)], 128),
     ([(512, 2048, 12, 4), (1024, 1024, 3, 0), (384, 640, 4, 4), (130, 250, 2, 1), (64, 64, 1, 0)], 128),
     ([(512, 768, 2, 1), (256, 1024, 2, 1), (700, 500, 1, 0), (300, 300, 1, 0), (256, 256, 3, 0)], 256),
+    # one matrix with more partial sums than the joined norm and staging launch takes
+    ([(256, 768, 3, 1), (2048, 2112, 1, 0)], 128),
 ]
 
 
