@@ -591,8 +591,8 @@ __global__ __launch_bounds__(kFinThreads) void norm_finalize_est_kernel(const No
 // Norm and exact staging of small matrices in one launch: every block of a matrix sums its (few)
 // partials itself, the first one writes the outputs, and the matrix's blocks stage its tiles if
 // its kept scale does not do (or there is none). One launch less on every step of a small model
-// (twelve 512x2048 matrices 293.1 -> 290.3 us, one 1024x1024 155.1 -> 154.0, ragged ones 258.4 ->
-// 255.1, one 128x512 Newton-Schulz 67.3 -> 65.8).
+// (twelve 512x2048 matrices 301.3 -> 298.2 us, one 1024x1024 155.3 -> 154.2, ragged ones 258.8 ->
+// 255.2, one 128x512 Newton-Schulz 66.6 -> 65.9; both sides in turn on one card).
 template <class ARGS>
 __global__ __launch_bounds__(256) void norm_stage_kernel(const NormBatch b, const ARGS args,
                                                          float eps) {
