@@ -215,7 +215,8 @@ int plan(int rows, int cols, int batch, int tile_req, int num_cus, int gram, int
 // is fixed + slices of K (64 wide) at its kernel's rate, measured on MI355X as K sweeps (64 ..
 // 8192) of triangle products with 36 .. 1020 tiles: 256-tiles 13 us + 1.0 per slice on a third of
 // the CUs and 1.4 on all of them, 128-tiles one per CU 6 + 0.39 .. 0.46, two per CU 8 + 0.93 for
-// the pair, 64-tiles 5 + 0.18. Only the comparison of two splits matters.
+// the pair, 64-tiles 5 + 0.18 (two of them per CU take 1 .. 2 us less than the 128-tiles one per CU
+// that stand for them here). Only the comparison of two splits matters.
 double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, bool gram) {
   // launches of one NS run of five steps: X X^T, m x m triangle products, Q updates, P X
   const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_full = gram ? 3 : 0,

@@ -19,7 +19,7 @@
 //   128x128 tiles (nt_mfma_kernel): 4 waves of 64x64, two blocks per CU, for batches too small
 //     to fill the machine with 256-tiles; fragments double-buffered per substep, one barrier
 //     per slice. Per launch (launch_nt), a 128-tile product that leaves CUs idle runs on 64x64
-//     tiles (4 waves, eight-slot ring) or on 8 waves with a four-slot ring, one block per CU,
+//     tiles (4 waves, eight-slot ring; four slots two per CU) or on 8 waves with a four-slot ring,
 //     and one with more than two 128-tiles per CU may take 256-tiles: such small launches wait
 //     on load latency, not bandwidth. Tile size, waves and ring depth change where operands
 //     wait, not the arithmetic, so every variant gives the same bits.
@@ -1395,13 +1395,14 @@ void launch_pp(const ARGS& p, int mode, bool kmajor, long long nb, hipStream_t s
 }
 
 // Which kernel runs a launch of a 128- or 256-tile plan.
-enum NtKernel { NT_PP256, NT_128, NT_128_DEEP, NT_64 };
+enum NtKernel { NT_PP256, NT_128, NT_128_DEEP, NT_64, NT_64_PAIR };
 
 template <int E, class ARGS>
 void launch_kernel(NtKernel k, const ARGS& p, int mode, bool kmajor, long long nb,
                    hipStream_t stream) {
   if (k == NT_PP256) launch_pp<E>(p, mode, kmajor, nb, stream);
   else if (k == NT_64) launch_mfma<64, kT64S, 1, kT64WN, E>(p, mode, kmajor, nb, stream);
+  else if (k == NT_64_PAIR) launch_mfma<64, kT64S / 2, 1, kT64WN, E>(p, mode, kmajor, nb, stream);
   else if (k == NT_128_DEEP) launch_mfma<128, kT128S, 2, kT128WN, E>(p, mode, kmajor, nb, stream);
   else launch_mfma<128, 2, 2, 2, E>(p, mode, kmajor, nb, stream);
 }
@@ -1425,6 +1426,15 @@ void launch_kernel(NtKernel k, const ARGS& p, int mode, bool kmajor, long long n
 //    waits on load latency. Every value keeps its K order -- the slice rotation depends only on
 //    the 256-aligned block of the tile's columns. A k-major B is one 64-value block of 128-byte
 //    k-rows per slice;
+//  - 64-tiles two per CU, each with half that ring (64 KiB), while they fit one wave of such
+//    blocks and B is not k-major: one block's waits run under the other's work. Against the
+//    128-tiles one per CU that ran them before, launch to launch, with 264 .. 512 64-tiles:
+//    512 x 512 triangles of 12 matrices 6.2 -> 5.4 us at K = 64, 8.7 -> 7.5 at 512, 11.6 -> 9.9
+//    at 1024, 30.3 -> 27.9 at 4096; no K and no count in that range lost. Past two per CU a
+//    second wave begins, and three per CU were slower. A k-major B stays on the 128-tiles: its
+//    X was written by the launch before and 64-tiles read it twice as often, so that inside a
+//    step 8 products of 384 x 576 took 7.7 us on 128-tiles and 8.6 in pairs (8.2 and 7.4 where
+//    one launch repeats on operands the caches hold);
 //  - else 128-tiles.
 namespace {
 
@@ -1473,6 +1483,7 @@ NtChoice choose_kernel(const NtArgs* const* a, int cnt, int tile) {
     const double c128 = 2.7 * (double)((nb + 2LL * cus - 1) / (2LL * cus));
     if (!a[0]->edge && split256 && nb > 2LL * cus && c256 < c128) return {NT_PP256, 256, nb256, cus};
     if (nb64 <= cus) return {NT_64, 64, nb64, cus};
+    if (nb64 <= 2LL * cus && !a[0]->b_kmajor) return {NT_64_PAIR, 64, nb64, 2LL * cus};
     if (nb <= cus) return {NT_128_DEEP, 128, nb, cus};
   }
   return {NT_128, 128, nb, 2LL * cus};
@@ -1495,7 +1506,7 @@ hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int ti
   if ((cnt > 1 || fill) && a[0].elt != ELT_F16) return hipErrorInvalidValue;
   // an edge product runs on the 128- and 64-tile kernels only
   if (a[0].edge && (cnt > 1 || fill || tile != 128)) return hipErrorInvalidValue;
-  const NtChoice k = choose_kernel(list, cnt, tile);
+  NtChoice k = choose_kernel(list, cnt, tile);
   long long nb = k.nb;
   NtBatch b;
   b.n = 0;
@@ -1537,6 +1548,10 @@ hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int ti
       before += whole;
     }
     if (all && fill->next < before) return hipErrorInvalidValue;
+    // the last tiles of a fill may take a launch of 64-tiles past one per CU: the same rule again
+    // (a Newton-Schulz of eight 384 x 398: 144.9 us before pairs, 147.1 without this line, 144.5)
+    if (k.kernel == NT_64 && nb > k.slots && nb <= 2 * k.slots && !a[0].b_kmajor)
+      k.kernel = NT_64_PAIR;
   }
   const int mode = a[0].mode;
   const bool km = a[0].b_kmajor != 0;
