@@ -112,7 +112,8 @@ int dmuon_stream_copy(const void* src, void* dst, int64_t bytes, void* stream);
  * better, with the same bits as the 128-tile kernel.
  * Any M >= 0 and K >= 0 are accepted. When M is a multiple of the tile, K of 64, and every base
  * is 16-byte aligned with leading dimensions and batch strides that are multiples of 8, the
- * kernel reads the operands in place and `workspace` may be NULL; otherwise the call runs on
+ * kernel reads the operands in place and `workspace` may be NULL; so it does, so aligned, when M
+ * and K are only multiples of 8 and a 128-tile plan has at most 512 tiles; otherwise the call runs on
  * zero-padded copies in `workspace` (device memory of dmuon_syrk_workspace_size bytes, at least
  * 16-byte aligned; contents need no initialisation) and copies the M x M result into D.
  */
