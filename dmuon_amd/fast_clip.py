@@ -22,6 +22,7 @@ stays rank-uniform.
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 from collections import OrderedDict
 from dataclasses import dataclass
@@ -188,7 +189,11 @@ class _JobTable:
                 base + 4 * (k + 1), base + at, base + at + k, ws.data_ptr(), need,
                 self._stream())
         floats, flags = out[:at].view(torch.float32), out[at:].view(torch.bool)
-        return floats[:k + 1], floats[k + 1:], flags[:k], flags[k:]
+        norms, coefs = floats[:k + 1], floats[k + 1:]
+        if max_norm is not None and math.isnan(max_norm):
+            # NaN is the entry point's "no limit"; as a caller's limit it is min(nan / norm, 1)
+            coefs.fill_(max_norm)
+        return norms, coefs, flags[:k], flags[k:]
 
     def scale(self, coefs: torch.Tensor, segments=None) -> None:
         _C.call("dmuon_segmented_scale", self.ptrs, self.numels, self.dtypes,

@@ -5,6 +5,7 @@ import math
 import pytest
 import torch
 
+import dmuon_amd as dmuon
 from dmuon_amd import _C, fast_clip
 from dmuon_amd.fast_clip import GradClipBucket, clip_grad_norm_buckets_
 
@@ -81,3 +82,30 @@ def test_one_norm_over_all_rounds_each_to_its_dtype(gpu, bad):
     assert not math.isfinite(float(norms[0])) and bool(found[0]) and not bool(clipped[0])
     want = 0.0 if bad == float("inf") else bad
     assert float(coefs[0]) == want or math.isnan(want) and math.isnan(float(coefs[0]))
+
+
+@pytest.mark.gpu
+def test_a_nan_limit_is_a_limit(gpu):
+    """max_norm=nan gives NaN coefficients and gradients, as min(nan / norm, 1) does; only None is
+    no limit."""
+    nan = float("nan")
+    for dt in DT:
+        grads = _grads([33, 9000], [dt, dt], gpu, 5)
+        norms = [float(g.double().norm()) for g in grads]
+        buckets = tuple(GradClipBucket(str(i), [g], reduce=False) for i, g in enumerate(grads))
+        res = clip_grad_norm_buckets_(buckets, nan)
+        for s, g, n in zip(res.bucket_stats, grads, norms):
+            assert math.isnan(float(s.clip_coef)) and not bool(s.clipped)
+            assert float(s.total_norm) == pytest.approx(n, rel=1e-6) and not bool(s.found_inf)
+            assert g.isnan().all()
+        grads = _grads([33, 9000], [dt, dt], gpu, 6)
+        model = torch.nn.Module()
+        model.mats = torch.nn.ParameterList(
+            [torch.nn.Parameter(torch.zeros(g.numel() // 3, 3, dtype=dt, device=gpu)) for g in grads])
+        dmuon.dedicate_params(model, None, lambda name, p: True)
+        dmuon.replicate(model)
+        for p, g in zip(model.mats, grads):
+            p.grad = g.view(p.shape)
+        stats = dmuon.Muon(model).clip_grad_norm_(nan)
+        assert math.isnan(float(stats.clip_coef)) and not bool(stats.clipped)
+        assert all(g.isnan().all() for g in grads)
