@@ -150,6 +150,27 @@ class _JobTable:
         self.device = device
         self._dtypes = [g.dtype for g in tensors]
         self._dtype_groups = None
+        self._uploaded, self._on_device = torch.cuda.Event(), ()
+        self._note_upload(self._d64, self._d32)
+
+    def _note_upload(self, *tensors) -> None:
+        stream = torch.cuda.current_stream(self.device)
+        if not torch.cuda.is_current_stream_capturing():
+            self._uploaded.record(stream)
+        self._streams = {stream.cuda_stream}        # those that come after the last upload
+        self._on_device += tensors
+
+    def order_on_current_stream(self) -> None:
+        """Lets the current stream read a table that another stream's work uploaded: it waits for
+        the upload, and an evicted table's memory waits for what it has enqueued. (A graph
+        capture begins with the device synchronised, and may not wait for work outside it.)"""
+        stream = torch.cuda.current_stream(self.device)
+        if stream.cuda_stream in self._streams or torch.cuda.is_current_stream_capturing():
+            return
+        stream.wait_event(self._uploaded)
+        for t in self._on_device:
+            t.record_stream(stream)
+        self._streams.add(stream.cuda_stream)
 
     def dtype_groups(self):
         """(dtype, device index tensor of the table's tensors of that dtype, or None when all
@@ -162,6 +183,9 @@ class _JobTable:
                     self.device, non_blocking=True)
                 groups.append((dt, idx))
             self._dtype_groups = groups
+            indexes = [idx for _, idx in groups if idx is not None]
+            if indexes:
+                self._note_upload(*indexes)
         return self._dtype_groups
 
     def _stream(self):
@@ -221,6 +245,7 @@ def _job_table(tensors, segments, device, chunk) -> _JobTable:
             _TABLE_CACHE.popitem(last=False)
     else:
         _TABLE_CACHE.move_to_end(key)
+        table.order_on_current_stream()
     return table
 
 

@@ -1,6 +1,7 @@
 """``dmuon_clip_norms``: norms, coefficients and flags of a job table in two launches."""
 import ctypes
 import math
+import time
 
 import pytest
 import torch
@@ -109,3 +110,30 @@ def test_a_nan_limit_is_a_limit(gpu):
         stats = dmuon.Muon(model).clip_grad_norm_(nan)
         assert math.isnan(float(stats.clip_coef)) and not bool(stats.clipped)
         assert all(g.isnan().all() for g in grads)
+
+
+@pytest.mark.gpu
+def test_a_cached_table_waits_for_its_upload_on_another_stream(gpu):
+    """The device table is uploaded in the order of the stream that built it: a later call on
+    another stream waits for that before its kernels read the table."""
+    grads = _grads([33, 9000], [torch.float32, torch.bfloat16], gpu, 9)
+    # no earlier work is left to wait for, and the first upload's own allocations exist
+    fast_clip._job_table(grads[:1], [0], gpu, 4096)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(200_000_000)                # about 0.1 s
+        table = fast_clip._job_table(grads, [0, 1], gpu, 4096)
+    with torch.cuda.stream(b):
+        assert fast_clip._job_table(grads, [0, 1], gpu, 4096) is table
+        reached = torch.cuda.Event()
+        reached.record()
+    time.sleep(0.01)                                  # an event with nothing before it is done
+    waits, asleep = not reached.query(), not a.query()
+    torch.cuda.synchronize()
+    assert asleep and waits
+    with torch.cuda.stream(b):                         # now there is nothing to wait for
+        fast_clip._job_table(grads, [0, 1], gpu, 4096)
+        norms = table.norms(2, None)[0]
+    for n, g in zip(norms.tolist(), grads):
+        assert n == pytest.approx(float(g.double().norm()), rel=1e-6)
