@@ -987,7 +987,7 @@ int syrk_plan(const char* who, const void* A, int64_t lda, int64_t strideA, cons
   if (C) off += align256(xd);
   pl->offD = off;
   off += align256(xd);
-  pl->bytes = pl->direct ? 0 : off;
+  pl->bytes = pl->direct || pl->edge ? 0 : off;
   return 0;
 }
 

@@ -75,3 +75,22 @@ def test_what_needs_copies_still_asks_for_a_workspace():
     need = ctypes.c_int64()
     assert lib.dmuon_syrk_workspace_size(_C.DTYPE_F16, p, 3000, 0, None, 0, 0, None, 0, 0, 1 << 30,
                                          1000, 0, 1000, 3000, 1, 0, ctypes.byref(need)) == 0
+
+
+def _need(M, K, L=1, a=1 << 24, c=None, d=1 << 30, lda=0, ldd=0, b=None):
+    lib, need = _C.lib(), ctypes.c_int64(-1)
+    lda, ldd = lda or K, ldd or M
+    assert lib.dmuon_syrk_workspace_size(
+        _C.DTYPE_F16, a, lda, M * lda, b, 0 if b is None else lda, 0 if b is None else M * lda, c,
+        0 if c is None else M, 0 if c is None else M * M, d, ldd, M * ldd, M, K, L, 0,
+        ctypes.byref(need)) == 0, lib.dmuon_last_error()
+    return need.value
+
+
+def test_operands_used_in_place_ask_for_no_workspace():
+    assert _need(1024, 3072) == 0                                # whole tiles
+    for M, K, L in CASES:
+        if M % 128 or K % 64:
+            assert _need(M, K, L) == 0 and _need(M, K, L, c=1 << 28) == 0, (M, K, L)
+    # padded copies of A (1024 x 3008) and D
+    assert _need(1001, 3000) == 2 * (1024 * 3008 + 1024 * 1024)
