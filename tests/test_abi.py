@@ -247,9 +247,10 @@ def test_syrk_any_shape_workspace_plan_without_gpu():
         return -(-x // 256) * 256
 
     assert ws(512, 1024) == 0 and ws(1408, 2048) == 0
-    assert ws(1000, 3000) == al(1024 * 3008 * 2) + al(1024 * 1024 * 2)
-    assert ws(1000, 3000, c=1 << 24) == al(1024 * 3008 * 2) + 2 * al(1024 * 1024 * 2)
-    assert ws(1000, 3000, b=1 << 26, ldb=3000) == 2 * al(1024 * 3008 * 2) + al(1024 * 1024 * 2)
+    assert ws(1000, 3000) == 0                           # ragged in whole 16-byte chunks
+    assert ws(1001, 3000) == al(1024 * 3008 * 2) + al(1024 * 1024 * 2)
+    assert ws(1001, 3000, c=1 << 24) == al(1024 * 3008 * 2) + 2 * al(1024 * 1024 * 2)
+    assert ws(1001, 3000, b=1 << 26, ldb=3000) == 2 * al(1024 * 3008 * 2) + al(1024 * 1024 * 2)
     assert ws(512, 1024, lda=1025) > 0                   # rows not 16-byte aligned
     assert ws(512, 1024, a=(1 << 20) + 2) > 0            # base not 16-byte aligned
     assert ws(384, 640, L=3, tile=256) == 3 * 512 * 640 * 2 + al(3 * 512 * 512 * 2)
