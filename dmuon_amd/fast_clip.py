@@ -160,12 +160,11 @@ class _JobTable:
         self._streams = {stream.cuda_stream}        # those that come after the last upload
         self._on_device += tensors
 
-    def order_on_current_stream(self) -> None:
-        """Lets the current stream read a table that another stream's work uploaded: it waits for
-        the upload, and an evicted table's memory waits for what it has enqueued. (A graph
-        capture begins with the device synchronised, and may not wait for work outside it.)"""
-        stream = torch.cuda.current_stream(self.device)
-        if stream.cuda_stream in self._streams or torch.cuda.is_current_stream_capturing():
+    def _order(self, stream) -> None:
+        """Lets ``stream`` read a table that another stream's work uploaded: it waits for the
+        upload, and an evicted table's memory waits for what it has enqueued. (A graph capture
+        begins with the device synchronised, and may not wait for work outside it.)"""
+        if torch.cuda.is_current_stream_capturing():
             return
         stream.wait_event(self._uploaded)
         for t in self._on_device:
@@ -188,8 +187,13 @@ class _JobTable:
                 self._note_upload(*indexes)
         return self._dtype_groups
 
-    def _stream(self):
-        return torch.cuda.current_stream(self.device).cuda_stream
+    def _stream(self) -> int:
+        """The current stream's handle, for a launch that reads the table."""
+        stream = torch.cuda.current_stream(self.device)
+        handle = stream.cuda_stream
+        if handle not in self._streams:
+            self._order(stream)
+        return handle
 
     def sumsq(self, local_sq: torch.Tensor, segments=None) -> None:
         _C.call("dmuon_segmented_l2_norm_sq", self.ptrs, self.numels, self.dtypes,
@@ -245,7 +249,6 @@ def _job_table(tensors, segments, device, chunk) -> _JobTable:
             _TABLE_CACHE.popitem(last=False)
     else:
         _TABLE_CACHE.move_to_end(key)
-        table.order_on_current_stream()
     return table
 
 

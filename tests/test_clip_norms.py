@@ -126,6 +126,7 @@ def test_a_cached_table_waits_for_its_upload_on_another_stream(gpu):
         table = fast_clip._job_table(grads, [0, 1], gpu, 4096)
     with torch.cuda.stream(b):
         assert fast_clip._job_table(grads, [0, 1], gpu, 4096) is table
+        assert table._stream() == b.cuda_stream        # what each of its kernels is launched on
         reached = torch.cuda.Event()
         reached.record()
     time.sleep(0.01)                                  # an event with nothing before it is done
@@ -133,7 +134,6 @@ def test_a_cached_table_waits_for_its_upload_on_another_stream(gpu):
     torch.cuda.synchronize()
     assert asleep and waits
     with torch.cuda.stream(b):                         # now there is nothing to wait for
-        fast_clip._job_table(grads, [0, 1], gpu, 4096)
         norms = table.norms(2, None)[0]
     for n, g in zip(norms.tolist(), grads):
         assert n == pytest.approx(float(g.double().norm()), rel=1e-6)
