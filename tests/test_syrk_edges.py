@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from dmuon_amd import _C
+from dmuon_amd.optim.syrk_dispatch import syrk_or_cublas
 
 # sides around the 8-value chunk, the 64-wide slice and the 64- and 128-tiles; a batch that runs
 # on each of the 64-tile and the two 128-tile kernels
@@ -94,3 +95,38 @@ def test_operands_used_in_place_ask_for_no_workspace():
             assert _need(M, K, L) == 0 and _need(M, K, L, c=1 << 28) == 0, (M, K, L)
     # padded copies of A (1024 x 3008) and D
     assert _need(1001, 3000) == 2 * (1024 * 3008 + 1024 * 1024)
+
+
+def test_a_result_inside_the_operands_memory_takes_the_copies():
+    """In place, a block may store D before another has read its operands: memory they share (also
+    with no value in common) keeps the padded copies, whose result is stored last."""
+    M, K = 200, 328
+    a = 1 << 24
+    end = a + 2 * M * K
+    copies = 2 * (256 * 384 + 256 * 256)
+    assert _need(M, K, a=a, d=end) == 0                              # D right behind A
+    assert _need(M, K, a=a, d=end - 16) == copies
+    assert _need(M, K, a=a, d=a - 2 * M * M + 16) == copies
+    assert _need(M, K, a=a, d=a - 2 * M * M) == 0
+    assert _need(M, K, a=a, d=a + 2 * K, lda=K + M, ldd=K + M) == copies   # columns of one tensor
+    c = 1 << 28
+    assert _need(M, K, c=c, d=c + 2 * M * M) == 0 and _need(M, K, c=c, d=c + 16) > copies
+    assert _need(M, K, L=3, b=1 << 29, d=(1 << 29) + 2 * 2 * M * K + 16) > 3 * copies
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("over", ["A", "C"])
+def test_a_result_over_its_operands(gpu, over):
+    M, K, L = 200, 328, 2
+    gen = torch.Generator(device=gpu).manual_seed(4)
+    A = (torch.randn(L, M, K, device=gpu, generator=gen) * 0.1).to(torch.float16)
+    C = torch.randn(L, M, M, device=gpu, generator=gen).to(torch.float16)
+    C = (C.float() + C.float().transpose(1, 2).contiguous()).to(torch.float16)
+    want = torch.empty_like(C)
+    syrk_or_cublas(A, want, C=C, alpha=0.5, beta=0.25)
+    flat = torch.zeros(8 + L * M * K, dtype=torch.float16, device=gpu)
+    src = A if over == "A" else C
+    x, d = flat[:src.numel()].view_as(src), flat[8:8 + L * M * M].view(L, M, M)
+    x.copy_(src)
+    syrk_or_cublas(x if over == "A" else A, d, C=C if over == "A" else x, alpha=0.5, beta=0.25)
+    assert torch.equal(d, want)
