@@ -934,6 +934,17 @@ struct SyrkPlan {
   int64_t offB, offC, offD, bytes;
 };
 
+// Whether two batches of matrices in row pitch ld and batch stride share any byte of the ranges
+// they span.
+bool spans_overlap(const void* a, int64_t lda, int64_t sa, int cols_a, const void* b, int64_t ldb,
+                   int64_t sb, int cols_b, int rows, int batch) {
+  auto last = [&](int64_t ld, int64_t s, int cols) {
+    return 2 * ((batch > 1 ? (batch - 1) * s : 0) + (rows - 1) * ld + cols);
+  };
+  const intptr_t x = reinterpret_cast<intptr_t>(a), y = reinterpret_cast<intptr_t>(b);
+  return x < y + last(ldb, sb, cols_b) && y < x + last(lda, sa, cols_a);
+}
+
 int syrk_plan(const char* who, const void* A, int64_t lda, int64_t strideA, const void* B,
               int64_t ldb, int64_t strideB, const void* C, int64_t ldc, int64_t strideC,
               const void* D, int64_t ldd, int64_t strideD, int M, int K, int batch, int tile_req,
@@ -957,17 +968,6 @@ int syrk_plan(const char* who, const void* A, int64_t lda, int64_t strideA, cons
   if (t == 0) {
     t = auto_tile(M, K > 0 ? K : 1, batch, 256);
     if (t == 256 && round_up(M, 256) != round_up(M, 128)) t = 128;   // no padded copy for 256
-// Whether two batches of matrices in row pitch ld and batch stride share any byte of the ranges
-// they span.
-bool spans_overlap(const void* a, int64_t lda, int64_t sa, int cols_a, const void* b, int64_t ldb,
-                   int64_t sb, int cols_b, int rows, int batch) {
-  auto last = [&](int64_t ld, int64_t s, int cols) {
-    return 2 * ((batch > 1 ? (batch - 1) * s : 0) + (rows - 1) * ld + cols);
-  };
-  const intptr_t x = reinterpret_cast<intptr_t>(a), y = reinterpret_cast<intptr_t>(b);
-  return x < y + last(ldb, sb, cols_b) && y < x + last(lda, sa, cols_a);
-}
-
   }
   pl->tile = t;
   pl->Mp = (int)round_up(M, t);
@@ -990,6 +990,11 @@ bool spans_overlap(const void* a, int64_t lda, int64_t sa, int cols_a, const voi
              stride_ok(strideB, batch) && stride_ok(strideD, batch) &&
              (!C || stride_ok(strideC, batch)) && 128 * lda * 2 < (1LL << 31) &&
              128 * ldb * 2 < (1LL << 31) && mt * (mt + 1) / 2 * batch <= 512;
+  // The copies read everything before D is stored: a D that lies over an operand or the addend in
+  // part (its own address is refused above) keeps them.
+  pl->edge = pl->edge && !spans_overlap(A, lda, strideA, K, D, ldd, strideD, M, M, batch) &&
+             !spans_overlap(B, ldb, strideB, K, D, ldd, strideD, M, M, batch) &&
+             !(C && spans_overlap(C, ldc, strideC, M, D, ldd, strideD, M, M, batch));
   const int64_t L = batch, xa = L * pl->Mp * (int64_t)pl->Kp * 2, xd = L * pl->Mp * (int64_t)pl->Mp * 2;
   int64_t off = align256(xa);
   pl->offB = pl->b_copy ? off : 0;
@@ -1013,11 +1018,6 @@ int syrk_impl(const char* who, int elt, const void* A, int64_t lda, int64_t stri
   if (syrk_plan(who, A, lda, strideA, B, ldb, strideB, C, ldc, strideC, D, ldd, strideD, M, K,
                 batch, tile_req, &pl))
     return 1;
-  // The copies read everything before D is stored: a D that lies over an operand or the addend in
-  // part (its own address is refused above) keeps them.
-  pl->edge = pl->edge && !spans_overlap(A, lda, strideA, K, D, ldd, strideD, M, M, batch) &&
-             !spans_overlap(B, ldb, strideB, K, D, ldd, strideD, M, M, batch) &&
-             !(C && spans_overlap(C, ldc, strideC, M, D, ldd, strideD, M, M, batch));
   NtArgs s{};
   s.elt = elt;
   s.M = pl.Mp; s.N = pl.Mp; s.K = pl.Kp; s.L = batch;
