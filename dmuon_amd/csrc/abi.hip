@@ -219,8 +219,27 @@ int plan(int rows, int cols, int batch, int tile_req, int num_cus, int gram, int
 // that stand for them here). Only the comparison of two splits matters.
 double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, bool gram) {
   // launches of one NS run of five steps: X X^T, m x m triangle products, Q updates, P X
-  const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_full = gram ? 3 : 0,
-               n_px = gram ? 2 : 5;
+  const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_px = gram ? 2 : 5;
+  double n_full = gram ? 3 : 0;
+  if (gram && 2 * n <= kMaxGroups) {
+    NtArgs tri[kMaxGroups], q[kMaxGroups];
+    for (int i = 0; i < n; ++i) {
+      const int m = g[i].rows < g[i].cols ? g[i].rows : g[i].cols;
+      NtArgs& s = tri[i];
+      s = NtArgs{};
+      s.M = s.N = s.K = (int)round_up(m, tile);
+      s.k_loop = (int)round_up(m, 64);
+      s.live_rows = s.live_cols = s.k_loop < s.M ? s.k_loop : 0;
+      s.L = g[i].batch;
+      q[i] = s;
+      s.tri = 1;
+      s.tiles_per_mat = tri_tiles(s.M, tile);
+      q[i].tiles_per_mat = (s.M / tile) * (s.M / tile);
+    }
+    // one of the Q updates in the CUs that the triangle launches leave idle: about half of its
+    // time comes back (one 1024^2 matrix 4.6 of 10 us, one 4096^2 55 of 104)
+    if (nt_fill_pays(tri, q, n, tile, num_cus)) n_full = 2.5;
+  }
   auto launch = [&](auto&& dims) {   // dims(group, tile): (tiles of one matrix, K)
     auto total = [&](int t) {
       double tiles = 0;
@@ -523,10 +542,10 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
                       [&](Group& g, NtArgs& s) { q_args(g, s, from, a_, last); });
   };
   // A Q update with R's update and another step behind it: W, R and the next Z do not read Q, so
-  // its tiles go where these triangle launches leave CUs idle, and what is left runs with the
-  // last of them. One 4096^2 matrix: 136 tiles each on 256 CUs, so the 256 tiles of the update
-  // cost no launch of their own. As a D-only product it is EPI_SYM's arithmetic without a
-  // triangle (alpha = 1: the same bits). Needs a table entry per group.
+  // its tiles may go where these triangle launches leave CUs idle, and what is left run with the
+  // last of them (nt_fill_pays). One 4096^2 matrix: 136 tiles each on 256 CUs, so the 256 tiles of
+  // the update cost no launch of their own. As a D-only product it is EPI_SYM's arithmetic without
+  // a triangle (alpha = 1: the same bits). Needs a table entry per group.
   NtFill fill;
   bool filling = false;
   // iterations from it up to the next restart (or T): the Q updates the segment has left
@@ -598,26 +617,31 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
         }, filling ? &fill : nullptr, true))
       return 1;
     filling = false;
-    if (fresh) {
-      qs = 0;
-    } else if (evolve && 2 * c.n <= kMaxGroups) {
-      fill.next = 0;
+    auto w_args = [&](Group& g, NtArgs& s) {   // W = Z R + a R (the stored R is rs times R)
+      symmetric_square(g, s, g.w.Pm, g.w.Am, g.w.Am, g.w.Wm, 1.f, ca, 0.f);
+    };
+    if (!fresh && evolve && 2 * c.n <= kMaxGroups) {
+      NtArgs tri[kMaxGroups];
+      product_args(c, tri, w_args);
       product_args(c, fill.a, [&](Group& g, NtArgs& s) {
         q_args(g, s, qs, ca, false);
         s.mode = EPI_SYM;
       });
-      filling = true;
+      fill.next = 0;
+      filling = nt_fill_pays(tri, fill.a, c.n, c.tile, 0);
+    }
+    if (fresh) {
+      qs = 0;
+    } else if (filling) {
       qs = 1 - qs;
     } else {
       if (q_update(qs, ca, updates_left(it) == 1)) return 1;   // Q <- Z Q + a Q
       qs = 1 - qs;
     }
     if (evolve) {
-      // W = Z R + a R (the stored R is rs times R), then R = P R P = W Z + a W
+      // W, then R = P R P = W Z + a W
       NtFill* more = filling ? &fill : nullptr;
-      if (nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
-            symmetric_square(g, s, g.w.Pm, g.w.Am, g.w.Am, g.w.Wm, 1.f, ca, 0.f);
-          }, more) ||
+      if (nt_product(c, PC_POLY, poly_flops, w_args, more) ||
           nt_product(c, PC_POLY, poly_flops, [&](Group& g, NtArgs& s) {
             symmetric_square(g, s, g.w.Wm, g.w.Pm, g.w.Wm, g.w.Am, 1.f / g.rs, ca / g.rs, 0.f);
           }, more))

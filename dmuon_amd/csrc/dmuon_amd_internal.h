@@ -99,6 +99,9 @@ struct NtFill {
 };
 hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int tile,
                           hipStream_t stream);
+// Whether three launches of `a` do better with `fill`'s tiles among them (the last one `all`) than
+// with a launch of its own for `fill`; num_cus 0: of the current device. Host only.
+bool nt_fill_pays(const NtArgs* a, const NtArgs* fill, int n, int tile, int num_cus);
 // The logical tile the NT kernels give hardware block b of a launch of nb blocks (host copy of
 // the device mapping, for tests: it must be a permutation of 0 .. nb - 1).
 int nt_block_tile(int b, int nb);

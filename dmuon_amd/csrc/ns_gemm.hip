@@ -25,6 +25,7 @@
 //     wait, not the arithmetic, so every variant gives the same bits.
 #include "dmuon_amd_internal.h"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -1465,8 +1466,7 @@ struct NtChoice {
   int tile;
   long long nb, slots;
 };
-NtChoice choose_kernel(const NtArgs* const* a, int cnt, int tile) {
-  const int cus = current_device_cus();
+NtChoice choose_kernel(const NtArgs* const* a, int cnt, int tile, int cus) {
   long long nb = 0, nb256 = 0, nb64 = 0;
   bool split256 = true;
   for (int i = 0; i < cnt; ++i) {
@@ -1491,6 +1491,50 @@ NtChoice choose_kernel(const NtArgs* const* a, int cnt, int tile) {
 
 }  // namespace
 
+// Three launches of `a` with `fill`'s tiles in their idle slots against the same three and one
+// launch of `fill`. The last of the three takes every tile that is left, at its own tile size and
+// blocks per CU, where the launch alone takes the kernel that suits it. So the fill pays while the
+// last launch gains no more waves than the launch alone has. Measured as the gain of a whole
+// Newton-Schulz call, percent (1 .. 80 matrices of 192 .. 4096 rows, both ways in turn on several
+// cards):
+//  - no wave more: 1 .. 5.8 (one 1024^2 2.2, one 4096^2 2.5, two 3072^2 5.8);
+//  - one more against one: -1 .. 3.9, which side differing from card to card (two 128-tiles per CU:
+//    sixteen 704^2 1.4, three 2048^2 -0.4; one: ten 768^2 2.4, twelve 640^2 -1.2; 64-tiles, which
+//    then run in pairs: one 1152^2 2.8);
+//  - two more against one: -4.7 .. 0.5 but for twelve 1024^2 (1.1): one 2560^2 -2.4, one 3840^2
+//    -1.5, two 1408^2 -3.6, one 1280^2 -1.6, eight 896^2 -3.5. Against two waves 0.6 .. 2.0
+//    (thirty-two 576^2), on 256-tiles -1.1 .. 0.1 (six 2048^2) unless the launches have several
+//    waves in any case (twenty-four 1408^2 1.3).
+// 64-tiles with K loops of up to 8 slices take 4 us either way, and three launches that are nearly
+// full cost more of it than one: sixteen 256^2 -3.6, four 512^2 -1.4, eight 384^2 -2.3 (but three
+// 512^2, 192 tiles, 1.2, and as well filled pairs ten 384^2 1.7).
+bool nt_fill_pays(const NtArgs* a, const NtArgs* fill, int n, int tile, int num_cus) {
+  const int cus = num_cus > 0 ? num_cus : current_device_cus();
+  if (n < 1 || 2 * n > kMaxGroups || cus <= 0) return false;
+  const NtArgs *pa[kMaxGroups], *pf[kMaxGroups];
+  long long tiles = 0;
+  int slices = 0;
+  for (int i = 0; i < n; ++i) {
+    pa[i] = &a[i];
+    pf[i] = &fill[i];
+    slices = std::max(slices, (a[i].k_loop > 0 ? a[i].k_loop : a[i].K) / 64);
+  }
+  const NtChoice k = choose_kernel(pa, n, tile, cus), own = choose_kernel(pf, n, tile, cus);
+  for (int i = 0; i < n; ++i) {
+    int mt, nt;
+    tiles += tiles_of(fill[i], k.tile, &mt, &nt) * fill[i].L;
+  }
+  if (k.nb <= 0 || tiles <= 0) return false;
+  const long long room = (k.slots - k.nb % k.slots) % k.slots;
+  const long long last = k.nb + std::max(0LL, tiles - 2 * room);
+  if (k.kernel == NT_64 && slices <= 8 && 4 * tiles > 3 * k.slots && 4 * last <= 5 * k.slots)
+    return false;
+  auto waves = [](long long nb, long long slots) { return (nb + slots - 1) / slots; };
+  const long long more = waves(last, k.slots) - waves(k.nb, k.slots);
+  const long long alone = waves(own.nb, own.slots);
+  return more < alone || (more == alone && !(k.kernel == NT_PP256 && k.nb <= k.slots));
+}
+
 hipError_t launch_nt_batch(const NtArgs* a, int n, int tile, hipStream_t stream) {
   return launch_nt_fill(a, n, nullptr, false, tile, stream);
 }
@@ -1506,7 +1550,7 @@ hipError_t launch_nt_fill(const NtArgs* a, int n, NtFill* fill, bool all, int ti
   if ((cnt > 1 || fill) && a[0].elt != ELT_F16) return hipErrorInvalidValue;
   // an edge product runs on the 128- and 64-tile kernels only
   if (a[0].edge && (cnt > 1 || fill || tile != 128)) return hipErrorInvalidValue;
-  NtChoice k = choose_kernel(list, cnt, tile);
+  NtChoice k = choose_kernel(list, cnt, tile, current_device_cus());
   long long nb = k.nb;
   NtBatch b;
   b.n = 0;
