@@ -662,7 +662,7 @@ int run_gram(Call& c, const float* coeffs, int T, const int* restarts, int n_res
 int run_stage(const Call& c, float mu, int nesterov, float eps) {
   PreArgs p[2 * kMaxGroups];
   int np = 0;
-  bool est = false, exact = false, few_parts = true;
+  bool est = false, exact = false;
   double pre_bytes = 0.0, st_bytes = 0.0, norm_bytes = 0.0;
   NormArgs na[kMaxGroups];
   for (int i = 0; i < c.n; ++i) {
@@ -714,7 +714,6 @@ int run_stage(const Call& c, float mu, int nesterov, float eps) {
     }
     na[i] = NormArgs{g.w.partials, g.w.nparts, g.batch, g.w.scale, g.w.est_old, g.est_ptrs,
                      g.w.ratio, g.w.ratio_sq, g.w.restage};
-    few_parts = few_parts && g.w.nparts <= kNormStageParts;
     norm_bytes += (double)g.batch * g.w.nparts * 4;
   }
   if (est && exact)
@@ -737,7 +736,7 @@ int run_stage(const Call& c, float mu, int nesterov, float eps) {
             [&] { return launch_pre_batch(p, np, c.stream); }))
     return 1;
   // small matrices: the norm and the exact staging in one launch
-  if (few_parts) {
+  if (norm_stage_pays(na, c.n, p, np)) {
     stage(PRE_F16, false);
     return timed(PC_NORM, 0.0, norm_bytes + st_bytes, c.stream, c.who,
                  [&] { return launch_norm_stage(na, c.n, p, np, eps, c.stream); });

@@ -775,16 +775,56 @@ hipError_t launch_pre_batch(const PreArgs* a, int n, hipStream_t stream) {
 
 hipError_t launch_pre(const PreArgs& a, hipStream_t stream) { return launch_pre_batch(&a, 1, stream); }
 
+namespace {
+
+// Blocks per matrix of norm_stage_kernel. Staged again only now and then: 1024 blocks over the
+// call's matrices (8 at least each), of which the usual step runs the sums only. Without kept
+// scales every tile has its block.
+int norm_stage_blocks(const PreArgs& s, bool kept, long long matrices) {
+  const long long tiles = (long long)(s.Rp / kTile) * (s.Cp / kTile);
+  return (int)(kept ? std::min(tiles, std::max(8LL, 1024 / matrices)) : tiles);
+}
+long long matrices_of(const NormArgs* a, int n) {
+  long long matrices = 0;
+  for (int g = 0; g < n; ++g) matrices += a[g].L;
+  return matrices;
+}
+
+}  // namespace
+
+// Every block sums its matrix's partials before its first tile, and the exact staging leaves the
+// contiguous-run kernels for the tiles, so the one launch pays for small matrices only. Measured
+// against two launches, both in turn:
+//  - without kept scales, by the partials that all blocks read: a call of eight 1024 x 4096 (2^25)
+//    738 -> 733 us and of eight 1024 x 2048 577 -> 572, but thirty-two 512 x 8192 (2^27) 1166 ->
+//    1193 and sixty-four 1408 x 2048 5881 -> 5945;
+//  - with kept scales the usual step only sums (a gain of 1 .. 3 us at any size), while the first
+//    one, which stages every matrix, has few blocks: the staging of sixty-four 2048 x 1408 (3072
+//    partials each) 637 -> 720 us, of thirty-two 1024 x 4096 398 -> 420, of four 59.1 -> 59.2, and
+//    of sixty-four 1024 x 1024 233 -> 205.
+bool norm_stage_pays(const NormArgs* a, int n, const PreArgs* p, int np) {
+  const long long matrices = matrices_of(a, n);
+  long long reads = 0;
+  for (int g = 0; g < n; ++g) {
+    if (a[g].nparts > kNormStageParts) return false;
+    if (a[g].est_ptrs && a[g].nparts > kNormStageParts / 2 &&
+        (long long)a[g].L * a[g].nparts > kNormStageFirst)
+      return false;
+  }
+  for (int i = 0; i < np; ++i) {
+    const NormArgs& g = a[p[i].norm_group];
+    reads += (long long)norm_stage_blocks(p[i], g.est_ptrs != nullptr, matrices) * p[i].L * g.nparts;
+  }
+  return reads <= kNormStageReads;
+}
+
 hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np, float eps,
                              hipStream_t stream) {
   if (n < 1 || n > kMaxGroups || np < 1 || np > 2 * kMaxGroups) return hipErrorInvalidValue;
   NormBatch b;
   b.n = n;
-  long long matrices = 0;
-  for (int g = 0; g < n; ++g) {
-    b.a[g] = a[g];
-    matrices += a[g].L;
-  }
+  const long long matrices = matrices_of(a, n);
+  for (int g = 0; g < n; ++g) b.a[g] = a[g];
   PreBatch q;
   q.n = 0;
   long long blocks = 0;
@@ -796,11 +836,7 @@ hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np,
     PreArgs& s = q.a[q.n];
     s = p[i];
     s.restage = nullptr;
-    // Staged again only now and then: 1024 blocks over the call's matrices (8 at least each), of
-    // which the usual step runs the sums only. Without kept scales every tile has its block.
-    const long long tiles = (long long)(s.Rp / kTile) * (s.Cp / kTile);
-    const long long few = std::max(8LL, 1024 / matrices);
-    s.stage_blocks = (int)(a[s.norm_group].est_ptrs ? std::min(tiles, few) : tiles);
+    s.stage_blocks = norm_stage_blocks(s, a[s.norm_group].est_ptrs != nullptr, matrices);
     q.first[q.n++] = (unsigned)blocks;
     blocks += (long long)s.stage_blocks * s.L;
   }
