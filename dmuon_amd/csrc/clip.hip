@@ -245,28 +245,58 @@ __device__ __forceinline__ float clip_coef(float norm, float max_norm) {
   return c > 1.f ? 1.f : c;
 }
 
-// From the pieces' sums to norms, coefficients and flags, in one block of 16 waves: a wave per
-// tensor sums its pieces in fp64 in a fixed order, then
+// From the pieces' sums to norms, coefficients and flags. A wave per tensor sums its pieces in fp64
+// in a fixed order, then
 //   global:    the tensor norms, each rounded to its tensor's dtype (as torch._foreach_norm
 //              returns them), make one norm and one coefficient;
 //   otherwise: one norm and coefficient per segment, and the norm of those.
-// Bounded by latency (a few thousand pieces); it takes the place of ~20 torch operations on
-// one-element tensors, about 4 us each on the device and more on the host: one transformer
-// layer's gradients (218 M bf16 elements) 251 -> 218 us a call, three small ones 99 -> 37 us.
-constexpr int kFinishWaves = 16;
-__global__ __launch_bounds__(64 * kFinishWaves) void clip_finish_kernel(const ClipFinishArgs a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int t = wave; t < a.n; t += kFinishWaves) {
-    const long long k1 = (long long)a.first_job[t + 1] * a.pieces;
-    double s = 0.0;
-    for (long long k = (long long)a.first_job[t] * a.pieces + lane; k < k1; k += 64)
-      s += (double)a.partials[k];
-    s = wave_sum(s);
-    if (lane == 0) a.tensor_sq[t] = s;
-  }
+// Few tensors and segments: one block of 16 waves does it all (FINISH_ALL), bounded by latency; it
+// takes the place of ~20 torch operations on one-element tensors, about 4 us each on the device and
+// more on the host: one transformer layer's gradients (218 M bf16 elements) 251 -> 218 us a call,
+// three small ones 99 -> 37 us. That block's loops over tensors and segments are serial chains of
+// loads (0.6 us for 16 tensors), so more than kFinishTensors of either take a launch per stage,
+// spread over the device: FINISH_TENSORS (16 tensors a block), FINISH_SEGMENTS (a block per segment,
+// or the one of the global norm) and FINISH_TOTAL. Norms of 1000 tensors of 16384 bf16 values 52 ->
+// 14 us on the device, of 10000 of 4096 455 -> 30; 256 of 65536 would be 26 -> 17, but the host
+// takes 4 us more for the two launches.
+constexpr int kFinishWaves = 16, kFinishTensors = 256;
+enum { FINISH_ALL, FINISH_TENSORS, FINISH_SEGMENTS, FINISH_TOTAL };
+
+// sum over the block; the result is in thread 0
+__device__ __forceinline__ double finish_sum(double v, double* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
+  double all = 0.0;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < kFinishWaves; ++w) all += red[w];
+  return all;
+}
+__device__ __forceinline__ void finish_segment(const ClipFinishArgs& a, int g, float norm) {
+  a.norms[g] = norm;
+  a.coefs[g] = a.has_max ? clip_coef(norm, a.max_norm) : 1.f;
+  a.clipped[g] = a.has_max && finite(norm) && norm > a.max_norm;
+  a.found_inf[g] = !finite(norm);
+}
+
+template <int PART>
+__global__ __launch_bounds__(64 * kFinishWaves) void clip_finish_kernel(const ClipFinishArgs a) {
   __shared__ double red[kFinishWaves];
-  if (a.global) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if constexpr (PART == FINISH_ALL || PART == FINISH_TENSORS) {
+    const int step = kFinishWaves * gridDim.x;
+    for (int t = blockIdx.x * kFinishWaves + wave; t < a.n; t += step) {
+      const long long k1 = (long long)a.first_job[t + 1] * a.pieces;
+      double s = 0.0;
+      for (long long k = (long long)a.first_job[t] * a.pieces + lane; k < k1; k += 64)
+        s += (double)a.partials[k];
+      s = wave_sum(s);
+      if (lane == 0) a.tensor_sq[t] = s;
+    }
+    if constexpr (PART == FINISH_TENSORS) return;
+    __syncthreads();
+  }
+  if (PART != FINISH_TOTAL && a.global) {
     double s = 0.0;
     for (int t = threadIdx.x; t < a.n; t += 64 * kFinishWaves) {
       float norm = sqrtf((float)a.tensor_sq[t]);
@@ -274,13 +304,9 @@ __global__ __launch_bounds__(64 * kFinishWaves) void clip_finish_kernel(const Cl
       else if (a.dtypes[t] == CBF16) norm = to_f<CBF16>(from_f<CBF16>(norm));
       s += (double)norm * (double)norm;
     }
-    s = wave_sum(s);
-    if (lane == 0) red[wave] = s;
-    __syncthreads();
+    s = finish_sum(s, red);
     if (threadIdx.x == 0) {
-      double all = 0.0;
-      for (int w = 0; w < kFinishWaves; ++w) all += red[w];
-      const float total = (float)sqrt(all);
+      const float total = (float)sqrt(s);
       const float c = a.max_norm / (total + 1e-6f);
       a.norms[0] = total;
       a.coefs[0] = a.has_max ? clip_coef(total, a.max_norm) : 1.f;
@@ -289,28 +315,32 @@ __global__ __launch_bounds__(64 * kFinishWaves) void clip_finish_kernel(const Cl
     }
     return;
   }
-  double all = 0.0;                      // of this wave's segments
-  for (int g = wave; g < a.n_segments; g += kFinishWaves) {
+  if constexpr (PART == FINISH_SEGMENTS) {
     double s = 0.0;
-    for (int t = lane; t < a.n; t += 64)
-      if (a.segments[t] == g) s += a.tensor_sq[t];
-    s = wave_sum(s);
-    const float norm = sqrtf((float)s);
-    all += (double)norm * (double)norm;
-    if (lane == 0) {
-      a.norms[g] = norm;
-      a.coefs[g] = a.has_max ? clip_coef(norm, a.max_norm) : 1.f;
-      a.clipped[g] = a.has_max && finite(norm) && norm > a.max_norm;
-      a.found_inf[g] = !finite(norm);
+    for (int t = threadIdx.x; t < a.n; t += 64 * kFinishWaves)
+      if (a.segments[t] == (int)blockIdx.x) s += a.tensor_sq[t];
+    s = finish_sum(s, red);
+    if (threadIdx.x == 0) finish_segment(a, blockIdx.x, sqrtf((float)s));
+    return;
+  }
+  double all = 0.0;
+  if constexpr (PART == FINISH_ALL) {     // of this wave's segments
+    for (int g = wave; g < a.n_segments; g += kFinishWaves) {
+      double s = 0.0;
+      for (int t = lane; t < a.n; t += 64)
+        if (a.segments[t] == g) s += a.tensor_sq[t];
+      const float norm = sqrtf((float)wave_sum(s));
+      if (lane == 0) {
+        all += (double)norm * (double)norm;
+        finish_segment(a, g, norm);
+      }
     }
+  } else {
+    for (int g = threadIdx.x; g < a.n_segments; g += 64 * kFinishWaves)
+      all += (double)a.norms[g] * (double)a.norms[g];
   }
-  if (lane == 0) red[wave] = all;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    all = 0.0;
-    for (int w = 0; w < kFinishWaves; ++w) all += red[w];
-    a.norms[a.n_segments] = (float)sqrt(all);
-  }
+  all = finish_sum(all, red);
+  if (threadIdx.x == 0) a.norms[a.n_segments] = (float)sqrt(all);
 }
 
 }  // namespace
@@ -327,7 +357,16 @@ hipError_t launch_clip_norms(ClipArgs a, const ClipFinishArgs& f, hipStream_t st
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(clip_finish_kernel, dim3(1), dim3(64 * kFinishWaves), 0, stream, f);
+  const dim3 one(1), threads(64 * kFinishWaves);
+  if (f.n <= kFinishTensors && f.n_segments <= kFinishTensors) {
+    hipLaunchKernelGGL(clip_finish_kernel<FINISH_ALL>, one, threads, 0, stream, f);
+    return hipGetLastError();
+  }
+  const unsigned blocks = (unsigned)((f.n + kFinishWaves - 1) / kFinishWaves);
+  hipLaunchKernelGGL(clip_finish_kernel<FINISH_TENSORS>, dim3(blocks), threads, 0, stream, f);
+  hipLaunchKernelGGL(clip_finish_kernel<FINISH_SEGMENTS>,
+                     dim3(f.global ? 1u : (unsigned)f.n_segments), threads, 0, stream, f);
+  if (!f.global) hipLaunchKernelGGL(clip_finish_kernel<FINISH_TOTAL>, one, threads, 0, stream, f);
   return hipGetLastError();
 }
 

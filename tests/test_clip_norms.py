@@ -137,3 +137,38 @@ def test_a_cached_table_waits_for_its_upload_on_another_stream(gpu):
         norms = table.norms(2, None)[0]
     for n, g in zip(norms.tolist(), grads):
         assert n == pytest.approx(float(g.double().norm()), rel=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,n_segments", [(256, 256), (257, 1), (257, 257), (2000, 3), (40, 700)])
+def test_many_tensors_and_segments(gpu, n, n_segments):
+    """On both sides of what one finishing block takes: norms, total, coefficients and flags, for
+    segments (some of them empty) and for one norm over all tensors."""
+    sizes = [1 + (7 * i) % 300 for i in range(n)]
+    sizes[n // 2] = 40_000
+    dts = [DT[i % 3] for i in range(n)]
+    grads = _grads(sizes, dts, gpu, n)
+    of = [(5 * i) % n_segments for i in range(n)]
+    sq = [0.0] * n_segments
+    for g, s in zip(grads, of):
+        sq[s] += float(g.double().square().sum())
+    table = fast_clip._JobTable(grads, of, gpu, 4096)
+    norms, coefs, clipped, found = table.norms(n_segments, 6.0)
+    want = torch.tensor(sq, dtype=torch.float64).sqrt()
+    torch.testing.assert_close(norms[:-1].cpu().double(), want, rtol=1e-6, atol=1e-30)
+    assert float(norms[-1]) == pytest.approx(float(want.norm()), rel=1e-6)
+    torch.testing.assert_close(coefs.cpu().double(), (6.0 / (want + 1e-6)).clamp(max=1.0),
+                               rtol=1e-6, atol=0.0)
+    assert clipped.tolist() == (want > 6.0).tolist() and not found.any()
+    one = table.norms(0, 6.0)
+    total = math.sqrt(sum(float(g.double().norm().to(g.dtype)) ** 2 for g in grads))
+    assert float(one[0][0]) == pytest.approx(total, rel=1e-6)
+    assert float(one[1][0]) == pytest.approx(min(1.0, 6.0 / (total + 1e-6)), rel=1e-6)
+    assert bool(one[2][0]) == (total > 6.0) and not bool(one[3][0])
+    for a, b in zip((*table.norms(n_segments, 6.0), *table.norms(0, 6.0)),
+                    (norms, coefs, clipped, found, *one)):
+        assert torch.equal(a[:1], b[:1])               # the same bits on every call
+    grads[n - 1][0] = float("nan")
+    found = table.norms(n_segments, 6.0)[3]
+    assert found.tolist() == [s == of[n - 1] for s in range(n_segments)]
+    assert bool(table.norms(0, 6.0)[3][0])
