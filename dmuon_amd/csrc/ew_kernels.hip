@@ -61,10 +61,6 @@ typedef unsigned u32x4_copy_t __attribute__((ext_vector_type(4)));
 // memory and would emit flat accesses (which also count against lgkmcnt); cast to the global
 // address space.
 template <class V>
-__device__ __forceinline__ V ldg_nt(const V* p) {
-  return __builtin_nontemporal_load((const __attribute__((address_space(1))) V*)p);
-}
-template <class V>
 __device__ __forceinline__ void stg_nt(V* p, V v) {
   __builtin_nontemporal_store(v, (__attribute__((address_space(1))) V*)p);
 }
@@ -76,9 +72,9 @@ __device__ __forceinline__ float staged_scale(const PreArgs& a, int l, bool firs
   return est;
 }
 
-// Four values of a row whose pitch may be any number of elements: vector accesses that state the
-// element's own alignment (global memory takes them; a row of 3001 columns is never 8-byte
-// aligned).
+// Four values of a caller's tensor, whose base and row pitch may be any number of elements: vector
+// accesses that state the element's own alignment (global memory takes them; a view need not start
+// at 8 bytes, and a row of 3001 columns is never 8-byte aligned).
 typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
 typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
 __device__ __forceinline__ f32x4_t ldg_nt_any(const float* p) {
@@ -295,9 +291,9 @@ using GradWords = typename std::conditional<GF, f32x4_t, u32x2_t>::type;
 template <bool GF>
 __device__ __forceinline__ GradWords<GF> pre_load_g(const void* g, long long i) {
   if constexpr (GF)
-    return ldg_nt(reinterpret_cast<const f32x4_t*>(static_cast<const float*>(g) + i));
+    return ldg_nt_any(static_cast<const float*>(g) + i);
   else
-    return ldg_nt(reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(g) + i));
+    return ldg_nt_any(static_cast<const uint16_t*>(g) + i);
 }
 template <bool GF>
 __device__ __forceinline__ void pre_unpack(const GradWords<GF>& t, const f32x4_t& b,
@@ -342,8 +338,7 @@ __global__ __launch_bounds__(256) void muon_pre_wide_kernel(const ARGS args) {
   bool copy;
   const float sc = pre_scale<ST>(a, l, blk == l * per, copy);
   const GradWords<GF> gw = pre_load_g<GF>(g, i);
-  const f32x4_t bw = read_buf ? ldg_nt(reinterpret_cast<const f32x4_t*>(buf + i))
-                              : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const f32x4_t bw = read_buf ? ldg_nt_any(buf + i) : f32x4_t{0.f, 0.f, 0.f, 0.f};
   float gv[4], bv[4], nb[4], ns[4];
   pre_unpack<GF>(gw, bw, gv, bv);
   float ss = 0.f;
@@ -353,7 +348,7 @@ __global__ __launch_bounds__(256) void muon_pre_wide_kernel(const ARGS args) {
     ss += ns[e] * ns[e];
   }
   if (ST != PRE_F16 && buf)
-    stg_nt(reinterpret_cast<f32x4_t*>(buf + i), f32x4_t{nb[0], nb[1], nb[2], nb[3]});
+    stg_nt_any(buf + i, f32x4_t{nb[0], nb[1], nb[2], nb[3]});
   if (copy) {
     u32x2_t p;
     p.x = (uint32_t)pre_out<ST>(ns[0], sc) | ((uint32_t)pre_out<ST>(ns[1], sc) << 16);
@@ -403,8 +398,7 @@ __global__ __launch_bounds__(256) void muon_pre_tall_kernel(const ARGS args) {
     if (read_buf) {
 #pragma unroll
       for (int q = 0; q < RB; ++q)
-        bw[q] = ldg_nt(reinterpret_cast<const f32x4_t*>(buf + (r0 + w + 4 * (rb + q)) * a.cols +
-                                                        c0 + c));
+        bw[q] = ldg_nt_any(buf + (r0 + w + 4 * (rb + q)) * a.cols + c0 + c);
     } else {
 #pragma unroll
       for (int q = 0; q < RB; ++q) bw[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -420,8 +414,7 @@ __global__ __launch_bounds__(256) void muon_pre_tall_kernel(const ARGS args) {
         ss[(rb + q) / 4] += ns[e] * ns[e];
       }
       if (ST != PRE_F16 && buf)
-        stg_nt(reinterpret_cast<f32x4_t*>(buf + (r0 + rl) * a.cols + c0 + c),
-               f32x4_t{nb[0], nb[1], nb[2], nb[3]});
+        stg_nt_any(buf + (r0 + rl) * a.cols + c0 + c, f32x4_t{nb[0], nb[1], nb[2], nb[3]});
       if (copy) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) tt[c + e][rl] = pre_out<ST>(ns[e], sc);

@@ -11,20 +11,30 @@ from dmuon_amd.optim.syrk_dispatch import syrk_or_cublas
 LR, MU, WD = 0.02, 0.95, 0.1
 
 
-def _off(t, off):
-    """``t`` at ``off`` elements past an aligned base."""
-    base = torch.empty(t.numel() + off, dtype=t.dtype, device=t.device)
-    v = base[off:].view(t.shape)
-    v.copy_(t)
-    return v
+class _Off:
+    """``t`` at ``off`` elements past an aligned base, between margins of a known value."""
+
+    def __init__(self, t, off):
+        self.off, self.n = off, t.numel()
+        self.base = torch.full((off + self.n + 64,), 7.0, dtype=t.dtype, device=t.device)
+        self.t = self.base[off:off + self.n].view(t.shape)
+        self.t.copy_(t)
+
+    def margins_are_whole(self):
+        return bool((self.base[:self.off] == 7.0).all()
+                    and (self.base[self.off + self.n:] == 7.0).all())
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("wdt,pdt", [(torch.float32, torch.bfloat16), (torch.bfloat16, None),
                                      (torch.float32, None)])
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,cols", [(65, 131), (131, 65), (64, 7), (257, 300), (300, 257)])
-def test_step_at_any_element_alignment(gpu, rows, cols, gdt, wdt, pdt):
+# padded shapes (the 64x64 staging tiles) and whole ones (the flat and, with a kept scale, the tall
+# staging kernel)
+@pytest.mark.parametrize("rows,cols", [(65, 131), (131, 65), (64, 7), (257, 300), (300, 257),
+                                       (128, 256), (512, 256)])
+@pytest.mark.parametrize("kept", [False, True])
+def test_step_at_any_element_alignment(gpu, rows, cols, kept, gdt, wdt, pdt):
     gen = torch.Generator(device=gpu).manual_seed(rows)
     g = torch.randn(rows, cols, device=gpu, generator=gen).mul_(0.02).to(gdt)
     b = torch.randn(rows, cols, device=gpu, generator=gen).mul_(0.02)
@@ -34,24 +44,30 @@ def test_step_at_any_element_alignment(gpu, rows, cols, gdt, wdt, pdt):
     code = {torch.float32: _C.DTYPE_F32, torch.bfloat16: _C.DTYPE_BF16}
     _, nbytes, _ = _C.plan_groups([(rows, cols, 1)], 128, backend=_C.NS_GRAM)
     runs = []
+    momentum = b * MU + g.float()
+    scale = 1.0 / float((g.double() + MU * momentum.double()).norm())
     for off in (0, 1, 3, 5):
-        t = [_off(x, off) for x in (g, b, w)]
-        p = None if pdt is None else _off(torch.zeros(rows, cols, dtype=pdt, device=gpu), off)
-        guard = torch.full((64,), 7.0, device=gpu)
-        ptr = torch.tensor([x.data_ptr() for x in (*t, *([] if p is None else [p]))],
+        held = [_Off(x, off) for x in (g, b, w)]
+        if pdt is not None:
+            held.append(_Off(torch.zeros(rows, cols, dtype=pdt, device=gpu), off))
+        t = [h.t for h in held]
+        p = None if pdt is None else t[3]
+        est = torch.tensor([scale], device=gpu)
+        ptr = torch.tensor([x.data_ptr() for x in t] + [0] * (4 - len(t)) + [est.data_ptr()],
                            dtype=torch.int64, device=gpu)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
         base = ptr.data_ptr()
-        _C.call("dmuon_muon_step_group", base, code[gdt], base + 8, None, base + 16, code[wdt],
+        _C.call("dmuon_muon_step_group", base, code[gdt], base + 8,
+                base + 32 if kept else None, base + 16, code[wdt],
                 None if p is None else base + 24, 0 if p is None else code[pdt], rows, cols, 1, 0,
                 LR, MU, WD, 1, 0, coeff, T, _C.NS_GRAM, rst, n_rst, 1e-7, ws.data_ptr(), nbytes,
                 128, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        assert (guard == 7.0).all()
+        assert all(h.margins_are_whole() for h in held)
         runs.append([t[1].clone(), t[2].clone()] + ([] if p is None else [p.clone()]))
         assert torch.equal(t[0], g)
     # the momentum in the reference's two roundings, the forward copy one rounding of the weight
-    assert torch.equal(runs[0][0], b * MU + g.float())
+    assert torch.equal(runs[0][0], momentum)
     if pdt is not None:
         assert torch.equal(runs[0][2], runs[0][1].to(pdt))
     for r in runs[1:]:
