@@ -584,8 +584,8 @@ __global__ __launch_bounds__(kFinThreads) void norm_finalize_est_kernel(const No
 // Norm and exact staging of small matrices in one launch: every block of a matrix sums its (few)
 // partials itself, the first one writes the outputs, and the matrix's blocks stage its tiles if
 // its kept scale does not do (or there is none). One launch less on every step of a small model
-// (twelve 512x2048 matrices 301.3 -> 298.2 us, one 1024x1024 155.3 -> 154.2, ragged ones 258.8 ->
-// 255.2, one 128x512 Newton-Schulz 66.6 -> 65.9; both sides in turn on one card).
+// (twelve 512x2048 matrices 301.3 -> 298.2 us, ragged ones 258.8 -> 255.2, one 128x512 Newton-Schulz
+// 66.6 -> 65.9, both sides in turn on one card; one 1024x1024 by no more than its runs differ).
 template <class ARGS>
 __global__ __launch_bounds__(256) void norm_stage_kernel(const NormBatch b, const ARGS args,
                                                          float eps) {
@@ -835,15 +835,13 @@ hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np,
   }
   if (blocks == 0) return hipSuccess;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (sizeof(NormBatch) + sizeof(PreBatch) + 64 > 4096 || q.n == 1) {
-    for (int i = 0; i < q.n; ++i)
-      hipLaunchKernelGGL(norm_stage_kernel<PreArgs>,
-                         dim3((unsigned)((long long)q.a[i].stage_blocks * q.a[i].L)), dim3(256), 0,
-                         stream, b, q.a[i], eps);
-  } else {
+  static_assert(sizeof(NormBatch) + sizeof(PreBatch) + 64 <= 4096, "launch arguments");
+  if (q.n == 1)
+    hipLaunchKernelGGL(norm_stage_kernel<PreArgs>, dim3((unsigned)blocks), dim3(256), 0, stream, b,
+                       q.a[0], eps);
+  else
     hipLaunchKernelGGL(norm_stage_kernel<PreBatch>, dim3((unsigned)blocks), dim3(256), 0, stream,
                        b, q, eps);
-  }
   return hipGetLastError();
 }
 
