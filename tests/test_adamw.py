@@ -1,4 +1,5 @@
-"""Fused AdamW (dmuon_adamw_multi): the oracle pinned on the CPU, then the HIP kernel against it.
+"""Fused AdamW (dmuon_adamw_tensors, and dmuon_adamw_multi with a device table): the oracle pinned on
+the CPU, then the HIP kernels against it.
 
 CPU (not gpu): oracle/adamw_oracle.py against the reference's own call sequence
 (muon.py:1902-1916) run through torch._foreach on CPU tensors (bit for bit with bf16 state;
@@ -263,6 +264,48 @@ def test_kernel_large_bucket(gpu):
     # several blocks per tensor and tensors straddling block ranges; more than 16 M elements
     _run_and_check("bf16", "bf16", [(1 << 24) + 3, 4096, 12345, 1 << 20], gpu, 0.1, steps=1,
                    seed=11)
+
+
+# on both sides of 512 * 2048 elements, where a block's share changes; an empty tensor, unaligned views
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[5, 0, 1001, 4099, 65541], [1 << 20, 0, 12345, 4097]])
+@pytest.mark.parametrize("pdt,gdt", [("fp32", "fp32"), ("fp32", "bf16"), ("bf16", "bf16"),
+                                     ("bf16", "fp32")])
+@pytest.mark.parametrize("qdt", [None, "bf16", "fp32"])
+def test_device_table_entry_point(gpu, sizes, pdt, gdt, qdt):
+    """dmuon_adamw_multi on a device table: the oracle's bits, and those of the host-table call, for
+    params, states and forward copies (one tensor without a copy)."""
+    wd, step = 0.1, 3
+    ps, ms, vs = _bucket(pdt, gdt, sizes, gpu, 21, unaligned=True)
+    gs = [_rand(n, 400 + i, 0.01, _DT[gdt]).to(gpu) for i, n in enumerate(sizes)]
+    for i, (m, v) in enumerate(zip(ms, vs)):
+        m.copy_(_rand(m.numel(), 500 + i, 0.005))
+        v.copy_(_rand(v.numel(), 600 + i, 0.01).square())
+    qs = [None if qdt is None or i == 2 else torch.zeros(n, dtype=_DT[qdt], device=gpu)
+          for i, n in enumerate(sizes)]
+    ora = [ao.adamw_step(_np(p.cpu()), _np(g.cpu()), _np(m.cpu()), _np(v.cpu()), step, LR, BETAS, wd,
+                         EPS, pdt) for p, g, m, v in zip(ps, gs, ms, vs)]
+    other = [[t.clone() for t in ts] for ts in (ps, ms, vs)]
+    other_q = [None if q is None else q.clone() for q in qs]
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    rows = [[t.data_ptr() for t in ts] for ts in (ps, gs, ms, vs)]
+    rows += [[0 if q is None else q.data_ptr() for q in qs], off.tolist()]
+    table = torch.tensor([x for r in rows for x in r], dtype=torch.int64).to(gpu)
+    n, base, code = len(sizes), table.data_ptr(), {"fp32": _C.DTYPE_F32, "bf16": _C.DTYPE_BF16}
+    s = adamw_scalars(step, LR, BETAS, wd, EPS)
+    _C.call("dmuon_adamw_multi", base, base + 8 * n, base + 16 * n, base + 24 * n,
+            None if qdt is None else base + 32 * n, base + 40 * n, n, int(off[-1]), code[pdt],
+            code[gdt], 0 if qdt is None else code[qdt], s["apply_wd"], s["wd_scale"], s["beta1"],
+            s["alpha1"], s["beta2"], s["alpha2"], s["bc2_sqrt"], s["eps"], s["neg_step"],
+            torch.cuda.current_stream().cuda_stream)
+    dmuon.fused_adamw_(other[0], gs, other[1], other[2], step=step, lr=LR, betas=BETAS,
+                       weight_decay=wd, eps=EPS, publish=None if qdt is None else other_q)
+    for i, ref in enumerate(ora):
+        for t, o2, r in zip((ps[i], ms[i], vs[i]), (x[i] for x in other), ref):
+            assert torch.equal(_bits(t), _bits(torch.from_numpy(r).to(_DT[pdt]))), (i, sizes[i])
+            assert torch.equal(_bits(t), _bits(o2)), (i, sizes[i])
+        if qs[i] is not None:
+            assert torch.equal(qs[i], ps[i].to(qs[i].dtype)) and torch.equal(qs[i], other_q[i])
 
 
 @pytest.mark.gpu

@@ -1,4 +1,5 @@
-"""Segmented gradient clipping (dmuon_segmented_l2_norm_sq / dmuon_segmented_scale).
+"""Segmented gradient clipping (dmuon_clip_norms / dmuon_segmented_scale, and the reference's norm
+seam dmuon_segmented_l2_norm_sq).
 
 CPU (not gpu): the oracle (oracle/clip_oracle.py) pinned to the known answers of the
 reference's tests (tests/unit/test_fast_clip.py:37-61), to numpy.linalg.norm and to planted
@@ -234,6 +235,56 @@ def test_kernels_match_oracle_reference_buckets(gpu):
 @pytest.mark.parametrize("chunk", [1, 1000, 4097, 20001, 65536])
 def test_kernels_ragged_chunks_and_unaligned(gpu, chunk):
     _check_against_oracle(_mixed_buckets(gpu), gpu, 2.0, chunk_size=chunk, unaligned=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("chunk", [1000, 65536])
+def test_norm_seam_adds_each_segments_sum_of_squares(gpu, chunk):
+    """dmuon_segmented_l2_norm_sq on mixed dtypes, an empty tensor and an unaligned view: adds to what
+    local_sq holds, against float64."""
+    gen = torch.Generator().manual_seed(13)
+    sizes = [300_001, 0, 4096 * 33, 17, 65_537]
+    dts = [torch.float32, torch.float32, torch.bfloat16, torch.float16, torch.float32]
+    grads = [torch.randn(n, generator=gen).to(dt).to(gpu) for n, dt in zip(sizes, dts)]
+    base = torch.zeros(sizes[4] + 1, device=gpu)
+    base[1:] = grads[4]
+    grads[4] = base[1:]
+    segments = [0, 0, 1, 1, 2]
+    local = torch.tensor([1.0, 2.0, 3.0, 4.0], device=gpu)
+    fast_clip._JobTable(grads, segments, gpu, chunk).sumsq(local)
+    want = [1.0, 2.0, 3.0, 4.0]
+    for g, s in zip(grads, segments):
+        want[s] += float(g.double().square().sum())
+    # fp32 sums of at most 300001 terms, each thread a few hundred of them
+    assert local.tolist() == pytest.approx(want, rel=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("max_norm", [2.0, None])
+def test_a_gradient_off_the_kernels_takes_the_others_along(gpu, max_norm):
+    """One non-contiguous gradient: the bucket's norms come from the norm seam and torch together."""
+    gen = torch.Generator().manual_seed(14)
+    host = [torch.randn(5000, generator=gen), torch.randn(64, 48, generator=gen).to(torch.bfloat16),
+            torch.randn(777, generator=gen).to(torch.float16)]
+    grads = [host[0].to(gpu), host[1].to(gpu).t(), host[2].to(gpu)]
+    assert not grads[1].is_contiguous()
+    res = clip_grad_norm_buckets_((GradClipBucket("a", grads[:2], reduce=False),
+                                   GradClipBucket("b", grads[2:], reduce=False)), max_norm)
+    assert res.fastpath
+    norms = co.segment_sumsq([[_np(h) for h in host[:2]], [_np(host[2])]]) ** 0.5
+    for name, norm, gs, hs in (("a", norms[0], grads[:2], [host[0], host[1].t()]),
+                               ("b", norms[1], grads[2:], host[2:])):
+        st = _stats(res)[name]
+        assert float(st.total_norm) == pytest.approx(norm, rel=1e-5)
+        assert float(st.clip_coef) == pytest.approx(
+            float(co.clip_coefs(np.array([norm]), max_norm)[0]), rel=1e-5)
+        coef = np.float32(float(st.clip_coef))
+        for d, h in zip(gs[:1] if name == "a" else gs, hs[:1] if name == "a" else hs):
+            want = _np(h) if max_norm is None else co.scale(_np(h), coef, _DTS[h.dtype])
+            assert np.array_equal(_np(d), want)
+    if max_norm is not None:                            # torch scales the other one
+        coef = _stats(res)["a"].clip_coef
+        assert torch.equal(grads[1], host[1].to(gpu).t() * coef)
 
 
 @pytest.mark.gpu
