@@ -1004,8 +1004,9 @@ int syrk_plan(const char* who, const void* A, int64_t lda, int64_t strideA, cons
   // Ragged operands in whole 16-byte chunks (M and K multiples of 8, aligned rows) are read and
   // written in place by the edge variant of the 128- and 64-tile kernels: one launch instead of
   // up to four (fp16 1000 x 3000, X X^T and its polynomial: 45.4 -> 28.1 us the pair, 3-6 us
-  // for each copy). A product of more than two 128-tiles per CU keeps the copies and the
-  // 256-tile kernel, which are small beside it.
+  // for each copy). A product of more than two 128-tiles per CU (512: the plan of a call, like its
+  // tile, is for 256 CUs, without a look at the device) keeps the copies and the 256-tile kernel,
+  // which are small beside it.
   const int64_t mt = pl->Mp / 128;
   pl->edge = !pl->direct && t == 128 && M % 8 == 0 && K % 8 == 0 && K > 0 && aligned16(A) &&
              aligned16(B) && aligned16(D) && (!C || aligned16(C)) && ld_ok(lda) && ld_ok(ldb) &&

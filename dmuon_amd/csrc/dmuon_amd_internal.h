@@ -60,10 +60,11 @@ struct NtArgs {
   // DIAG_SKIP_WAVES skips the two waves that hold no kept value; DIAG_SKIP_BLOCKS also skips the
   // 16x16 blocks strictly below the diagonal in the waves that straddle it. Same bits each way.
   int diag_skip;
-  // 256-tiles: output rows from live_rows on and columns from live_cols on are padding that no
-  // later product reads (every K loop stops before it; 0: none). A wave whose 128 x 64
-  // sub-tile lies wholly in it does no MFMA work and stores nothing; the padding then holds
-  // whatever it held.
+  // Output rows from live_rows on and columns from live_cols on (multiples of 64; 0: none) are
+  // padding that no later product reads (every K loop stops before it). On 256-tiles a wave whose
+  // 128 x 64 sub-tile lies wholly in it does no MFMA work and stores nothing, and a launch of
+  // 64-tiles has no tiles there at all; the padding then holds whatever it held. An edge product
+  // relies on it: its 64-tiles past m_real rounded up to 64 would have no operands.
   int live_rows, live_cols;
   // EPI_SYM, tri: the operands are the caller's own, m_real x k_real inside the M x K of the tile
   // grid and slices (multiples of 8 elements, 16-byte aligned rows): loads past them give 0,
