@@ -188,10 +188,9 @@ hipError_t launch_norm_finalize_est(const NormArgs* a, int n, float eps, hipStre
 // The same with the PRE_F16 pass over the sets that need it, in one launch (restage[] is not
 // written): every block sums its matrix's partials, so only where those are few.
 constexpr int kNormStageParts = 4096;
-constexpr long long kNormStageReads = 1LL << 25, kNormStageFirst = 1LL << 14;
+constexpr long long kNormStageReads = 1LL << 25;
 // Whether it pays: matrices of at most kNormStageParts partials, at most kNormStageReads of them
-// read by all blocks, and with kept scales at most kNormStageFirst in a group whose matrices have
-// more than half of kNormStageParts. Host only.
+// read by all blocks. Host only.
 bool norm_stage_pays(const NormArgs* a, int n, const PreArgs* p, int np);
 hipError_t launch_norm_stage(const NormArgs* a, int n, const PreArgs* p, int np, float eps,
                              hipStream_t stream);

@@ -770,12 +770,12 @@ hipError_t launch_pre(const PreArgs& a, hipStream_t stream) { return launch_pre_
 
 namespace {
 
-// Blocks per matrix of norm_stage_kernel. Staged again only now and then: 1024 blocks over the
+// Blocks per matrix of norm_stage_kernel. Staged again only now and then: 2048 blocks over the
 // call's matrices (8 at least each), of which the usual step runs the sums only. Without kept
 // scales every tile has its block.
 int norm_stage_blocks(const PreArgs& s, bool kept, long long matrices) {
   const long long tiles = (long long)(s.Rp / kTile) * (s.Cp / kTile);
-  return (int)(kept ? std::min(tiles, std::max(8LL, 1024 / matrices)) : tiles);
+  return (int)(kept ? std::min(tiles, std::max(8LL, 2048 / matrices)) : tiles);
 }
 long long matrices_of(const NormArgs* a, int n) {
   long long matrices = 0;
@@ -791,19 +791,16 @@ long long matrices_of(const NormArgs* a, int n) {
 //  - without kept scales, by the partials that all blocks read: a call of eight 1024 x 4096 (2^25)
 //    738 -> 733 us and of eight 1024 x 2048 577 -> 572, but thirty-two 512 x 8192 (2^27) 1166 ->
 //    1193 and sixty-four 1408 x 2048 5881 -> 5945;
-//  - with kept scales the usual step only sums (a gain of 1 .. 3 us at any size), while the first
-//    one, which stages every matrix, has few blocks: the staging of sixty-four 2048 x 1408 (3072
-//    partials each) 637 -> 720 us, of thirty-two 1024 x 4096 398 -> 420, of four 59.1 -> 59.2, and
-//    of sixty-four 1024 x 1024 233 -> 205.
+//  - with kept scales the usual step only sums: the staging of sixty-four 1408 x 2048 430 -> 426 us,
+//    of sixty-four 512 x 512 44 -> 37, of sixteen sets of four ragged shapes 173 -> 163. The first
+//    one stages every matrix on the same few blocks: those ragged ones 461 -> 337 and the 512 x 512
+//    149 -> 62, but matrices of 3072 or 4096 partials up to 6% slower (sixty-four 2048 x 1408 640 ->
+//    681, with half of the blocks 720), which the later steps outweigh.
 bool norm_stage_pays(const NormArgs* a, int n, const PreArgs* p, int np) {
   const long long matrices = matrices_of(a, n);
   long long reads = 0;
-  for (int g = 0; g < n; ++g) {
+  for (int g = 0; g < n; ++g)
     if (a[g].nparts > kNormStageParts) return false;
-    if (a[g].est_ptrs && a[g].nparts > kNormStageParts / 2 &&
-        (long long)a[g].L * a[g].nparts > kNormStageFirst)
-      return false;
-  }
   for (int i = 0; i < np; ++i) {
     const NormArgs& g = a[p[i].norm_group];
     reads += (long long)norm_stage_blocks(p[i], g.est_ptrs != nullptr, matrices) * p[i].L * g.nparts;
