@@ -649,7 +649,7 @@ def main():
         a_gbs = adam["bytes"] / (adam["ms"] * 1e-3) / 1e9
         adamw = {"ms_per_step": round(a_ms, 3), "params": rest_elems,
                  "impl": "fused HIP multi-tensor AdamW inside the timed opt.step() "
-                         "(dmuon_adamw_multi; reference muon.py:1857-1916 semantics)",
+                         "(dmuon_adamw_tensors; reference muon.py:1857-1916 semantics)",
                  "roofline": {"bound": "hbm", "achieved": round(a_gbs, 1), "peak": HBM_PEAK_GBS,
                               "unit": "GB/s", "frac": round(a_gbs / HBM_PEAK_GBS, 4),
                               "algorithmic_bytes_per_elem": 14}}
@@ -670,7 +670,7 @@ def main():
         c_bytes = n_elems * 2 * 3           # bf16: read for the norms, read + write to scale
         c_gbs = c_bytes / (c_ms * 1e-3) / 1e9
         clip = {"ms_per_call": round(c_ms, 3), "grads": n_mats, "elements": n_elems,
-                "impl": "Muon.clip_grad_norm_ on dmuon_segmented_l2_norm_sq + "
+                "impl": "Muon.clip_grad_norm_ on dmuon_clip_norms + "
                         "dmuon_segmented_scale (reference fast_clip_kernel.cu semantics)",
                 "roofline": {"bound": "hbm", "achieved": round(c_gbs, 1), "peak": HBM_PEAK_GBS,
                              "unit": "GB/s", "frac": round(c_gbs / HBM_PEAK_GBS, 4),

@@ -72,10 +72,13 @@ class Muon(torch.optim.Optimizer):
     Extra keyword arguments of the reference that concern multi-rank scheduling
     (``replicate_async``, ``group_prepare_ahead``, ``tp_distributed_gram*``,
     ``post_step_prefetch_*``, ``forward_prefetch_depth``, ...) are accepted and have no effect
-    at world_size=1. ``workspace_limit_bytes`` bounds the NS scratch of one chunk (a bucket of
-    same-shape matrices is processed in chunks that fit, sized to waste little of the last wave
-    of tiles; the 24 GiB default holds a whole 4096 x 4096 Llama bucket of 64, or 32 of the
-    4096 x 14336 ones, in one chunk -- a small part of MI355X's 288 GB); ``overlap_staging=True`` stages the
+    at world_size=1. ``workspace_limit_bytes`` bounds the NS scratch of one call, which the optimizer
+    keeps: a chunk (a bucket of same-shape matrices is processed in chunks that fit, sized to waste
+    little of the last wave of tiles; the 24 GiB default holds a whole 4096 x 4096 Llama bucket of
+    64, or 32 of the 4096 x 14336 ones, in one chunk -- a small part of MI355X's 288 GB), or up to 8
+    chunks of different shapes that are faster together, whose scratch is then the sum of theirs (32
+    matrices of 4096 x 4096 and 16 of 4096 x 11008: 12.5 GB against 7.2 GB for the larger alone);
+    a limit below the sum keeps them apart. ``overlap_staging=True`` stages the
     next chunk on a side stream while the current chunk's NS runs, with two such workspaces
     (bit-identical results; off by default: on MI355X the concurrent staging traffic slows the
     MFMA kernels by about as much as it hides). ``single_pass_staging=True`` (the default) keeps

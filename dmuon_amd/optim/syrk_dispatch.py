@@ -6,9 +6,11 @@ the gfx950 HIP kernel.
 ``gram_newton_schulz``'s fp16 operands (``newton_schulz.py:376-433``). The reference chooses
 between a CuTeDSL / quack SYRK and cuBLAS per shape; here one kernel family serves every call:
 upper-triangle tiles with the mirror written by the epilogue, fp32 accumulation, fp16 or bf16
-operands (``dmuon_syrk``). Shapes the kernel cannot read in place (M not a multiple of the
-tile, K not a multiple of 64, unaligned rows) run on zero-padded copies in a workspace this
-module keeps per device and stream, which is where the reference would fall back to cuBLAS.
+operands (``dmuon_syrk``). Whole tiles are read and written in place, and so are ragged M and K in
+whole 16-byte chunks (multiples of 8, aligned rows) up to two 128-tiles per CU. Other shapes (odd
+sides, unaligned rows, a large ragged product, a result laid over its operands) run on zero-padded
+copies in a workspace this module keeps per device and stream, which is where the reference would
+fall back to cuBLAS.
 
 As in the reference, ``B`` other than ``A`` is allowed only when ``A @ B^T`` is symmetric (the
 caller's responsibility: only one triangle is computed), a non-K-contiguous operand is copied
