@@ -216,30 +216,14 @@ int plan(int rows, int cols, int batch, int tile_req, int num_cus, int gram, int
 // 8192) of triangle products with 36 .. 1020 tiles: 256-tiles 13 us + 1.0 per slice on a third of
 // the CUs and 1.4 on all of them, 128-tiles one per CU 6 + 0.39 .. 0.46, two per CU 8 + 0.93 for
 // the pair, 64-tiles 5 + 0.18 (two of them per CU take 1 .. 2 us less than the 128-tiles one per CU
-// that stand for them here). Only the comparison of two splits matters.
+// that stand for them here). Only the comparison of two splits matters. That one of the Q updates may
+// run in the CUs the triangle launches leave idle (nt_fill_pays, up to four groups) is left out: with
+// it counted, 59 of 400 random sets of 2 .. 9 shapes were split another way, and forty of those ran 0.7%
+// slower in the mean (0.93 .. 1.15 of the time), the estimate's other errors being larger.
 double groups_cost_us(const dmuon_muon_group* g, int n, int tile, int num_cus, bool gram) {
   // launches of one NS run of five steps: X X^T, m x m triangle products, Q updates, P X
-  const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_px = gram ? 2 : 5;
-  double n_full = gram ? 3 : 0;
-  if (gram && 2 * n <= kMaxGroups) {
-    NtArgs tri[kMaxGroups], q[kMaxGroups];
-    for (int i = 0; i < n; ++i) {
-      const int m = g[i].rows < g[i].cols ? g[i].rows : g[i].cols;
-      NtArgs& s = tri[i];
-      s = NtArgs{};
-      s.M = s.N = s.K = (int)round_up(m, tile);
-      s.k_loop = (int)round_up(m, 64);
-      s.live_rows = s.live_cols = s.k_loop < s.M ? s.k_loop : 0;
-      s.L = g[i].batch;
-      q[i] = s;
-      s.tri = 1;
-      s.tiles_per_mat = tri_tiles(s.M, tile);
-      q[i].tiles_per_mat = (s.M / tile) * (s.M / tile);
-    }
-    // one of the Q updates in the CUs that the triangle launches leave idle: about half of its
-    // time comes back (one 1024^2 matrix 4.6 of 10 us, one 4096^2 55 of 104)
-    if (nt_fill_pays(tri, q, n, tile, num_cus)) n_full = 2.5;
-  }
+  const double n_xx = gram ? 2 : 5, n_tri = gram ? 11 : 5, n_full = gram ? 3 : 0,
+               n_px = gram ? 2 : 5;
   auto launch = [&](auto&& dims) {   // dims(group, tile): (tiles of one matrix, K)
     auto total = [&](int t) {
       double tiles = 0;

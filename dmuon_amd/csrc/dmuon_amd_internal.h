@@ -253,7 +253,7 @@ struct ClipArgs {
 hipError_t launch_clip_sumsq(const ClipArgs& a, hipStream_t stream);
 hipError_t launch_clip_scale(ClipArgs a, hipStream_t stream);
 
-// Norms, coefficients and flags of a job table's tensors in two launches. Tensor t's jobs are
+// Norms, coefficients and flags of a job table's tensors in two to four launches. Tensor t's jobs are
 // first_job[t] .. first_job[t + 1] - 1, each split into `pieces` pieces (clip_pieces) whose sums
 // go to partials[job * pieces + piece].
 struct ClipFinishArgs {

@@ -113,7 +113,8 @@ int dmuon_stream_copy(const void* src, void* dst, int64_t bytes, void* stream);
  * Any M >= 0 and K >= 0 are accepted. When M is a multiple of the tile, K of 64, and every base
  * is 16-byte aligned with leading dimensions and batch strides that are multiples of 8, the
  * kernel reads the operands in place and `workspace` may be NULL; so it does, so aligned, when M
- * and K are only multiples of 8 and a 128-tile plan has at most 512 tiles; otherwise the call runs on
+ * and K are only multiples of 8, a 128-tile plan has at most 512 tiles and D shares no memory with
+ * A, B or C; otherwise the call runs on
  * zero-padded copies in `workspace` (device memory of dmuon_syrk_workspace_size bytes, at least
  * 16-byte aligned; contents need no initialisation) and copies the M x M result into D.
  */
@@ -423,8 +424,8 @@ int dmuon_segmented_scale(const int64_t* ptrs, const int64_t* numels, const int3
                           const float* coefs, void* stream);
 
 /*
- * Norms, clip coefficients and flags of the tensors of such a job table, in two launches and
- * without atomics (the same bits on every call). Tensor t's jobs are first_job[t] ..
+ * Norms, clip coefficients and flags of the tensors of such a job table, in two launches (four past
+ * 256 tensors or segments) and without atomics (the same bits on every call). Tensor t's jobs are first_job[t] ..
  * first_job[t + 1] - 1 (DEVICE array of n_tensors + 1).
  *   n_segments > 0: norms[s] = sqrt of segment s's sum of squares, coefs[s] = min(max_norm /
  *     (norms[s] + 1e-6), 1), clipped[s] = norms[s] finite and > max_norm, found_inf[s] = not

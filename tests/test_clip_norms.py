@@ -1,4 +1,4 @@
-"""``dmuon_clip_norms``: norms, coefficients and flags of a job table in two launches."""
+"""``dmuon_clip_norms``: norms, coefficients and flags of a job table in two to four launches."""
 import ctypes
 import math
 import time

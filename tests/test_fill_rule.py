@@ -1,7 +1,5 @@
 """Where the middle Q update of a Gram segment runs: in the idle CUs of three triangle launches, or
 in a launch of its own. The choice changes no bit, only the time."""
-import pytest
-
 from dmuon_amd import _C
 
 # (rows, matrices): whether the update in the triangle launches was the faster one, measured on
@@ -21,13 +19,3 @@ def test_the_faster_place_of_the_q_update(cpp_harness):
     for (m, batch), _ in FILL:
         args += [m, batch, _C.plan(m, m, batch, 0, 256, _C.NS_GRAM)[0]]
     assert cpp_harness("nt_fill", *args) == "".join(str(want) for _, want in FILL)
-
-
-def test_the_estimate_knows_the_fill():
-    """A call of five groups has no room for a second table entry each: its Q update is a launch of
-    its own, which the estimate counts. Up to four groups it is the one of a single batch."""
-    us = lambda shapes: _C.plan_groups(shapes, 128, 256, _C.NS_GRAM)[2]  # noqa: E731
-    assert us([(256, 512, 1)] * 4) == pytest.approx(us([(256, 512, 4)]))
-    assert us([(256, 512, 1)] * 5) > us([(256, 512, 5)])
-    # where the update has its own launch in any case there is no difference
-    assert us([(1024, 1024, 1)] * 6) == pytest.approx(us([(1024, 1024, 6)]))
