@@ -172,3 +172,29 @@ def test_many_tensors_and_segments(gpu, n, n_segments):
     found = table.norms(n_segments, 6.0)[3]
     assert found.tolist() == [s == of[n - 1] for s in range(n_segments)]
     assert bool(table.norms(0, 6.0)[3][0])
+
+
+@pytest.mark.gpu
+def test_a_captured_call_reads_the_kept_table(gpu):
+    """After one eager call a clip can be captured: the capture's own stream finds the kept table and
+    waits for nothing outside the graph; every replay clips what the gradients then hold."""
+    grads = _grads([70_001, 33, 9000], DT, gpu, 8)
+    buckets = (GradClipBucket("a", grads[:2], reduce=False), GradClipBucket("b", grads[2:], reduce=False))
+    values = [[g * (k + 1) for g in grads] for k in range(3)]
+    want = []
+    for v in values:
+        for g, x in zip(grads, v):
+            g.copy_(x)
+        res = clip_grad_norm_buckets_(buckets, 3.0)
+        want.append(([g.clone() for g in grads], res.total_norm.clone()))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        res = clip_grad_norm_buckets_(buckets, 3.0)
+    for v, (after, total) in zip(values, want):
+        for g, x in zip(grads, v):
+            g.copy_(x)
+        graph.replay()
+        assert all(torch.equal(g, a) for g, a in zip(grads, after))
+        assert torch.equal(res.total_norm, total)
+        clip_grad_norm_buckets_(buckets, None)          # eager work between the replays
+        torch.cuda.synchronize()
